@@ -12,37 +12,125 @@ namespace {
 
 using namespace r2;
 
-// avg[x] = sum_y log(r + g + b + FLT_MIN) / (W H 3)  (computeGlobalTonemapping1)
-__global__ void k_tm_columns(const float* __restrict__ hdr, int w, int h, float* __restrict__ avg) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= w) return;
-  const float divisor = (float)(h * w * 3);
-  float a = 0.f;
-  for (int y = 0; y < h; ++y) {
-    const float* p = hdr + 3 * ((size_t)y * w + x);
-    a += det_logf(p[0] + p[1] + p[2] + FLT_MIN) / divisor;
+// a + q[0] + q[1] + ... in that order, n values of LDS (16-byte aligned).  The chain
+// of additions is the bound: the next 32 values are read while 32 are added, so that
+// no addition waits for LDS (read four by four as they were needed, 1920 values took
+// 24 us, 29 cycles an addition).
+__device__ __forceinline__ float add_in_order(float a, const float* q, int n) {
+  const float4* q4 = reinterpret_cast<const float4*>(q);
+  int r = 0;
+  if (n >= 32) {
+    float4 v[8], u[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = q4[j];
+    for (; r + 32 <= n; r += 32) {
+      const int nx = r + 64 <= n ? r / 4 + 8 : 0;  // the last round reads the first values again
+#pragma unroll
+      for (int j = 0; j < 8; ++j) u[j] = q4[nx + j];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        a += v[j].x;
+        a += v[j].y;
+        a += v[j].z;
+        a += v[j].w;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = u[j];
+    }
   }
-  avg[x] = a;
+  for (; r < n; ++r) a += q[r];
+  return a;
 }
 
-// k = exp(sum_x avg[x]) - W H FLT_MIN  (computeGlobalTonemapping2)
-__global__ void k_tm_factor(const float* __restrict__ avg, int w, int h, float* __restrict__ factor) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+// avg[x] = sum_y log(r + g + b + FLT_MIN) / (W H 3)  (computeGlobalTonemapping1)
+//
+// A column's terms are added one after another (the reference's order), but they
+// do not depend on each other: a block takes kTmCols columns, its waves 1.. compute
+// the terms of kTmRows rows into LDS while wave 0 adds those of the kTmRows rows
+// before, one column per lane, four terms per LDS read.  What bounds it is the
+// chain of h additions (about 3 us for 1080) behind the double-evaluated logs of
+// one chunk; with one thread per column it was the load, log and addition of every
+// row in turn: 81 us for 1920 x 1080, now 14 us.  8 columns per block give 240
+// blocks at 1920 (fewer columns would cut a row's 96 bytes below a line).
+constexpr int kTmCols = 8, kTmRows = 512, kTmThreads = 1024;
+constexpr int kTmStride = kTmRows + 4;  // columns 4 banks apart, 16-byte aligned
+__global__ __launch_bounds__(kTmThreads) void k_tm_columns(const float* __restrict__ hdr, int w, int h,
+                                                           float* __restrict__ avg) {
+  __shared__ __align__(16) float term[2][kTmCols * kTmStride];
+  const int x0 = blockIdx.x * kTmCols;
+  const float divisor = (float)(h * w * 3);
+  const int nchunk = (h + kTmRows - 1) / kTmRows;
+  const int t = (int)threadIdx.x - 64;
+  float a = 0.f;
+  for (int c = 0; c <= nchunk; ++c) {
+    if (t >= 0) {
+      const int y0 = c * kTmRows, rows = min(kTmRows, h - y0);  // rows <= 0 past the last chunk
+      for (int i = t; i < rows * kTmCols; i += kTmThreads - 64) {
+        const int col = i % kTmCols, r = i / kTmCols, x = x0 + col;
+        if (x < w) {
+          const float* p = hdr + 3 * ((size_t)(y0 + r) * w + x);
+          term[c & 1][col * kTmStride + r] = det_logf(p[0] + p[1] + p[2] + FLT_MIN) / divisor;
+        }
+      }
+    } else if (c > 0 && threadIdx.x < kTmCols) {
+      const int rows = min(kTmRows, h - (c - 1) * kTmRows);
+      a = add_in_order(a, term[(c - 1) & 1] + threadIdx.x * kTmStride, rows);
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < kTmCols && x0 + (int)threadIdx.x < w) avg[x0 + threadIdx.x] = a;
+}
+
+// k = exp(sum_x avg[x]) - W H FLT_MIN  (computeGlobalTonemapping2): one chain of w
+// additions, staged through LDS by the whole block (reading each column sum from
+// memory in the chain took 510 us for 1920 columns, now 10 us)
+constexpr int kTmFactorThreads = 1024;
+__global__ __launch_bounds__(kTmFactorThreads) void k_tm_factor(const float* __restrict__ avg, int w, int h,
+                                                                float* __restrict__ factor) {
+  __shared__ __align__(16) float s[kTmFactorThreads];
   float r = 0.f;
-  for (int x = 0; x < w; ++x) r += avg[x];
-  *factor = det_expf(r) - (float)(w * h) * FLT_MIN;
+  for (int x0 = 0; x0 < w; x0 += kTmFactorThreads) {
+    const int n = min(kTmFactorThreads, w - x0);
+    if ((int)threadIdx.x < n) s[threadIdx.x] = avg[x0 + threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x == 0) r = add_in_order(r, s, n);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *factor = det_expf(r) - (float)(w * h) * FLT_MIN;
 }
 
-// applyTonemapping, correctGamma, fillByteFrame
+// applyTonemapping, correctGamma, fillByteFrame.  Bound by the double-evaluated
+// power (26 us at 1920 x 1080, 11 us of which the memory needs); a thread takes four values, so that the frame moves in 16-byte loads and
+// stores and the bytes in whole words where the pointers are aligned for it (kVec).
+template <bool kVec>
 __global__ void k_tm_apply(const float* __restrict__ hdr, size_t n3, const float* __restrict__ factor, float inv_gamma,
                            float* __restrict__ ldr, uint8_t* __restrict__ bytes) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= n3) return;
   const float k = *factor;
-  const float c = hdr[i];
-  const float t = det_powf(c / (c + k), inv_gamma);
-  if (ldr) ldr[i] = t;
-  if (bytes) bytes[i] = (uint8_t)roundf(t * 255.0f);
+  const int n = n3 - i < 4 ? (int)(n3 - i) : 4;
+  float c[4] = {0.f, 0.f, 0.f, 0.f}, t[4];
+  uint8_t b[4];
+  if (kVec && n == 4) {
+    const float4 v = *reinterpret_cast<const float4*>(hdr + i);
+    c[0] = v.x; c[1] = v.y; c[2] = v.z; c[3] = v.w;
+  } else {
+    for (int j = 0; j < n; ++j) c[j] = hdr[i + j];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    t[j] = det_powf(c[j] / (c[j] + k), inv_gamma);
+    b[j] = (uint8_t)roundf(t[j] * 255.0f);
+  }
+  if (kVec && n == 4) {
+    if (ldr) *reinterpret_cast<float4*>(ldr + i) = make_float4(t[0], t[1], t[2], t[3]);
+    if (bytes) *reinterpret_cast<uchar4*>(bytes + i) = make_uchar4(b[0], b[1], b[2], b[3]);
+  } else {
+    for (int j = 0; j < n; ++j) {
+      if (ldr) ldr[i + j] = t[j];
+      if (bytes) bytes[i + j] = b[j];
+    }
+  }
 }
 
 }  // namespace
@@ -64,19 +152,24 @@ extern "C" int r2_postprocess(r2_ctx* ctx, const float* hdr, int32_t w, int32_t 
   float* d_ldr = ldr;
   uint8_t* d_bytes = bytes;
   if (!on_device) {
-    float* base = factor + 64;
-    float* in = base;
-    float* outf = base + n3;
-    uint8_t* outb = (uint8_t*)(outf + n3);
+    // each array 16-byte aligned (the 512 spare bytes cover the rounding)
+    const size_t n3p = (n3 + 3) & ~(size_t)3;
+    float* in = (float*)(((uintptr_t)(factor + 64) + 15) & ~(uintptr_t)15);
+    float* outf = in + n3p;
+    uint8_t* outb = (uint8_t*)(outf + n3p);
     R2_HIP(ctx, hipMemcpyAsync(in, hdr, n3 * 4, hipMemcpyHostToDevice, st));
     d_hdr = in;
     d_ldr = ldr ? outf : nullptr;
     d_bytes = bytes ? outb : nullptr;
   }
-  hipLaunchKernelGGL(k_tm_columns, dim3((w + 127) / 128), dim3(128), 0, st, d_hdr, w, h, avg);
-  hipLaunchKernelGGL(k_tm_factor, dim3(1), dim3(64), 0, st, avg, w, h, factor);
-  hipLaunchKernelGGL(k_tm_apply, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, st, d_hdr, n3, factor,
-                     1.f / gamma, d_ldr, d_bytes);
+  hipLaunchKernelGGL(k_tm_columns, dim3((w + kTmCols - 1) / kTmCols), dim3(kTmThreads), 0, st, d_hdr, w, h, avg);
+  hipLaunchKernelGGL(k_tm_factor, dim3(1), dim3(kTmFactorThreads), 0, st, avg, w, h, factor);
+  const dim3 ablk((unsigned)((n3 + 1023) / 1024));
+  const bool vec = (((uintptr_t)d_hdr | (uintptr_t)d_ldr) & 15) == 0 && ((uintptr_t)d_bytes & 3) == 0;
+  if (vec)
+    hipLaunchKernelGGL(k_tm_apply<true>, ablk, dim3(256), 0, st, d_hdr, n3, factor, 1.f / gamma, d_ldr, d_bytes);
+  else
+    hipLaunchKernelGGL(k_tm_apply<false>, ablk, dim3(256), 0, st, d_hdr, n3, factor, 1.f / gamma, d_ldr, d_bytes);
   R2_HIP(ctx, hipGetLastError());
   if (!on_device) {
     if (ldr) R2_HIP(ctx, hipMemcpyAsync(ldr, d_ldr, n3 * 4, hipMemcpyDeviceToHost, st));

@@ -19,7 +19,7 @@ import pytest
 
 import oracle as O
 import renderer2_amd as r2
-from renderer2_amd import capi, scenes
+from renderer2_amd import _hip, capi, scenes
 
 from brickgrid_io import check_against_device
 
@@ -38,6 +38,29 @@ def test_postprocess_matches_oracle(ctx):
         assert np.array_equal(ldr.view(np.uint32), ref_ldr.view(np.uint32))
         assert np.array_equal(by, ref_by)
         assert 0 < by.mean() < 255
+
+
+# rows around the 512-row chunk, columns around the 8-column block and the
+# 1024-column stage, value counts that are no multiple of 4; the device form also
+# with pointers that are not aligned for 16-byte access
+@pytest.mark.parametrize("h,w,shift", [(1, 1, 0), (5, 1025, 0), (511, 7, 1), (513, 9, 0), (1030, 33, 1), (64, 2051, 0)])
+def test_postprocess_shapes_equal_the_oracle(ctx, h, w, shift):
+    rng = np.random.default_rng(h * 7919 + w)
+    hdr = (rng.lognormal(0.0, 2.0, (h, w, 3)) * (rng.random((h, w, 1)) > 0.05)).astype(np.float32)
+    ref_ldr, ref_by = O.postprocess(hdr, 1.8)
+    n = hdr.size
+    src, ldr, by = _hip.DeviceBuffer(4 * (n + 4)), _hip.DeviceBuffer(4 * (n + 4)), _hip.DeviceBuffer(n + 4)
+    src.from_host(np.concatenate([np.zeros(shift, np.float32), hdr.reshape(-1)]))
+    capi.check(capi.lib().r2_postprocess(ctx.h, src.addr + 4 * shift, w, h, C.c_float(1.8), ldr.addr + 4 * shift,
+                                         by.addr + shift, 1), ctx.h)
+    out_ldr = ldr.to_host(np.float32)[shift:shift + n]
+    out_by = by.to_host(np.uint8)[shift:shift + n]
+    assert np.array_equal(out_ldr.view(np.uint32), ref_ldr.reshape(-1).view(np.uint32))
+    assert np.array_equal(out_by, ref_by.reshape(-1))
+    host_ldr, host_by = np.zeros_like(hdr), np.zeros(hdr.shape, np.uint8)
+    capi.check(capi.lib().r2_postprocess(ctx.h, hdr.ctypes.data, w, h, C.c_float(1.8), host_ldr.ctypes.data,
+                                         host_by.ctypes.data, 0), ctx.h)
+    assert np.array_equal(host_ldr.view(np.uint32), ref_ldr.view(np.uint32)) and np.array_equal(host_by, ref_by)
 
 
 def write_obj(path: Path, mesh: dict):
