@@ -176,8 +176,12 @@ size_t scene_bytes_for(int n_inst) {
   return h.device_bytes();
 }
 
+uint64_t* scene_counter(r2_ctx* ctx, const HostScene& hs) {
+  return (uint64_t*)((char*)ctx->d_scene + hs.device_bytes());
+}
+
 int upload_scene(r2_ctx* ctx, const HostScene& hs, bool may_alloc) {
-  const size_t need = hs.device_bytes();
+  const size_t need = hs.device_bytes() + kSceneCounterBytes;
   if (need > ctx->scene_cap) {
     if (!may_alloc)
       return fail(ctx, R2_ERR_UNSUPPORTED,
@@ -192,6 +196,7 @@ int upload_scene(r2_ctx* ctx, const HostScene& hs, bool may_alloc) {
   }
   // the image stays in the context until the next upload, past the stream's copy
   hs.pack(ctx->d_scene, ctx->scene_img);
+  ctx->scene_img.resize(need, 0);  // the item counter: 0
   R2_HIP(ctx, hipMemcpyAsync(ctx->d_scene, ctx->scene_img.data(), need, hipMemcpyHostToDevice, ctx->stream));
   return R2_OK;
 }
@@ -323,12 +328,11 @@ int r2_create(r2_ctx** out, int device) {
       hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&c->side_done, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->main_mark, hipEventDisableTiming) != hipSuccess ||
-      hipMalloc((void**)&c->d_scene, scene_bytes_for(kCtxSceneInstances)) != hipSuccess ||
-      hipMalloc((void**)&c->d_counter, 64) != hipSuccess) {
+      hipMalloc((void**)&c->d_scene, scene_bytes_for(kCtxSceneInstances) + kSceneCounterBytes) != hipSuccess) {
     r2_destroy(c);
     return R2_ERR_HIP;
   }
-  c->scene_cap = scene_bytes_for(kCtxSceneInstances);
+  c->scene_cap = scene_bytes_for(kCtxSceneInstances) + kSceneCounterBytes;
   // the address of r2_render_noalloc's scratch array on this device (kept per
   // device; a failure is reported by that entry point, the context stays usable)
   (void)noalloc_scratch_init(c);
@@ -344,7 +348,6 @@ int r2_destroy(r2_ctx* c) {
   if (c->side) (void)hipStreamSynchronize(c->side);
   if (c->scratch) (void)hipFree(c->scratch);
   if (c->d_scene) (void)hipFree(c->d_scene);
-  if (c->d_counter) (void)hipFree(c->d_counter);
   for (int i = 0; i < r2_ctx::kPoolSlots; ++i)
     if (c->pool[i]) (void)hipFree(c->pool[i]);
   if (c->ev0) (void)hipEventDestroy(c->ev0);

@@ -26,7 +26,6 @@ struct r2_ctx {
   r2::DScene* d_scene = nullptr;
   size_t scene_cap = 0;
   std::vector<unsigned char> scene_img;
-  uint32_t* d_counter = nullptr;
   r2_filter_stats fstats{};
   // grow-only device buffers reused across calls (filter binning scratch)
   static constexpr int kPoolSlots = 24;
@@ -65,8 +64,8 @@ struct BatchEntry {
 // integrator launchers of the two record-precision instantiations
 #define R2K_DECLARE(NS)                                                                                              \
   namespace NS {                                                                                                     \
-  void launch_sm(hipStream_t st, int blocks, const r2::DScene* d_scene, uint64_t* counter, uint64_t total, int chunk, \
-                 void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp, const int32_t* ps, \
+  void launch_sm(hipStream_t st, int blocks, int lanes, const r2::DScene* d_scene, uint64_t* counter, uint64_t total, \
+                 int chunk, void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp, const int32_t* ps, \
                  float* po, uint32_t* pc);                                                                           \
   void launch_batch_group(hipStream_t st, int blocks, const void* ents, int n, uint64_t* counters, bool single,      \
                           bool surf, bool fp64);                                                                     \
@@ -104,8 +103,12 @@ struct HostScene {
 constexpr int kCtxSceneInstances = 4096;
 size_t scene_bytes_for(int n_inst);
 // copy the scene image to ctx->d_scene on ctx->stream, growing the buffer when
-// may_alloc (else R2_ERR_UNSUPPORTED beyond kCtxSceneInstances)
+// may_alloc (else R2_ERR_UNSUPPORTED beyond kCtxSceneInstances).  The item counter
+// of the launch to follow, 0, travels behind the image in 256 bytes of its own: one
+// copy instead of a copy and two fills
+constexpr size_t kSceneCounterBytes = 256;
 int upload_scene(r2_ctx* ctx, const HostScene& hs, bool may_alloc);
+uint64_t* scene_counter(r2_ctx* ctx, const HostScene& hs);
 // render kernels (r2_render.hip)
 int launch_render(r2_ctx* ctx, const HostScene& scene, float* d_out, bool fp64_accum);
 struct RenderOpts {

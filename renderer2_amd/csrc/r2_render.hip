@@ -27,13 +27,34 @@ static int num_cus(r2_ctx* ctx) {
   return g_num_cus;
 }
 
-static void launch_sm(r2_ctx* ctx, int prec, int blocks, uint64_t total, int chunk, void* partial, bool fp64, bool single,
-                      bool surf, bool count, const int32_t* pp, const int32_t* ps, float* po, uint32_t* pc) {
+// Shape of a persistent launch over `items` work items: kBlocksPerCu blocks of four
+// wavefronts per CU are resident (the LDS slots allow no more), and a wavefront
+// holds up to 64 items.  A launch of fewer items than kSpreadWaves wavefronts per CU
+// have lanes spreads them over that many wavefronts, `lanes` each: a wavefront's
+// steps serve its lanes one block of code at a time, so with few lanes a path is
+// through sooner, while beyond two wavefronts per SIMD they slow each other.
+// Frames of the 64^3 volume at 4 / 8 / 16 / 32 wavefronts per CU, us, and with 64
+// items to a wavefront: 14400 paths 450 / 432 / 439 / 448, 589; 57600 paths 564 /
+// 541 / 551 / 608, 610; 115200 paths 600 / 590 / 622 / 671, 611.
+constexpr int kBlocksPerCu = 4, kWavesPerBlock = 4, kSpreadWaves = 8;
+struct LaunchShape {
+  int blocks, lanes;
+};
+static LaunchShape launch_shape(r2_ctx* ctx, uint64_t items) {
+  const uint64_t cus = (uint64_t)num_cus(ctx), spread = cus * kSpreadWaves;
+  const uint64_t lanes = std::min<uint64_t>(64, std::max<uint64_t>(1, (items + spread - 1) / spread));
+  const uint64_t per_block = lanes * kWavesPerBlock;
+  return LaunchShape{(int)std::min<uint64_t>(cus * kBlocksPerCu, (items + per_block - 1) / per_block), (int)lanes};
+}
+
+static void launch_sm(r2_ctx* ctx, int prec, const LaunchShape& sh, uint64_t* counter, uint64_t total,
+                      int chunk, void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp,
+                      const int32_t* ps, float* po, uint32_t* pc) {
   if (prec == 1)
-    r2k_packed::launch_sm(ctx->stream, blocks, ctx->d_scene, (uint64_t*)ctx->d_counter, total, chunk, partial, fp64,
+    r2k_packed::launch_sm(ctx->stream, sh.blocks, sh.lanes, ctx->d_scene, counter, total, chunk, partial, fp64,
                           single, surf, count, pp, ps, po, pc);
   else
-    r2k_fp32::launch_sm(ctx->stream, blocks, ctx->d_scene, (uint64_t*)ctx->d_counter, total, chunk, partial, fp64,
+    r2k_fp32::launch_sm(ctx->stream, sh.blocks, sh.lanes, ctx->d_scene, counter, total, chunk, partial, fp64,
                         single, surf, count, pp, ps, po, pc);
 }
 
@@ -84,7 +105,7 @@ int launch_batch(r2_ctx* ctx, hipStream_t st, const std::vector<BatchSlice>& ite
     BatchEntry* de = (BatchEntry*)d_ents + first;
     R2_HIP(ctx, hipMemcpyAsync(de, &host[first], sizeof(BatchEntry) * n, hipMemcpyHostToDevice, st));
     R2_HIP(ctx, hipMemsetAsync(d_counters + first, 0, sizeof(uint64_t) * n, st));
-    const int blocks = (int)std::min<uint64_t>((uint64_t)num_cus(ctx) * 8, (total + 255) / 256);
+    const int blocks = (int)std::min<uint64_t>((uint64_t)num_cus(ctx) * kBlocksPerCu, (total + 255) / 256);
     if (packed) r2k_packed::launch_batch_group(st, blocks, de, n, d_counters + first, single, surf, fp64);
     else r2k_fp32::launch_batch_group(st, blocks, de, n, d_counters + first, single, surf, fp64);
     R2_HIP(ctx, hipGetLastError());
@@ -98,14 +119,11 @@ int launch_batch(r2_ctx* ctx, hipStream_t st, const std::vector<BatchSlice>& ite
 // sample chunk, like the reference's one launch per sample: a launch takes the
 // items [first, total) by starting the shared item counter at `first`.  Each item
 // writes its own chunk sum, so the frame is the same bit for bit either way.
-static int launch_items(r2_ctx* ctx, int prec, bool single, bool surf, bool fp64, uint64_t first, uint64_t total,
-                        int chunk, void* partial) {
-  hipStream_t st = ctx->stream;
-  // the counter's low word = first (< 2^32: items of a launch fit 32 bits), high word 0
-  R2_HIP(ctx, hipMemsetD32Async((hipDeviceptr_t)ctx->d_counter, (int)(uint32_t)first, 1, st));
-  R2_HIP(ctx, hipMemsetD32Async((hipDeviceptr_t)(ctx->d_counter + 1), 0, 1, st));
-  const int blocks = (int)std::min<uint64_t>((uint64_t)num_cus(ctx) * 8, (total - first + 255) / 256);
-  launch_sm(ctx, prec, blocks, total, chunk, partial, fp64, single, surf, false, nullptr, nullptr, nullptr, nullptr);
+static int launch_items(r2_ctx* ctx, int prec, bool single, bool surf, bool fp64, uint64_t* counter, uint64_t first,
+                        uint64_t total, int chunk, void* partial) {
+  const LaunchShape sh = launch_shape(ctx, total - first);
+  launch_sm(ctx, prec, sh, counter, total, chunk, partial, fp64, single, surf, false, nullptr, nullptr, nullptr,
+            nullptr);
   R2_HIP(ctx, hipGetLastError());
   return R2_OK;
 }
@@ -144,11 +162,12 @@ int launch_render_ex(r2_ctx* ctx, const HostScene& hs, float* d_out, bool fp64, 
     const int rc = upload_scene(ctx, hs, o.scene_alloc);
     if (rc) return rc;
   }
+  uint64_t* counter = scene_counter(ctx, hs);
   R2_HIP(ctx, hipEventRecord(ctx->ev0, st));
   int done_chunks = nchunks;
   int launches = 1;
   if (!o.progress) {
-    int rc = launch_items(ctx, prec, single, surf, fp64, 0, total, chunk, partial);
+    int rc = launch_items(ctx, prec, single, surf, fp64, counter, 0, total, chunk, partial);
     if (rc) return rc;
   } else {
     // one launch per sample chunk, with up to two in flight; the callback runs
@@ -164,8 +183,11 @@ int launch_render_ex(r2_ctx* ctx, const HostScene& hs, float* d_out, bool fp64, 
     bool stop = false;
     while (completed < nchunks) {
       while (!stop && queued < nchunks && queued - completed < 2) {
-        rc = launch_items(ctx, prec, single, surf, fp64, (uint64_t)queued * npix, (uint64_t)(queued + 1) * npix,
-                          chunk, partial);
+        // the counter's low word (items of a launch fit 32 bits); its high word is 0
+        const uint64_t first = (uint64_t)queued * npix;
+        R2_HIP(ctx, hipMemsetD32Async((hipDeviceptr_t)counter,
+                                      (int)(uint32_t)first, 1, st));
+        rc = launch_items(ctx, prec, single, surf, fp64, counter, first, first + npix, chunk, partial);
         if (rc) break;
         R2_HIP(ctx, hipEventRecord(evs[queued & 1], st));
         ++queued;
@@ -258,9 +280,7 @@ int launch_paths(r2_ctx* ctx, const HostScene& hs, int n, const int32_t* d_pix, 
     const int rc = upload_scene(ctx, hs, true);
     if (rc) return rc;
   }
-  R2_HIP(ctx, hipMemsetAsync(ctx->d_counter, 0, 8, st));
-  const int blocks = (int)std::min<uint64_t>((uint64_t)num_cus(ctx) * 8, ((uint64_t)n + 255) / 256);
-  launch_sm(ctx, prec, blocks, (uint64_t)n, 1, nullptr, false, scene.n_inst == 1, scene.n_surf > 0, true, d_pix, d_smp,
+  launch_sm(ctx, prec, launch_shape(ctx, (uint64_t)n), scene_counter(ctx, hs), (uint64_t)n, 1, nullptr, false, scene.n_inst == 1, scene.n_surf > 0, true, d_pix, d_smp,
             d_out, d_cnt);
   R2_HIP(ctx, hipGetLastError());
   R2_HIP(ctx, hipStreamSynchronize(st));

@@ -219,9 +219,13 @@ struct FrameFetch {
 // waiting at it, chosen from ballots so that the costly blocks run with many
 // lanes: shading once at least R2_SHADE_MIN lanes wait for it (or nothing else
 // is left), followed by segment starts for the lanes at them; else segment
-// starts once at least R2_SEG_MIN lanes, or R2_SEG_RATIO times as many lanes as
-// are in traversals, wait for them; else a traversal step.  Returns false when
-// every lane is idle.
+// starts once at least R2_SEG_MIN of 64 lanes, or R2_SEG_RATIO times as many
+// lanes as are in traversals, wait for them; else a traversal step.  The segment
+// threshold is a share of the lanes that still hold a path: at the end of a launch,
+// and in one of few paths, half of the lanes left do not wait for the others (with
+// the fixed 32 a 333 x 217 x 16 frame took 790 us, now 746; a share for the shading
+// too costs more passes of the largest block: 830).  Returns false when every lane
+// is idle.
 #ifndef R2_SHADE_MIN
 #define R2_SHADE_MIN 48
 #endif
@@ -245,7 +249,8 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
   const bool at_seg = p.stage == ST_SEG;
   const bool at_trav = p.stage == ST_TRAV;
   const int nh = __popcll(__ballot(at_shade)), ns = __popcll(__ballot(at_seg)), nt = __popcll(__ballot(at_trav));
-  if (nh + ns + nt == 0) return false;
+  const int live = nh + ns + nt;
+  if (live == 0) return false;
 #ifdef R2_SM_STATS
   const uint64_t t0 = SM_CLOCK();
 #endif
@@ -268,7 +273,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
       seg_step<kSingle, kSurf>(s, p);
     }
     __builtin_amdgcn_s_setprio(0);
-  } else if (ns >= R2_SEG_MIN || ns >= R2_SEG_RATIO * nt) {
+  } else if (ns * 64 >= R2_SEG_MIN * live || ns >= R2_SEG_RATIO * nt) {
     SM_STAT(3, 1);
     SM_STAT(4, ns);
     __builtin_amdgcn_s_setprio(kPrioSeg);
@@ -301,7 +306,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
 #endif
 template <bool kSingle, bool kSurf, bool kCount, typename Acc>
 __global__ void __launch_bounds__(256, R2_SM_WAVES) k_paths_sm(const DScene* __restrict__ sp, uint64_t* __restrict__ counter,
-                                                  uint64_t total, int chunk, Acc* __restrict__ partial,
+                                                  int lanes, uint64_t total, int chunk, Acc* __restrict__ partial,
                                                   const int32_t* __restrict__ probe_pix,
                                                   const int32_t* __restrict__ probe_smp, float* __restrict__ probe_out,
                                                   uint32_t* __restrict__ probe_cnt) {
@@ -310,7 +315,7 @@ __global__ void __launch_bounds__(256, R2_SM_WAVES) k_paths_sm(const DScene* __r
   const uint32_t npix = (uint32_t)s.W * (uint32_t)s.H;
   __shared__ ColdLane cold[256];
   PathLane p(cold[threadIdx.x], s);
-  p.stage = ST_FETCH;
+  p.stage = lane < lanes ? ST_FETCH : ST_IDLE;  // a launch with fewer items than lanes leaves lanes idle
   p.cres = CR_START;
   Cnt cnt;
 #pragma unroll
@@ -420,12 +425,12 @@ __global__ void k_reduce(const Acc* __restrict__ partial, int nchunks, uint32_t 
 
 // host-side launchers of this instantiation.  Scenes with analytic surfaces run
 // the general-instance form with the surface code; the others the forms without.
-void launch_sm(hipStream_t st, int blocks, const DScene* d_scene, uint64_t* counter, uint64_t total, int chunk,
-               void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp, const int32_t* ps,
-               float* po, uint32_t* pc) {
+void launch_sm(hipStream_t st, int blocks, int lanes, const DScene* d_scene, uint64_t* counter, uint64_t total,
+               int chunk, void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp,
+               const int32_t* ps, float* po, uint32_t* pc) {
 #define R2K_LAUNCH(S, F, C, A)                                                                                  \
-  hipLaunchKernelGGL((k_paths_sm<S, F, C, A>), dim3(blocks), dim3(256), 0, st, d_scene, counter, total, chunk, \
-                     (A*)partial, pp, ps, po, pc)
+  hipLaunchKernelGGL((k_paths_sm<S, F, C, A>), dim3(blocks), dim3(256), 0, st, d_scene, counter, lanes, total, \
+                     chunk, (A*)partial, pp, ps, po, pc)
   if (surf) {
     if (count) R2K_LAUNCH(false, true, true, float);
     else if (fp64) R2K_LAUNCH(false, true, false, double);

@@ -50,6 +50,19 @@ def _paths_agree(ctx, grids_desc, instances, env_rgb, cfg):
     return float(np.mean(np.all(np.abs(gpu - ref) <= 1e-3 * np.maximum(np.abs(ref), 1e-3), axis=1)))
 
 
+# item counts around the steps of the lanes per wavefront (2048 wavefronts on 256
+# CUs): 1 lane, 2 lanes, 63 and 64 lanes, and the first that no longer spreads
+@pytest.mark.parametrize("W,H,spp", [(2047, 1, 1), (256, 8, 1), (683, 3, 1), (504, 256, 1), (512, 256, 1), (331, 99, 4)])
+def test_spread_launches(ctx, c1, W, H, spp):
+    w = c1
+    grids = [ctx.upload_grid(g) for g in w["grids"]]
+    env = ctx.upload_env(w["env"])
+    cfg = dict(w["render"], width=W, height=H, spp=spp)
+    img = ctx.render(cfg, grids, w["instances"], env)
+    ref = O.Scene(w["grids"], w["instances"], w["env"], "f32").render(cfg)
+    assert relmse(img, ref) <= 1e-5
+
+
 @pytest.mark.parametrize("W,H,spp", [(1, 1, 1), (7, 5, 3), (13, 29, 2), (64, 3, 5)])
 def test_ragged_and_tiny_frames(ctx, c1, W, H, spp):
     w = c1
