@@ -86,93 +86,106 @@ m44 get_rotation(v3 n) {
 
 // ------------------------------------------------------ instance hierarchy --
 // Median-split hierarchy over the instances' world boxes (the stand-in for the
-// OptiX instance acceleration structure, scene.cu:188-256): nodes in depth-first
-// order with the index of the node after each subtree, leaves of at most 4
-// instances.  The split is on the longest axis of the box centres, instances
-// ordered by centre then index, so the build is deterministic.
-static void bvh_build(const std::vector<DInstance>& inst, std::vector<DBvhNode>& nodes, std::vector<int32_t>& idx) {
+// OptiX instance acceleration structure, scene.cu:188-256), four children to a
+// node: a range of instances is halved along the longest axis of its box centres
+// and both halves along the axis that is then the longest; a range of at most four
+// becomes the node's children themselves.  Instances are ordered by centre then
+// index, so the build is deterministic.
+static int bvh_levels(int n) {
+  int l = 1;
+  while ((1ll << (2 * l)) < n) ++l;
+  return l;
+}
+static size_t bvh_nodes(int n) { return (((size_t)1 << (2 * bvh_levels(n))) - 1) / 3; }
+
+static void bvh_build(const std::vector<DInstance>& inst, std::vector<DBvhNode>& nodes) {
   const int n = (int)inst.size();
-  idx.resize(n);
+  std::vector<int32_t> idx(n);
   for (int i = 0; i < n; ++i) idx[i] = i;
-  nodes.clear();
-  nodes.reserve(2 * (size_t)n);
+  DBvhNode none{};
+  for (int k = 0; k < 4; ++k) none.child[k] = kBvhEmpty;
+  nodes.assign(bvh_nodes(n), none);
   struct Build {
     const std::vector<DInstance>& inst;
     std::vector<DBvhNode>& nodes;
     std::vector<int32_t>& idx;
-    void run(int lo, int hi) {
-      const int me = (int)nodes.size();
-      nodes.push_back(DBvhNode{});
-      DBvhNode nd{};
-      float clo[3], chi[3];
+    void centres(int lo, int hi, float ext[3]) const {
       for (int a = 0; a < 3; ++a) {
-        nd.lo[a] = clo[a] = INFINITY;
-        nd.hi[a] = chi[a] = -INFINITY;
-      }
-      for (int i = lo; i < hi; ++i) {
-        const DInstance& in = inst[idx[i]];
-        for (int a = 0; a < 3; ++a) {
-          nd.lo[a] = std::min(nd.lo[a], in.bb_min[a]);
-          nd.hi[a] = std::max(nd.hi[a], in.bb_max[a]);
-          const float c = 0.5f * (in.bb_min[a] + in.bb_max[a]);
-          clo[a] = std::min(clo[a], c);
-          chi[a] = std::max(chi[a], c);
+        float mn = INFINITY, mx = -INFINITY;
+        for (int i = lo; i < hi; ++i) {
+          const float c = 0.5f * (inst[idx[i]].bb_min[a] + inst[idx[i]].bb_max[a]);
+          mn = std::min(mn, c);
+          mx = std::max(mx, c);
         }
+        ext[a] = mx - mn;
       }
-      if (hi - lo <= 4) {
-        nd.leaf = (lo << 3) | (hi - lo);
-        nd.skip = me + 1;
-        nodes[me] = nd;
-        return;
-      }
-      int ax = 0;
-      for (int a = 1; a < 3; ++a)
-        if (chi[a] - clo[a] > chi[ax] - clo[ax]) ax = a;
+    }
+    static int longest(const float e[3]) { return e[0] >= e[1] ? (e[0] >= e[2] ? 0 : 2) : (e[1] >= e[2] ? 1 : 2); }
+    int halve(int lo, int hi, int ax) {
       const int mid = (lo + hi) / 2;
       std::nth_element(idx.begin() + lo, idx.begin() + mid, idx.begin() + hi, [&](int32_t x, int32_t y) {
         const float cx = inst[x].bb_min[ax] + inst[x].bb_max[ax], cy = inst[y].bb_min[ax] + inst[y].bb_max[ax];
         return cx < cy || (cx == cy && x < y);
       });
-      nd.leaf = -1;
-      run(lo, mid);
-      run(mid, hi);
-      nd.skip = (int)nodes.size();
-      nodes[me] = nd;
+      return mid;
+    }
+    void run(int level, size_t q, int lo, int hi) {
+      DBvhNode nd{};
+      int r[5] = {lo, 0, 0, 0, hi};
+      float e[3];
+      centres(lo, hi, e);
+      nd.axis0 = longest(e);
+      r[2] = halve(lo, hi, nd.axis0);
+      float e0[3], e1[3];
+      centres(lo, r[2], e0);
+      centres(r[2], hi, e1);
+      for (int a = 0; a < 3; ++a) e[a] = std::max(e0[a], e1[a]);
+      nd.axis1 = longest(e);
+      r[1] = halve(lo, r[2], nd.axis1);
+      r[3] = halve(r[2], hi, nd.axis1);
+      for (int k = 0; k < 4; ++k) {
+        const int cnt = r[k + 1] - r[k];
+        for (int a = 0; a < 3; ++a) {
+          nd.lo[a][k] = INFINITY;
+          nd.hi[a][k] = -INFINITY;
+          for (int i = r[k]; i < r[k + 1]; ++i) {
+            nd.lo[a][k] = std::min(nd.lo[a][k], inst[idx[i]].bb_min[a]);
+            nd.hi[a][k] = std::max(nd.hi[a][k], inst[idx[i]].bb_max[a]);
+          }
+        }
+        nd.child[k] = cnt == 0 ? kBvhEmpty : (cnt == 1 ? idx[r[k]] : kBvhInner);
+        if (cnt > 1) run(level + 1, 4 * q + k, r[k], r[k + 1]);
+      }
+      nodes[((((size_t)1 << (2 * level)) - 1) / 3) + q] = nd;
     }
   } b{inst, nodes, idx};
-  if (n > 0) b.run(0, n);
+  b.run(0, 0, 0, n);
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 size_t HostScene::device_bytes() const {
   return align256(sizeof(DScene)) + align256(inst.size() * sizeof(DInstance)) +
-         align256(bvh.size() * sizeof(DBvhNode)) + align256(bvh_idx.size() * sizeof(int32_t));
+         align256(bvh.size() * sizeof(DBvhNode));
 }
 
 void HostScene::pack(void* dev, std::vector<unsigned char>& out) const {
   out.assign(device_bytes(), 0);
   const size_t o_inst = align256(sizeof(DScene));
   const size_t o_bvh = o_inst + align256(inst.size() * sizeof(DInstance));
-  const size_t o_idx = o_bvh + align256(bvh.size() * sizeof(DBvhNode));
   DScene d = s;
   char* base = (char*)dev;
   d.inst = (const DInstance*)(base + o_inst);
   d.bvh = bvh.empty() ? nullptr : (const DBvhNode*)(base + o_bvh);
-  d.bvh_idx = bvh_idx.empty() ? nullptr : (const int32_t*)(base + o_idx);
   memcpy(out.data(), &d, sizeof(DScene));
   if (!inst.empty()) memcpy(out.data() + o_inst, inst.data(), inst.size() * sizeof(DInstance));
   if (!bvh.empty()) memcpy(out.data() + o_bvh, bvh.data(), bvh.size() * sizeof(DBvhNode));
-  if (!bvh_idx.empty()) memcpy(out.data() + o_idx, bvh_idx.data(), bvh_idx.size() * sizeof(int32_t));
 }
 
 size_t scene_bytes_for(int n_inst) {
   HostScene h;
   h.inst.resize(n_inst);
-  if (n_inst > kLinearInstances) {
-    h.bvh.resize(2 * (size_t)n_inst);
-    h.bvh_idx.resize(n_inst);
-  }
+  if (n_inst > kLinearInstances) h.bvh.resize(bvh_nodes(n_inst));
   return h.device_bytes();
 }
 
@@ -211,7 +224,6 @@ int build_scene(r2_ctx* ctx, const r2_render_params* p, HostScene* hs) {
   if (!p->env) return fail(ctx, R2_ERR_INVALID, "render: an environment map is required (config Scene.Envmap)");
   hs->inst.clear();
   hs->bvh.clear();
-  hs->bvh_idx.clear();
   DScene& s = hs->s;
   memset(&s, 0, sizeof(s));
   s.W = p->width; s.H = p->height; s.spp = p->spp; s.max_depth = p->max_depth;
@@ -270,7 +282,7 @@ int build_scene(r2_ctx* ctx, const r2_render_params* p, HostScene* hs) {
   }
   if (hs->precision == -2) hs->precision = 0;
   if (p->n_instances > kLinearInstances) {
-    bvh_build(hs->inst, hs->bvh, hs->bvh_idx);
+    bvh_build(hs->inst, hs->bvh);
     s.n_bvh = (int32_t)hs->bvh.size();
   }
   // analytic surfaces (CHostSceneobject(shape, material ...), sceneobject.cu:28-48)

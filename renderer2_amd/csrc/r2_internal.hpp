@@ -92,7 +92,6 @@ struct HostScene {
   r2::DScene s{};
   std::vector<r2::DInstance> inst;
   std::vector<r2::DBvhNode> bvh;
-  std::vector<int32_t> bvh_idx;
   int precision = 0;
   size_t device_bytes() const;
   // the device image for base address `dev`: the scene with its table pointers

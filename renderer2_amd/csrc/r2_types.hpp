@@ -88,22 +88,28 @@ struct DSurface {
   float alpha_x, alpha_y, eta_i, eta_t;
 };
 
-// Node of the instance hierarchy, in depth-first order: the box of its
-// subtree, the index of the node after the subtree, and for a leaf
-// (first << 3 | count) into DScene::bvh_idx (count 1..4); -1 for an inner node.
-struct DBvhNode {
-  float lo[3];
-  int32_t skip;
-  float hi[3];
-  int32_t leaf;
+// Node of the instance hierarchy: the boxes of its four children per axis, so that a
+// lane tests all four from seven 16-byte loads.  child: an instance (>= 0, then the
+// box is the instance's own), kBvhInner for a node, kBvhEmpty.  Children 0, 1 lie
+// before children 2, 3 along axis0, and 0 before 1, 2 before 3 along axis1.  Nodes
+// are numbered as in a full 4-ary tree, level l from (4^l - 1) / 3 on, child k of
+// the q-th node of a level being the (4 q + k)-th of the next: a walk needs no
+// child indices and climbs by shifts.
+constexpr int32_t kBvhInner = -1, kBvhEmpty = -2;
+constexpr int kBvhMaxLevels = 10;  // 4^10 = kMaxInstances
+struct alignas(128) DBvhNode {
+  float lo[3][4], hi[3][4];
+  int32_t child[4];
+  int32_t axis0, axis1;
+  int32_t pad[2];
 };
+static_assert(sizeof(DBvhNode) == 128, "one 128-byte line per node");
 
 struct DScene {
   int32_t n_inst;
   const DInstance* inst;     // n_inst instances (device memory, after the scene)
   int32_t n_bvh;             // 0: linear scan
   const DBvhNode* bvh;
-  const int32_t* bvh_idx;
   int32_t n_grid;
   DGrid grid[kMaxGrids];
   int32_t n_surf;

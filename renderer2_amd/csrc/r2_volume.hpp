@@ -741,34 +741,89 @@ __device__ __forceinline__ bool instance_box_t(const float* bmin, const float* b
   t_out = inside ? t1 : t0;
   return true;
 }
-// Culling test of a hierarchy node: the same rejections as instance_box_t on
-// the node's box, which contains its instances' boxes.  Each rejection compares
-// an entry against an exit, and a contained box has a later (or equal) entry
-// and an earlier (or equal) exit under the same rounded arithmetic, so a node
-// is rejected only when all its instances are (comparisons with NaN never
-// reject).  The node is also skipped when its entry lies beyond `cur`: every
-// instance inside then reports a larger t.
-__device__ __forceinline__ bool node_may_hit(const DBvhNode& nd, const float o[3], const float inv[3], int sg0,
-                                             int sg1, int sg2, float cur) {
-  const float* bmin = nd.lo;
-  const float* bmax = nd.hi;
-  float t0 = ((sg0 ? bmax : bmin)[0] - o[0]) * inv[0];
-  float t2 = ((sg1 ? bmin : bmax)[1] - o[1]) * inv[1];
-  if (t0 > t2) return false;
-  float t1 = ((sg0 ? bmin : bmax)[0] - o[0]) * inv[0];
-  float t3 = ((sg1 ? bmax : bmin)[1] - o[1]) * inv[1];
-  if (t3 > t1) return false;
-  if (t3 > t0) t0 = t3;
-  if (t2 < t1) t1 = t2;
-  t3 = ((sg2 ? bmax : bmin)[2] - o[2]) * inv[2];
-  if (t3 > t1) return false;
-  t2 = ((sg2 ? bmin : bmax)[2] - o[2]) * inv[2];
-  if (t0 > t2) return false;
-  if (t3 > t0) t0 = t3;
-  if (kDefaultTmax < t0) return false;
-  if (t2 < t1) t1 = t2;
-  if (0.f > t1) return false;
-  return !(t0 > cur);
+// The closest instance box of a ray through the hierarchy.  A child that is an
+// instance takes the test of instance_box_t on its own box; a node is culled by the
+// same rejections on its box, which contains its instances' boxes: each compares an
+// entry against an exit, and a contained box has a later (or equal) entry and an
+// earlier (or equal) exit under the same rounded arithmetic, so a node is rejected
+// only when all its instances are (comparisons with NaN never reject).  A node is
+// also culled when its entry lies beyond the closest hit so far: every instance
+// inside then reports a larger t.  So the result is that of a scan over all
+// instances: the smallest t, the lowest index among equal t.
+//
+// Bound by the chain of dependent node loads, 64 lanes at different nodes: nodes of
+// four children (the walk of a binary tree with four-instance leaves behind an index
+// table loaded two to three times as often), visited front to back, so that the
+// closest box culls the rest.  `pend` holds six bits per level: the children still
+// to visit, in visiting order (k ^ code), and that level's code.
+__device__ __forceinline__ void bvh_closest(const DScene& s, const float o[3], const float inv[3], int sg0, int sg1,
+                                            int sg2, float best, Hit& h) {
+  const char* base = (const char*)&kconst_at(s.bvh, 0);
+  // byte offsets of the near and far planes of each axis in a node
+  const uint32_t n0 = sg0 ? 48u : 0u, n1 = sg1 ? 64u : 16u, n2 = sg2 ? 80u : 32u;
+  const uint32_t f0 = 48u - n0, f1 = 80u - n1, f2 = 112u - n2;
+  const int sg = sg0 | (sg1 << 1) | (sg2 << 2);
+  uint64_t pend = 0;
+  int level = 0;
+  uint32_t q = 0;
+  for (;;) {
+    const uint32_t node = (0x55555555u & ((1u << (2 * level)) - 1u)) + q;
+    const char* nd = base + (size_t)node * sizeof(DBvhNode);
+    const float4 a0 = *(const float4*)(nd + n0), a1 = *(const float4*)(nd + n1), a2 = *(const float4*)(nd + n2);
+    const float4 b0 = *(const float4*)(nd + f0), b1 = *(const float4*)(nd + f1), b2 = *(const float4*)(nd + f2);
+    const int4 ch = *(const int4*)(nd + 96);
+    const int2 ax = *(const int2*)(nd + 112);
+    const int code = (((sg >> ax.x) & 1) << 1) | ((sg >> ax.y) & 1);
+    uint32_t m = 0;
+    auto child = [&](int k, float nx, float ny, float nz, float fx, float fy, float fz, int c) {
+      if (c == kBvhEmpty) return;
+      float t0 = (nx - o[0]) * inv[0], t2 = (fy - o[1]) * inv[1];
+      bool rej = t0 > t2;
+      float t1 = (fx - o[0]) * inv[0], t3 = (ny - o[1]) * inv[1];
+      rej |= t3 > t1;
+      t0 = t3 > t0 ? t3 : t0;
+      t1 = t2 < t1 ? t2 : t1;
+      t3 = (nz - o[2]) * inv[2];
+      rej |= t3 > t1;
+      t2 = (fz - o[2]) * inv[2];
+      rej |= t0 > t2;
+      t0 = t3 > t0 ? t3 : t0;
+      rej |= kDefaultTmax < t0;
+      t1 = t2 < t1 ? t2 : t1;
+      rej |= 0.f > t1;
+      if (rej) return;
+      if (c < 0) {
+        if (!(t0 > (h.hit ? h.t : best))) m |= 1u << (k ^ code);
+        return;
+      }
+      t0 = 0.f > t0 ? 0.f : t0;
+      t1 = kDefaultTmax < t1 ? kDefaultTmax : t1;
+      if (!(t1 < kDefaultTmax)) return;
+      const bool inside = o[0] > fminf(nx, fx) && o[1] > fminf(ny, fy) && o[2] > fminf(nz, fz) &&
+                          o[0] < fmaxf(nx, fx) && o[1] < fmaxf(ny, fy) && o[2] < fmaxf(nz, fz);
+      const float t = inside ? t1 : t0;
+      if (!(t >= 0.f && t <= best)) return;
+      if (h.hit && !(t < h.t || (t == h.t && c < h.medium))) return;
+      h.hit = 1; h.t = t; h.medium = c;
+    };
+    child(0, a0.x, a1.x, a2.x, b0.x, b1.x, b2.x, ch.x);
+    child(1, a0.y, a1.y, a2.y, b0.y, b1.y, b2.y, ch.y);
+    child(2, a0.z, a1.z, a2.z, b0.z, b1.z, b2.z, ch.z);
+    child(3, a0.w, a1.w, a2.w, b0.w, b1.w, b2.w, ch.w);
+    pend |= (uint64_t)(m | ((uint32_t)code << 4)) << (6 * level);
+    // the deepest level with a child to visit
+    const uint64_t left = pend & 0x3CF3CF3CF3CF3CFull;
+    if (left == 0ull) break;
+    const int up = (63 - __clzll((long long)left)) / 6;
+    q >>= 2 * (level - up);
+    const uint32_t f = (uint32_t)(pend >> (6 * up));
+    const uint32_t j = (uint32_t)__ffs((int)(f & 15u)) - 1u;
+    q = 4u * q + (j ^ ((f >> 4) & 3u));
+    // the levels below are done; drop the child taken
+    pend &= (1ull << (6 * up + 6)) - 1ull;
+    pend &= ~(1ull << (6 * up + j));
+    level = up + 1;
+  }
 }
 
 // __intersection__volume (shaders.optix.cu:192-236) over the instance boxes, then
@@ -795,26 +850,7 @@ __device__ __forceinline__ Hit scene_intersect(const DScene& s, Ray& ray) {
       h.hit = 1; h.t = t; h.medium = k;
     }
   } else {
-    for (int i = 0; i < s.n_bvh;) {
-      const DBvhNode nd = kconst_at(s.bvh, i);
-      if (!node_may_hit(nd, o, inv, sg0, sg1, sg2, h.hit ? h.t : best)) {
-        i = nd.skip;
-        continue;
-      }
-      if (nd.leaf >= 0) {
-        const int first = nd.leaf >> 3, cnt = nd.leaf & 7;
-        for (int j = 0; j < cnt; ++j) {
-          const int k = kconst_at(s.bvh_idx, first + j);
-          const DInstance& in = inst_at(s, k);
-          float t;
-          if (!instance_box_t(in.bb_min, in.bb_max, o, inv, sg0, sg1, sg2, t)) continue;
-          if (!(t >= 0.f && t <= best)) continue;
-          if (h.hit && !(t < h.t || (t == h.t && k < h.medium))) continue;
-          h.hit = 1; h.t = t; h.medium = k;
-        }
-      }
-      ++i;
-    }
+    bvh_closest(s, o, inv, sg0, sg1, sg2, best, h);
   }
   if constexpr (kSurf) {
     for (int j = 0; j < s.n_surf; ++j) {
