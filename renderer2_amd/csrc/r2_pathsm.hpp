@@ -429,7 +429,9 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
   Ray r = cont ? p.ray : spawn_ray(p.ray.o, p.ray.d, cur);
   const Hit h = scene_intersect<kSurf, kSingle>(s, r);  // shortens r.tmax to the hit, as the reference's intersect does
   Ray tr = r;  // the ray of the traversal to start
-  int kind;
+  // a second intersection that both roles may need is made once for all lanes
+  Ray r2;
+  bool again = false;
   if (cont) {
     p.ray = r;
     p.si_pos = h.pos;
@@ -451,20 +453,10 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
         return;
       }
     } else {
-      Ray mr = mkray(h.pos, normalize(r.d), kDefaultTmax, h.medium);
-      ray_offset(mr, r.d);
-      const Hit se = scene_intersect<kSurf, kSingle>(s, mr);
-      if (!se.hit) {
-        cont_nohit(p);
-        return;
-      }
-      if (se.medium >= 0 && h.medium != se.medium) {
-        cont_done(p, CR_END);
-        return;
-      }
-      tr = mr;
+      r2 = mkray(h.pos, normalize(r.d), kDefaultTmax, h.medium);
+      ray_offset(r2, r.d);
+      again = true;
     }
-    kind = dda ? TK_FLIGHT_DDA : TK_FLIGHT_DELTA;
   } else {
     p.si_hit = h.hit;
     if (kSurf && h.surf >= 0) {  // intersectTr stops at a surface, whose zero emission zeroes the term
@@ -477,16 +469,32 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
       if (!h.hit) shadow_done(p);
       return;
     }
-    kind = dda ? TK_TR_DDA : TK_TR_RATIO;
     // The segment after this one starts at the box face, outside every medium,
     // toward p1.  Its scene intersection is made now (the same one, so the
     // same result); when it meets nothing (si_hit = 2 through the traversal),
     // the traversal's last step ends the walk without another segment pass.
     if (p.sh_seg < 64 + inst_extra(s)) {
-      Ray er = spawn_ray(p.ray.o, p.ray.d, p.ray.medium);
-      if (!scene_intersect<kSurf, kSingle>(s, er).hit) p.si_hit = 2;
+      r2 = spawn_ray(p.ray.o, p.ray.d, p.ray.medium);
+      again = true;
     }
   }
+  if (again) {
+    const Hit se = scene_intersect<kSurf, kSingle>(s, r2);
+    if (cont) {
+      if (!se.hit) {
+        cont_nohit(p);
+        return;
+      }
+      if (se.medium >= 0 && h.medium != se.medium) {
+        cont_done(p, CR_END);
+        return;
+      }
+      tr = r2;
+    } else if (!se.hit) {
+      p.si_hit = 2;
+    }
+  }
+  const int kind = cont ? (dda ? TK_FLIGHT_DDA : TK_FLIGHT_DELTA) : (dda ? TK_TR_DDA : TK_TR_RATIO);
   start_traversal<kSingle>(s, p, tr.medium, tr, kind);
 }
 
