@@ -10,12 +10,13 @@
 //                   pairs are counted (with the task's lane mask), then emitted
 //                   from the masks as 64-bit keys voxel<<32 | tri.
 //   3. radix sort + run-length encode: sorted candidate list per active voxel.
-//   4. k_filter     one wave per active voxel, the 64 lanes are the voxel's rays.
-//                   Every lane tests every candidate triangle (uniform loop; the
-//                   triangle is a wave-uniform load), keeps the lexicographic
-//                   minimum of (t, triangle index), and the per-ray sums are
-//                   reduced in ray order through LDS, so the record equals the
-//                   sequential loop of the reference bit for bit.
+//   4. k_filter     one wave per group of active voxels; voxel by voxel the 64 lanes
+//                   are the voxel's rays.  Every lane tests every candidate
+//                   triangle (uniform loop; the triangle is a wave-uniform load),
+//                   keeps the lexicographic minimum of (t, triangle index), and the
+//                   per-ray sums are reduced in ray order through LDS; then four
+//                   lanes per voxel estimate the densities of the whole group.  The
+//                   record equals the sequential loop of the reference bit for bit.
 // A voxel with no candidate cannot be hit by any of its rays: its record is the
 // no-hit record, written for all voxels up front by k_fill_empty.
 #include <hip/hip_runtime.h>
@@ -64,7 +65,6 @@ constexpr uint32_t kTag = 0xF17Eu;
 struct FConst {
   m43 i2m, m2w, w2m, i2w;  // indexToModel, modelToWorld, worldToModel, indexToWorld (mat4x3)
   m43 mesh_m2w;            // mesh object modelToWorld (hit normals)
-  m44 rs;                  // getRotation((1,0,0)) of the clip sphere
   int nx, ny, nz;
   float diagonal, tmax_fixed, radius;
   float reach;             // conservative distance from the voxel centre a ray can reach
@@ -224,11 +224,37 @@ __device__ __forceinline__ void range_voxel(const TriRange& r, unsigned long lon
 //     queue up per wave in LDS and take the exact test 64 at a time; a passing
 //     pair sets its bit in the task's mask with an LDS atomic OR.  Each task's
 //     mask and pair count then go to task_mask / task_cnt.
-//   kEmit = true: one wave per task, one bit per lane: the pairs of the stored
-//     mask are written from task_off[task] on, in lane order (no atomics: the
-//     scan of the counts places them), without testing again.
-constexpr int kTasksPerBlock = 256;
-template <bool kEmit>
+//   kEmit = true: the pairs of the stored masks, without testing again and without
+//     atomics (the scan of the counts places them).  A block's pairs are packed onto
+//     its lanes as in the test: a lane finds its task by binary search in the offsets
+//     and its voxel as the n-th bit of the mask, and neighbouring lanes write
+//     neighbouring keys.  (One wave per task, one lane per bit, left 60 of 64 lanes
+//     idle, a task holding four pairs: 585 us for 21.9 M pairs, now 110.)
+// kTasks: 256 tasks per block, 32 when that would make fewer than two blocks per CU
+// (8000 triangles: the test took 70 us in 31 blocks, 14 us in 250).
+constexpr int kTasksPerBlock = 256, kTasksPerSmallBlock = 32;
+// index of the n-th set bit (n < popcount)
+__device__ __forceinline__ int nth_bit(unsigned long long m, int n) {
+  uint32_t w = (uint32_t)m;
+  int base = 0;
+  const int c32 = __popc(w);
+  if (n >= c32) {
+    n -= c32;
+    w = (uint32_t)(m >> 32);
+    base = 32;
+  }
+#pragma unroll
+  for (int h = 16; h > 0; h >>= 1) {
+    const int c = __popc(w & ((1u << h) - 1u));
+    if (n >= c) {
+      n -= c;
+      w >>= h;
+      base += h;
+    }
+  }
+  return base;
+}
+template <bool kEmit, int kTasks>
 __global__ __launch_bounds__(256) void k_pairs(const float4* __restrict__ tri, FConst c,
                                                const TriRange* __restrict__ rng,
                                                const unsigned long long* __restrict__ task_begin,
@@ -237,23 +263,23 @@ __global__ __launch_bounds__(256) void k_pairs(const float4* __restrict__ tri, F
                                                unsigned long long* __restrict__ task_mask,
                                                const uint32_t* __restrict__ task_off,
                                                unsigned long long* __restrict__ keys) {
-  __shared__ uint32_t s_t[kTasksPerBlock];
-  __shared__ TriRange s_r[kTasksPerBlock];
-  __shared__ unsigned long long s_beg[kTasksPerBlock];
-  __shared__ unsigned long long s_mask[kTasksPerBlock];
-  __shared__ uint32_t s_off[kTasksPerBlock];  // emit: task_off; test: exclusive prefix of the voxel counts
+  __shared__ uint32_t s_t[kTasks];
+  __shared__ TriRange s_r[kTasks];
+  __shared__ unsigned long long s_beg[kTasks];
+  __shared__ unsigned long long s_mask[kTasks];
+  __shared__ uint32_t s_off[kTasks];  // emit: task_off; test: exclusive prefix of the voxel counts
   __shared__ uint32_t s_wsum[4];
-  __shared__ float4 s_tri[kEmit ? 1 : 3 * kTasksPerBlock];
-  __shared__ float4 s_sph[kEmit ? 1 : kTasksPerBlock];             // centroid, radius
+  __shared__ float4 s_tri[kEmit ? 1 : 3 * kTasks];
+  __shared__ float4 s_sph[kEmit ? 1 : kTasks];             // centroid, radius
   __shared__ uint32_t s_q[kEmit ? 1 : 4][kEmit ? 1 : 128];          // queued pairs: task << 8 | voxel
   __shared__ float4 s_qc[kEmit ? 1 : 4][kEmit ? 1 : 128];           // their voxel centres
   const int i = threadIdx.x, lane = i & 63;
   const int wave = __builtin_amdgcn_readfirstlane(i >> 6);
-  const unsigned long long base = (unsigned long long)blockIdx.x * kTasksPerBlock;
+  const unsigned long long base = (unsigned long long)blockIdx.x * kTasks;
   const unsigned long long mine = base + (unsigned long long)i;
-  const int nk = (int)(n_tasks - base < (unsigned long long)kTasksPerBlock ? n_tasks - base : kTasksPerBlock);
+  const int nk = (int)(n_tasks - base < (unsigned long long)kTasks ? n_tasks - base : kTasks);
   uint32_t act = 0;  // voxels of this thread's task
-  if (mine < n_tasks) {
+  if (i < kTasks && mine < n_tasks) {
     const uint32_t t = task_tri[mine];
     const TriRange r = rng[t];
     const unsigned long long beg = task_begin[t];
@@ -280,16 +306,19 @@ __global__ __launch_bounds__(256) void k_pairs(const float4* __restrict__ tri, F
   }
   if (kEmit) {
     __syncthreads();
-    for (int k = wave; k < nk; k += (int)(blockDim.x >> 6)) {
-      const unsigned long long ball = s_mask[k];
-      if ((ball >> lane) & 1ull) {
-        int ix, iy, iz;
-        range_voxel(s_r[k], (base + (unsigned long long)k - s_beg[k]) * 64ull + (unsigned long long)lane, ix, iy, iz);
-        const uint32_t vid = (uint32_t)ix + (uint32_t)c.nx * ((uint32_t)iy + (uint32_t)c.ny * (uint32_t)iz);
-        const unsigned long long slot =
-            (unsigned long long)s_off[k] + (unsigned long long)__popcll(ball & ((1ull << lane) - 1ull));
-        keys[slot] = ((unsigned long long)vid << 32) | (unsigned long long)s_t[k];
+    const uint32_t first = s_off[0];
+    const uint32_t total = s_off[nk - 1] - first + (uint32_t)__popcll(s_mask[nk - 1]);
+    for (uint32_t p = (uint32_t)i; p < total; p += 256u) {
+      int lo = 0, hi = nk - 1;  // last task with offset <= first + p: the others of equal offset before it are empty
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s_off[mid] - first <= p) lo = mid; else hi = mid - 1;
       }
+      const int bit = nth_bit(s_mask[lo], (int)(p - (s_off[lo] - first)));
+      int ix, iy, iz;
+      range_voxel(s_r[lo], (base + (unsigned long long)lo - s_beg[lo]) * 64ull + (unsigned long long)bit, ix, iy, iz);
+      const uint32_t vid = (uint32_t)ix + (uint32_t)c.nx * ((uint32_t)iy + (uint32_t)c.ny * (uint32_t)iz);
+      keys[(unsigned long long)first + p] = ((unsigned long long)vid << 32) | (unsigned long long)s_t[lo];
     }
     return;
   }
@@ -307,7 +336,7 @@ __global__ __launch_bounds__(256) void k_pairs(const float4* __restrict__ tri, F
     if (w < wave) wbase += s_wsum[w];
     total += s_wsum[w];
   }
-  s_off[i] = wbase + incl - act;
+  if (i < kTasks) s_off[i] = wbase + incl - act;
   __syncthreads();
   // the block's (task, voxel) pairs, 64 per wave step: sphere test, then the
   // survivors through the per-wave queue to the exact test
@@ -377,7 +406,7 @@ __global__ __launch_bounds__(256) void k_pairs(const float4* __restrict__ tri, F
     exact(qn);
   }
   __syncthreads();
-  if (mine < n_tasks) {
+  if (i < kTasks && mine < n_tasks) {
     task_mask[mine] = s_mask[i];
     task_cnt[mine] = (uint32_t)__popcll(s_mask[i]);
   }
@@ -422,10 +451,15 @@ __device__ __forceinline__ void ray_uniforms(uint32_t seed, uint32_t lod, uint32
   }
 }
 
-// Sphere::intersect of a world-space ray (sphere.hpp:33-90); 0 on a miss
-__device__ float sphere_exit(const m43& w2m_s, float radius, v3 o, v3 d, float ray_tmax) {
-  const v3 mo = mul_point(w2m_s, o);
-  const v3 md = normalize(mul_dir(w2m_s, d));
+// Sphere::intersect of a world-space ray (sphere.hpp:33-90); 0 on a miss.  The sphere's
+// model transform is translate(ctr) * getRotation((1,0,0)), whose rotation rounds to
+// the axis exchange (x, y, z) -> (-y, x, z).  Its 4x4 inverse holds only zeros, ones and
+// components of ctr, and multiplying by it adds zeros to one difference per
+// coordinate, so the transformed ray is written out: the same numbers without a
+// matrix product and inverse per voxel (about 400 of 2150 instructions).
+__device__ __forceinline__ float sphere_exit(v3 ctr, float radius, v3 o, v3 d, float ray_tmax) {
+  const v3 mo = mk(o.y - ctr.y, ctr.x - o.x, o.z - ctr.z);
+  const v3 md = normalize(mk(d.y, -d.x, d.z));
   const float a = dot(md, md);
   const float b = 2.0f * dot(md, mo);
   const float cc = dot(mo, mo) - radius * radius;
@@ -446,43 +480,51 @@ __device__ float sphere_exit(const m43& w2m_s, float radius, v3 o, v3 d, float r
   return 0.f;
 }
 
-// watertight ray/triangle test (Woop, Benthin, Wald, JCGT 2(1) 2013)
+// watertight ray/triangle test (Woop, Benthin, Wald, JCGT 2(1) 2013).  The ray's axes
+// are kz (its longest) and the two that follow it, kx and ky.  The published test
+// swaps kx and ky for a ray along -kz; that negates U, V, W, their sum and T, which
+// leaves every decision, the distance and the barycentric weights as they are, so
+// no ray swaps here.
 struct WRay {
-  int kx, ky, kz;
+  int kz;
+  float ox, oy, oz;  // origin's kx, ky, kz components
   float Sx, Sy, Sz;
 };
-__device__ __forceinline__ WRay wt_setup(v3 d) {
+__device__ __forceinline__ WRay wt_setup(v3 o, v3 d) {
   WRay w;
   const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
   w.kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
-  w.kx = w.kz + 1 == 3 ? 0 : w.kz + 1;
-  w.ky = w.kx + 1 == 3 ? 0 : w.kx + 1;
-  if (comp(d, w.kz) < 0.f) {
-    const int t = w.kx;
-    w.kx = w.ky;
-    w.ky = t;
-  }
-  w.Sx = comp(d, w.kx) / comp(d, w.kz);
-  w.Sy = comp(d, w.ky) / comp(d, w.kz);
-  w.Sz = 1.f / comp(d, w.kz);
+  const int kx = w.kz + 1 == 3 ? 0 : w.kz + 1;
+  const int ky = kx + 1 == 3 ? 0 : kx + 1;
+  w.ox = comp(o, kx);
+  w.oy = comp(o, ky);
+  w.oz = comp(o, w.kz);
+  const float dz = comp(d, w.kz);
+  w.Sx = comp(d, kx) / dz;
+  w.Sy = comp(d, ky) / dz;
+  w.Sz = 1.f / dz;
   return w;
 }
-__device__ __forceinline__ bool wt_hit(const WRay& w, v3 o, v3 v0, v3 v1, v3 v2, float tmax, float* t, float* b1,
-                                       float* b2) {
-  const v3 A = v0 - o, B = v1 - o, Cc = v2 - o;
-  const float Ax = comp(A, w.kx) - w.Sx * comp(A, w.kz), Ay = comp(A, w.ky) - w.Sy * comp(A, w.kz);
-  const float Bx = comp(B, w.kx) - w.Sx * comp(B, w.kz), By = comp(B, w.ky) - w.Sy * comp(B, w.kz);
-  const float Cx = comp(Cc, w.kx) - w.Sx * comp(Cc, w.kz), Cy = comp(Cc, w.ky) - w.Sy * comp(Cc, w.kz);
+// a triangle's vertices as a ray sees them: (kx, ky, kz) components, and its index
+struct WTri {
+  float4 a, b, c;  // A.x A.y A.z B.x | B.y B.z C.x C.y | C.z index - -
+};
+__device__ __forceinline__ bool wt_hit(const WRay& w, const WTri& q, float tmax, float* t, float* b1, float* b2) {
+  const float Akz = q.a.z - w.oz, Bkz = q.b.y - w.oz, Ckz = q.c.x - w.oz;
+  const float Ax = (q.a.x - w.ox) - w.Sx * Akz, Ay = (q.a.y - w.oy) - w.Sy * Akz;
+  const float Bx = (q.a.w - w.ox) - w.Sx * Bkz, By = (q.b.x - w.oy) - w.Sy * Bkz;
+  const float Cx = (q.b.z - w.ox) - w.Sx * Ckz, Cy = (q.b.w - w.oy) - w.Sy * Ckz;
   float U = Cx * By - Cy * Bx, V = Ax * Cy - Ay * Cx, W = Bx * Ay - By * Ax;
-  if (U == 0.f || V == 0.f || W == 0.f) {
+  if (fminf(fminf(fabsf(U), fabsf(V)), fabsf(W)) == 0.f) {
     U = (float)((double)Cx * (double)By - (double)Cy * (double)Bx);
     V = (float)((double)Ax * (double)Cy - (double)Ay * (double)Cx);
     W = (float)((double)Bx * (double)Ay - (double)By * (double)Ax);
   }
-  if ((U < 0.f || V < 0.f || W < 0.f) && (U > 0.f || V > 0.f || W > 0.f)) return false;
+  // some negative and some positive (fminf and fmaxf pass over a NaN)
+  if (fminf(fminf(U, V), W) < 0.f && fmaxf(fmaxf(U, V), W) > 0.f) return false;
   const float det = U + V + W;
   if (det == 0.f) return false;
-  const float Az = w.Sz * comp(A, w.kz), Bz = w.Sz * comp(B, w.kz), Cz = w.Sz * comp(Cc, w.kz);
+  const float Az = w.Sz * Akz, Bz = w.Sz * Bkz, Cz = w.Sz * Ckz;
   const float T = U * Az + V * Bz + W * Cz;
   if (det < 0.f && (T >= 0.f || T < tmax * det)) return false;
   if (det > 0.f && (T <= 0.f || T > tmax * det)) return false;
@@ -584,10 +626,47 @@ __device__ __forceinline__ v3 hit_normal(const FConst& c, const int32_t* __restr
   return normalize(mul_dir(c.mesh_m2w, n));
 }
 
-// one wave per work voxel.  direct: work[w] indexes act/off/cnt; otherwise work
-// holds voxel ids, looked up in the sorted active list, and records go to out[w].
+// value of lane k (wave-uniform k) in every lane
+__device__ __forceinline__ int lane_i(int v, int k) { return __builtin_amdgcn_readlane(v, k); }
+__device__ __forceinline__ float lane_f(float v, int k) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), k));
+}
+// e + v of lane 0 + v of lane 1 + ... of the lane's quad, in that order (the quad's
+// four lanes all get the sum)
+__device__ __forceinline__ float quad_add_in_order(float e, float v) {
+  const int b = (int)__float_as_uint(v);
+  e += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(b, 0x00, 0xf, 0xf, true));
+  e += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(b, 0x55, 0xf, 0xf, true));
+  e += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(b, 0xaa, 0xf, 0xf, true));
+  e += __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(b, 0xff, 0xf, 0xf, true));
+  return e;
+}
+
+// One wave per group of up to kGroup consecutive work voxels.  direct: work[w] indexes
+// act/off/cnt; otherwise work holds voxel ids, looked up in the sorted active list,
+// and records go to out[w].
+//   * Lane g prepares voxel g of the group (id, candidate list, centre).
+//   * Voxel by voxel, the lanes cast its rays and the sums are taken (see above).  The
+//     candidates are staged in LDS, 32 at a time and one per lane, in the three
+//     orders of axes that rays use, so that a lane reads its order in three 16-byte
+//     loads (it took 18 selects per test before, behind two dependent scalar loads).
+//   * Four lanes per voxel (more when the group is small) run the density iteration,
+//     compute the hits' exp terms four at a time and add them in hit order; then they
+//     write the records.
+// What bounds it is VALU issue.  With one voxel per wave, the preparation, the eight
+// density iterations and the encoding took 1500 of 2150 instructions, all lanes doing
+// the same or most of them nothing (a voxel has some 20 hits); a group shares them.
+// 5.1 M voxels of 64 rays and 4.3 candidates: 15.0 -> 9.3 ms; 568 K voxels of 20
+// candidates: 2.98 -> 2.23 ms.  A wave's voxels lie n_waves apart, so that a stretch
+// of voxels with many candidates spreads over waves (consecutive ones: 4.6 ms there).
 // kTex: the mesh has texture coordinates or material textures (alpha test,
 // textured colours, normal maps); without, the kernel carries none of that code.
+constexpr int kGroup = 16;        // voxels of a wave's density pass, four lanes each
+constexpr int kTsFloats = 1024;   // clip distances a wave's group may hold (kGroup * 64; a voxel has up to 1000)
+constexpr int kStage = 32;        // candidate triangles staged at a time (9 float4 each)
+static_assert(kStage * 9 * 4 <= kVals * kRow, "the staged triangles share the space of the per-hit values");
+static_assert(kTsFloats <= kVals * kRow, "so do the exp terms of the density iteration");
+constexpr int kSumRow = 19;       // per voxel: the kVals sums, the hit count; odd, so that rows fall on distinct banks
 template <bool kTex>
 __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __restrict__ work, uint32_t n_work,
                                                 int direct, const uint32_t* __restrict__ act,
@@ -596,195 +675,217 @@ __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __rest
                                                 const float4* __restrict__ tri, const int32_t* __restrict__ tidx,
                                                 const float* __restrict__ nrm, const int32_t* __restrict__ tmat,
                                                 const float* __restrict__ matf, uint4* __restrict__ out,
-                                                int ts_cap) {
+                                                int ts_cap, int group, int vshift, uint32_t n_waves) {
   extern __shared__ __align__(16) float lds[];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (uint32_t)wave));
-  if (w >= n_work) return;
+  const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (uint32_t)wave));
+  if (w0 >= n_waves) return;
+  const int ng = (int)((n_work - 1u - w0) / n_waves) + 1;  // voxels w0 + g n_waves < n_work
   // [kVals][kRow] per-hit values of a ray batch, value-major, hits compacted in
-  // ray order (later: the exp terms of the density iteration)
-  float* V = lds + wave * (kVals * kRow + ts_cap);
-  float* TS = V + kVals * kRow;  // [ts_cap] clip distances of the hits, in ray order
+  // ray order; before that the staged triangles of the batch
+  float* V = lds + wave * (kVals * kRow + group * (ts_cap + kSumRow));
+  float* TSG = V + kVals * kRow;            // [group][ts_cap] clip distances of the hits, in ray order
+  float* SUM = TSG + group * ts_cap;        // [group][kSumRow]
 
-  uint32_t vid, beg = 0, nc = 0;
-  size_t orec;
-  if (direct) {
-    vid = act[w];
-    beg = off[w];
-    nc = cnt[w];
-    orec = vid;
-  } else {
-    vid = work[w];
-    orec = w;
-    uint32_t lo = 0, hi = n_act;  // first active voxel >= vid
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (act[mid] < vid) lo = mid + 1; else hi = mid;
+  uint32_t vid = 0, beg = 0, nc = 0;
+  int ix = 0, iy = 0, iz = 0;
+  v3 ctr = mk(0.f, 0.f, 0.f);
+  if (lane < ng) {
+    if (direct) {
+      vid = act[w0 + (uint32_t)lane * n_waves];
+      beg = off[w0 + (uint32_t)lane * n_waves];
+      nc = cnt[w0 + (uint32_t)lane * n_waves];
+    } else {
+      vid = work[w0 + (uint32_t)lane * n_waves];
+      uint32_t lo = 0, hi = n_act;  // first active voxel >= vid
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (act[mid] < vid) lo = mid + 1; else hi = mid;
+      }
+      if (lo < n_act && act[lo] == vid) {
+        beg = off[lo];
+        nc = cnt[lo];
+      }
     }
-    if (lo < n_act && act[lo] == vid) {
-      beg = off[lo];
-      nc = cnt[lo];
-    }
+    ix = (int)(vid % (uint32_t)c.nx);
+    iy = (int)((vid / (uint32_t)c.nx) % (uint32_t)c.ny);
+    iz = (int)(vid / ((uint32_t)c.nx * (uint32_t)c.ny));
+    ctr = voxel_center(c, ix, iy, iz);
   }
-  vid = (uint32_t)__builtin_amdgcn_readfirstlane((int)vid);
-  beg = (uint32_t)__builtin_amdgcn_readfirstlane((int)beg);
-  nc = (uint32_t)__builtin_amdgcn_readfirstlane((int)nc);
-  const int ix = (int)(vid % (uint32_t)c.nx), iy = (int)((vid / (uint32_t)c.nx) % (uint32_t)c.ny),
-            iz = (int)(vid / ((uint32_t)c.nx * (uint32_t)c.ny));
-  const v3 ctr = voxel_center(c, ix, iy, iz);
-  // clip sphere: model = translate(ctr) * getRotation((1,0,0))
-  m44 Ts = identity44();
-  Ts.c[3][0] = ctr.x;
-  Ts.c[3][1] = ctr.y;
-  Ts.c[3][2] = ctr.z;
-  const m43 m2w_s = to43(mul44(Ts, c.rs));
-  const m43 w2m_s = to43(inverse44(to44(m2w_s)));
-
-  float acc = 0.f;  // lane q < kVals: running sum of quantity q over the hit rays, in ray order
-  uint32_t hits = 0;
-  for (int r0 = 0; r0 < c.n_samples; r0 += 64) {
-    const int i = r0 + lane;
-    const bool live = i < c.n_samples;
-    float u[5];
-    ray_uniforms(c.seed, c.lod, vid, i, u);
-    const v3 o = mul_point(c.i2w, mk((float)ix + u[0], (float)iy + u[1], (float)iz + u[2]));
-    const float z = 1.f - 2.f * u[3];
-    const float rr = sqrtf(gmax(0.f, 1.f - z * z));
-    const float phi = (float)(2.0 * 3.14159265358979323846 * (double)u[4]);
-    float sphi, cphi;
-    det_sincosf(phi, &sphi, &cphi);
-    const v3 d = mk(rr * cphi, rr * sphi, z);
-    const float cur_tmax = c.clip ? sphere_exit(w2m_s, c.radius, o, d, 1e12f) : c.tmax_fixed;
-    const WRay wr = wt_setup(d);
-    int best = -1;
-    float bt = 0.f, bb1 = 0.f, bb2 = 0.f;
-    for (uint32_t k = 0; k < nc; ++k) {
-      const uint32_t t = cand[beg + k];
-      const v3 p0 = f4v(tri[3 * t]), p1 = f4v(tri[3 * t + 1]), p2 = f4v(tri[3 * t + 2]);
-      float th, b1, b2;
-      if (live && wt_hit(wr, o, p0, p1, p2, cur_tmax, &th, &b1, &b2) &&
-          (!kTex || !c.alpha_on || hit_opaque(c, tidx, tmat, (int)t, b1, b2))) {
-        if (best < 0 || th < bt || (th == bt && (int)t < best)) {
-          best = (int)t;
-          bt = th;
-          bb1 = b1;
-          bb2 = b2;
+  for (int g = 0; g < ng; ++g) {
+    const uint32_t gvid = (uint32_t)lane_i((int)vid, g), gbeg = (uint32_t)lane_i((int)beg, g),
+                   gnc = (uint32_t)lane_i((int)nc, g);
+    const float gx = (float)lane_i(ix, g), gy = (float)lane_i(iy, g), gz = (float)lane_i(iz, g);
+    const v3 gctr = mk(lane_f(ctr.x, g), lane_f(ctr.y, g), lane_f(ctr.z, g));
+    float* TS = TSG + g * ts_cap;
+    float acc = 0.f;  // lane q < kVals: running sum of quantity q over the hit rays, in ray order
+    uint32_t hits = 0;
+    for (int r0 = 0; r0 < c.n_samples; r0 += 64) {
+      const int i = r0 + lane;
+      const bool live = i < c.n_samples;
+      float u[5];
+      ray_uniforms(c.seed, c.lod, gvid, i, u);
+      const v3 o = mul_point(c.i2w, mk(gx + u[0], gy + u[1], gz + u[2]));
+      const float z = 1.f - 2.f * u[3];
+      const float rr = sqrtf(gmax(0.f, 1.f - z * z));
+      const float phi = (float)(2.0 * 3.14159265358979323846 * (double)u[4]);
+      float sphi, cphi;
+      det_sincosf(phi, &sphi, &cphi);
+      const v3 d = mk(rr * cphi, rr * sphi, z);
+      const float cur_tmax = c.clip ? sphere_exit(gctr, c.radius, o, d, 1e12f) : c.tmax_fixed;
+      const WRay wr = wt_setup(o, d);
+      int best = -1;
+      float bt = 0.f, bb1 = 0.f, bb2 = 0.f;
+      for (uint32_t k0 = 0; k0 < gnc; k0 += kStage) {
+        const int nk = (int)min((uint32_t)kStage, gnc - k0);
+        if (lane < nk) {
+          const uint32_t t = cand[gbeg + k0 + (uint32_t)lane];
+          const float4 p0 = tri[3 * t], p1 = tri[3 * t + 1], p2 = tri[3 * t + 2];
+          const float id = __uint_as_float(t);
+          float4* q = reinterpret_cast<float4*>(V) + lane * 9;
+          q[0] = make_float4(p0.y, p0.z, p0.x, p1.y);  // kz = x
+          q[1] = make_float4(p1.z, p1.x, p2.y, p2.z);
+          q[2] = make_float4(p2.x, id, 0.f, 0.f);
+          q[3] = make_float4(p0.z, p0.x, p0.y, p1.z);  // kz = y
+          q[4] = make_float4(p1.x, p1.y, p2.z, p2.x);
+          q[5] = make_float4(p2.y, id, 0.f, 0.f);
+          q[6] = make_float4(p0.x, p0.y, p0.z, p1.x);  // kz = z
+          q[7] = make_float4(p1.y, p1.z, p2.x, p2.y);
+          q[8] = make_float4(p2.z, id, 0.f, 0.f);
         }
+        wave_sync();
+        if (live) {
+          const float4* q = reinterpret_cast<const float4*>(V) + 3 * wr.kz;
+          WTri cur{q[0], q[1], q[2]};
+          for (int k = 0; k < nk; ++k) {
+            // the next triangle is on its way while this one is tested
+            q += k + 1 < nk ? 9 : 0;
+            const WTri nxt{q[0], q[1], q[2]};
+            float th, b1, b2;
+            const int t = (int)__float_as_uint(cur.c.y);
+            if (wt_hit(wr, cur, cur_tmax, &th, &b1, &b2) &&
+                (!kTex || !c.alpha_on || hit_opaque(c, tidx, tmat, t, b1, b2))) {
+              if (best < 0 || th < bt || (th == bt && t < best)) {
+                best = t;
+                bt = th;
+                bb1 = b1;
+                bb2 = b2;
+              }
+            }
+            cur = nxt;
+          }
+        }
+        wave_sync();
       }
-    }
-    const bool hit = best >= 0;
-    float val[kVals];
-#pragma unroll
-    for (int q = 0; q < kVals; ++q) val[q] = 0.f;
-    if (hit) {
-      // closest-hit: the hit's texture coordinate (0 without texture coordinates) and
-      // normal (shaders.optix.cu:48-114)
-      int m = tmat ? tmat[best] : 0;
-      m = (m >= 0 && m < c.n_materials) ? m : 0;
-      const float* mf = matf + 8 * m;
-      const int4 mt = kTex && c.mtex ? c.mtex[m] : make_int4(-1, -1, -1, -1);
-      float2 tc = make_float2(0.f, 0.f);
-      if (kTex && c.uv) tc = tri_tc(c, tidx, best, bb1, bb2);
-      const v3 n = hit_normal(c, tidx, nrm, best, bb1, bb2, kTex && c.normal_on ? mt.z : -1, tc);
-      const float sg = mf[6];
-      // buildS(n, sigma) = n n^T + sigma (I - n n^T)  (sggx_phase_function.hpp:95-105)
-      const float xx = n.x * n.x, xy = n.x * n.y, xz = n.x * n.z, yy = n.y * n.y, yz = n.y * n.z, zz = n.z * n.z;
-      val[0] = xx + sg * (yy + zz);
-      val[1] = yy + sg * (xx + zz);
-      val[2] = zz + sg * (xx + yy);
-      val[3] = xy + sg * (-xy);
-      val[4] = xz + sg * (-xz);
-      val[5] = yz + sg * (-yz);
-      // CMaterial::diffuse / glossy (material.hpp:111-127): the texture at tc, else the constant
-      float4 dc = make_float4(mf[0], mf[1], mf[2], 0.f), gc = make_float4(mf[3], mf[4], mf[5], 0.f);
-      if (kTex && mt.x >= 0) dc = tex_fetch(c.texels, c.tex[mt.x], tc.x, tc.y);
-      if (kTex && mt.y >= 0) gc = tex_fetch(c.texels, c.tex[mt.y], tc.x, tc.y);
-      val[6] = dc.x;
-      val[7] = dc.y;
-      val[8] = dc.z;
-      val[9] = gc.x;
-      val[10] = gc.y;
-      val[11] = gc.z;
-      val[12] = n.x;
-      val[13] = n.y;
-      val[14] = n.z;
-      val[15] = mf[7];
-      val[16] = cur_tmax;
-    }
-    // the hit rays' values, compacted by hit rank (ray order) into rows of one
-    // value each; lane q < kVals then sums row q in order, four hits per load
-    const unsigned long long hb = __ballot(hit);
-    const uint32_t rank = (uint32_t)__popcll(hb & ((1ull << lane) - 1ull));
-    if (hit) {
-#pragma unroll
-      for (int q = 0; q < kVals; ++q) V[q * kRow + rank] = val[q];
-      TS[hits + rank] = cur_tmax;
-    }
-    wave_sync();
-    const uint32_t nh = (uint32_t)__popcll(hb);
-    if (lane < kVals) {
-      const float* row = V + lane * kRow;
-      const float4* row4 = reinterpret_cast<const float4*>(row);
-      uint32_t h = 0;
-      for (; h + 4u <= nh; h += 4u) {
-        const float4 v = row4[h >> 2];
-        acc += v.x;
-        acc += v.y;
-        acc += v.z;
-        acc += v.w;
+      const bool hit = best >= 0;
+      // the hit rays' values go, compacted by hit rank (ray order), into rows of one
+      // value each; lane q < kVals then sums row q in order, four hits per load
+      const unsigned long long hb = __ballot(hit);
+      const uint32_t rank = (uint32_t)__popcll(hb & ((1ull << lane) - 1ull));
+      if (hit) {
+        // closest-hit: the hit's texture coordinate (0 without texture coordinates) and
+        // normal (shaders.optix.cu:48-114)
+        int m = tmat ? tmat[best] : 0;
+        m = (m >= 0 && m < c.n_materials) ? m : 0;
+        const float* mf = matf + 8 * m;
+        const int4 mt = kTex && c.mtex ? c.mtex[m] : make_int4(-1, -1, -1, -1);
+        float2 tc = make_float2(0.f, 0.f);
+        if (kTex && c.uv) tc = tri_tc(c, tidx, best, bb1, bb2);
+        const v3 n = hit_normal(c, tidx, nrm, best, bb1, bb2, kTex && c.normal_on ? mt.z : -1, tc);
+        const float sg = mf[6];
+        float* v = V + rank;
+        // buildS(n, sigma) = n n^T + sigma (I - n n^T)  (sggx_phase_function.hpp:95-105)
+        const float xx = n.x * n.x, xy = n.x * n.y, xz = n.x * n.z, yy = n.y * n.y, yz = n.y * n.z, zz = n.z * n.z;
+        v[0 * kRow] = xx + sg * (yy + zz);
+        v[1 * kRow] = yy + sg * (xx + zz);
+        v[2 * kRow] = zz + sg * (xx + yy);
+        v[3 * kRow] = xy + sg * (-xy);
+        v[4 * kRow] = xz + sg * (-xz);
+        v[5 * kRow] = yz + sg * (-yz);
+        // CMaterial::diffuse / glossy (material.hpp:111-127): the texture at tc, else the constant
+        float4 dc = make_float4(mf[0], mf[1], mf[2], 0.f), gc = make_float4(mf[3], mf[4], mf[5], 0.f);
+        if (kTex && mt.x >= 0) dc = tex_fetch(c.texels, c.tex[mt.x], tc.x, tc.y);
+        if (kTex && mt.y >= 0) gc = tex_fetch(c.texels, c.tex[mt.y], tc.x, tc.y);
+        v[6 * kRow] = dc.x;
+        v[7 * kRow] = dc.y;
+        v[8 * kRow] = dc.z;
+        v[9 * kRow] = gc.x;
+        v[10 * kRow] = gc.y;
+        v[11 * kRow] = gc.z;
+        v[12 * kRow] = n.x;
+        v[13 * kRow] = n.y;
+        v[14 * kRow] = n.z;
+        v[15 * kRow] = mf[7];
+        v[16 * kRow] = cur_tmax;
+        TS[hits + rank] = cur_tmax;
       }
-      for (; h < nh; ++h) acc += row[h];
+      wave_sync();
+      const uint32_t nh = (uint32_t)__popcll(hb);
+      if (lane < kVals) {
+        const float* row = V + lane * kRow;
+        const float4* row4 = reinterpret_cast<const float4*>(row);
+        uint32_t h = 0;
+        for (; h + 4u <= nh; h += 4u) {
+          const float4 v = row4[h >> 2];
+          acc += v.x;
+          acc += v.y;
+          acc += v.z;
+          acc += v.w;
+        }
+        for (; h < nh; ++h) acc += row[h];
+      }
+      hits += nh;
+      wave_sync();
     }
-    hits += (uint32_t)__popcll(hb);
-    wave_sync();
+    if (lane < kVals) SUM[g * kSumRow + lane] = acc;
+    if (lane == kVals) SUM[g * kSumRow + kVals] = __uint_as_float(hits);
   }
-  float sum[kVals];
-#pragma unroll
-  for (int q = 0; q < kVals; ++q) sum[q] = __shfl(acc, q);
-
+  wave_sync();
+  // 2^vshift lanes per voxel: 4 for a full group, up to all 64 for a single voxel
+  const int g = lane >> vshift, j = lane & ((1 << vshift) - 1);
+  const uint32_t gvid = (uint32_t)__shfl((int)vid, g);
+  if (g >= ng) return;
+  const float* sum = SUM + g * kSumRow;
+  const uint32_t hits = __float_as_uint(sum[kVals]);
   uint32_t wout[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0x3C00u};
   if (hits > 0) {
     // estimateDensity (mesh_filter.hpp:182-204, 216-226)
+    const float* TS = TSG + g * ts_cap;
     const float avg = sum[16] / (float)hits;
     const float P = (float)hits / (float)c.n_samples;
     float dens = -det_logf(1.f - P) / (avg * c.sigma_t);
     const float na = c.alpha / c.sigma_t;
-    // with at most 64 rays, lane h keeps the clip distance of hit h in a register,
-    // computes its exp term and stores it to the wave's LDS area (free after the
-    // ray sums; 16-byte aligned); the hit-order sum reads four terms per load
-    const bool lane_sums = c.clip && c.n_samples <= 64;
-    const float ts_l = (lane_sums && (uint32_t)lane < hits) ? TS[lane] : 0.f;
     for (int it = 0; it < c.iterations; ++it) {
       float Pv;
-      if (lane_sums) {
-        V[lane] = (uint32_t)lane < hits ? det_expf(-dens * c.sigma_t * ts_l) : 0.f;
-        wave_sync();
-        const float4* V4 = reinterpret_cast<const float4*>(V);
+      if (c.clip) {
         float e = 0.f;
-        uint32_t h = 0;
-        for (; h + 4u <= hits; h += 4u) {
-          const float4 q = V4[h >> 2];
-          e += q.x;
-          e += q.y;
-          e += q.z;
-          e += q.w;
+        if (vshift == 2) {
+          // terms past the last hit are zeros, which leave the sum as it is
+          for (uint32_t h = 0; h < hits; h += 4u)
+            e = quad_add_in_order(e, h + (uint32_t)j < hits ? det_expf(-dens * c.sigma_t * TS[h + j]) : 0.f);
+        } else {
+          // few voxels: more lanes share the terms, which every lane then adds from LDS
+          float* E = V + g * ts_cap;
+          for (uint32_t h = (uint32_t)j; h < hits; h += 1u << vshift) E[h] = det_expf(-dens * c.sigma_t * TS[h]);
+          wave_sync();
+          uint32_t h = 0;
+          for (; h + 4u <= hits; h += 4u) {
+            const float4 q = *reinterpret_cast<const float4*>(E + h);
+            e += q.x;
+            e += q.y;
+            e += q.z;
+            e += q.w;
+          }
+          for (; h < hits; ++h) e += E[h];
+          wave_sync();
         }
-        for (; h < hits; ++h) e += V[h];
-        wave_sync();
-        Pv = 1.f - e / (float)hits;
-      } else if (c.clip) {
-        for (uint32_t h = (uint32_t)lane; h < hits; h += 64) V[h] = det_expf(-dens * c.sigma_t * TS[h]);
-        wave_sync();
-        float e = 0.f;
-        for (uint32_t h = 0; h < hits; ++h) e += V[h];
-        wave_sync();
         Pv = 1.f - e / (float)hits;
       } else {
         Pv = 1.f - det_expf(-dens * c.sigma_t * c.tmax_fixed);
       }
       // each iteration is a function of dens alone: once it returns dens unchanged
       // (bit for bit), every later one would too, so the remaining ones are skipped
-      // (the result is that of all iterations; dens is wave-uniform)
+      // (the result is that of all iterations; a voxel's lanes hold the same dens)
       const float nd = dens - na * (Pv - P);
       if (nd == dens) break;
       dens = nd;
@@ -797,7 +898,8 @@ __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __rest
     const float nv[3] = {nm.x, nm.y, nm.z};
     encode_record(dens, S6, dif, spec, nv, sum[15] * ih, wout);
   }
-  if (lane == 0) {
+  if (j == 0) {
+    const size_t orec = direct ? (size_t)gvid : (size_t)w0 + (size_t)g * n_waves;
     out[2 * orec] = make_uint4(wout[0], wout[1], wout[2], wout[3]);
     out[2 * orec + 1] = make_uint4(wout[4], wout[5], wout[6], wout[7]);
   }
@@ -870,7 +972,6 @@ FConst make_consts(const r2_mesh* m, const r2_filter_grid& g, const r2_filter_pa
   memcpy(c.w2m.m, g.world_to_model, sizeof(float) * 12);
   c.i2w = to43(mul44(to44(c.m2w), to44(c.i2m)));
   c.mesh_m2w = m->m2w;
-  c.rs = r2host::get_rotation(mk(1.f, 0.f, 0.f));
   c.nx = g.num_voxels[0];
   c.ny = g.num_voxels[1];
   c.nz = g.num_voxels[2];
@@ -970,14 +1071,17 @@ int bin_triangles(r2_ctx* ctx, const r2_mesh* m, const FConst& c, Binning* B) {
   R2F_HIP(hipcub::DeviceScan::InclusiveScan(nullptr, tb, mark, task_tri, hipcub::Max(), nt, s), "filter: scan size");
   R2F_HIP(r2host::pool_get(ctx, kSlotTemp, tb, &tmp), "filter: alloc scan temp");
   R2F_HIP(hipcub::DeviceScan::InclusiveScan(tmp, tb, mark, task_tri, hipcub::Max(), nt, s), "filter: task map");
-  const dim3 grid((unsigned)((B->n_tasks + kTasksPerBlock - 1) / kTasksPerBlock));
+  const bool small = B->n_tasks < (unsigned long long)kTasksPerBlock * 2u * (unsigned)r2host::num_cus(ctx);
+  const int per_block = small ? kTasksPerSmallBlock : kTasksPerBlock;
+  const dim3 grid((unsigned)((B->n_tasks + per_block - 1) / per_block));
   uint32_t *task_cnt = nullptr, *task_off = nullptr;
   unsigned long long* task_mask = nullptr;
   R2F_HIP(pooled(ctx, kSlotTaskCnt, nt, &task_cnt), "filter: alloc task counts");
   R2F_HIP(pooled(ctx, kSlotTaskOff, nt, &task_off), "filter: alloc task offsets");
   R2F_HIP(pooled(ctx, kSlotTaskMask, nt, &task_mask), "filter: alloc task masks");
-  hipLaunchKernelGGL(k_pairs<false>, grid, dim3(256), 0, s, m->tri, c, rng, begin, task_tri, B->n_tasks, task_cnt,
-                     task_mask, (const uint32_t*)nullptr, (unsigned long long*)nullptr);
+  const auto count_pairs = small ? k_pairs<false, kTasksPerSmallBlock> : k_pairs<false, kTasksPerBlock>;
+  hipLaunchKernelGGL(count_pairs, grid, dim3(256), 0, s, m->tri, c, rng, begin, task_tri, B->n_tasks, task_cnt, task_mask,
+                     (const uint32_t*)nullptr, (unsigned long long*)nullptr);
   R2F_HIP(hipGetLastError(), "filter: k_pairs count");
   R2F_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, task_cnt, task_off, nt, s), "filter: scan size");
   R2F_HIP(r2host::pool_get(ctx, kSlotTemp, tb, &tmp), "filter: alloc scan temp");
@@ -996,8 +1100,9 @@ int bin_triangles(r2_ctx* ctx, const r2_mesh* m, const FConst& c, Binning* B) {
   unsigned long long *keys = nullptr, *keys2 = nullptr;
   R2F_HIP(pooled(ctx, kSlotKeys, np, &keys), "filter: alloc keys");
   R2F_HIP(pooled(ctx, kSlotKeys2, np, &keys2), "filter: alloc keys");
-  hipLaunchKernelGGL(k_pairs<true>, grid, dim3(256), 0, s, m->tri, c, rng, begin, task_tri, B->n_tasks, task_cnt,
-                     task_mask, (const uint32_t*)task_off, keys);
+  const auto emit_pairs = small ? k_pairs<true, kTasksPerSmallBlock> : k_pairs<true, kTasksPerBlock>;
+  hipLaunchKernelGGL(emit_pairs, grid, dim3(256), 0, s, m->tri, c, rng, begin, task_tri, B->n_tasks, task_cnt, task_mask,
+                     (const uint32_t*)task_off, keys);
   R2F_HIP(hipGetLastError(), "filter: k_pairs emit");
   const unsigned long long nvox = (unsigned long long)c.nx * c.ny * c.nz;
   int vbits = 1;
@@ -1040,15 +1145,25 @@ int launch_filter(r2_ctx* ctx, const r2_mesh* m, const FConst& c, const Binning&
     return R2_OK;
   }
   const int ts_cap = ((c.n_samples + 63) / 64) * 64;
-  const size_t lds = sizeof(float) * kWaves * (kVals * kRow + ts_cap);
-  const unsigned blocks = (n_work + kWaves - 1) / kWaves;
+  // voxels per wave: as many as the LDS for clip distances and the density pass's
+  // lanes allow, fewer when there are not 16 waves per CU to make of them
+  const uint32_t fill = (uint32_t)r2host::num_cus(ctx) * 16u;
+  const int group = (int)std::max<uint32_t>(
+      1u, std::min<uint32_t>(std::min<uint32_t>(kGroup, (uint32_t)(kTsFloats / ts_cap)), n_work / fill));
+  const size_t lds = sizeof(float) * kWaves * (kVals * kRow + group * (ts_cap + kSumRow));
+  int vshift = 6;  // 2^vshift lanes per voxel of the density pass
+  while ((group << vshift) > 64) --vshift;
+  const uint32_t n_waves = (n_work + (uint32_t)group - 1u) / (uint32_t)group;
+  const unsigned blocks = (n_waves + kWaves - 1) / kWaves;
   R2F_HIP(hipEventRecord(ctx->ev0, ctx->stream), "filter: event");
   if (c.uv || c.mtex)
     hipLaunchKernelGGL(k_filter<true>, dim3(blocks), dim3(256), lds, ctx->stream, c, work, n_work, direct ? 1 : 0,
-                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, ts_cap);
+                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, ts_cap, group,
+                       vshift, n_waves);
   else
     hipLaunchKernelGGL(k_filter<false>, dim3(blocks), dim3(256), lds, ctx->stream, c, work, n_work, direct ? 1 : 0,
-                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, ts_cap);
+                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, ts_cap, group,
+                       vshift, n_waves);
   R2F_HIP(hipGetLastError(), "filter: k_filter");
   R2F_HIP(hipEventRecord(ctx->ev1, ctx->stream), "filter: event");
   R2F_HIP(hipEventSynchronize(ctx->ev1), "filter: sync");

@@ -149,6 +149,8 @@ int build_scene(r2_ctx* ctx, const r2_render_params* p, HostScene* out);
 // scene-intersection probe (r2_grid.hip): n x (hit, t, instance, surface)
 int scene_intersect_probe(r2_ctx* ctx, const HostScene& hs, int n, const float* rays7, float* out4);
 int ensure_scratch(r2_ctx* ctx, size_t bytes);
+// compute units of the context's device
+int num_cus(r2_ctx* ctx);
 // device buffer of at least `bytes` in pool slot `slot` (contents undefined)
 hipError_t pool_get(r2_ctx* ctx, int slot, size_t bytes, void** out);
 // getRotation (functions.hpp:128-142), host only

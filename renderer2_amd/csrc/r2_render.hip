@@ -18,7 +18,7 @@ namespace r2host {
 
 static int g_num_cus = 0;
 
-static int num_cus(r2_ctx* ctx) {
+int num_cus(r2_ctx* ctx) {
   if (!g_num_cus) {
     int v = 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) v = 0;

@@ -215,3 +215,30 @@ def test_filter_textured_materials_bit_exact(ctx, with_uvs):
         print(f"textured foliage uvs={with_uvs} {n}^3: {int((d['density'] > 0).sum())} voxels with hits", flush=True)
         assert (d["density"] > 0).sum() > 50
         assert np.array_equal(rec, ref), f"{n}^3: " + _diff_report(rec, ref)
+
+
+# a wave filters up to 16 voxels together (fewer with more rays, 1 with 1000), one
+# voxel per wave below 4096 of them, and stages candidates 32 at a time: the records
+# of a grid large enough for full groups equal those of its voxels in lists of group
+# size 1, 2 and of sizes that leave the last group short, and the oracle's
+@pytest.mark.parametrize("samples,iterations,clip", [(64, 8, True), (16, 8, True), (100, 5, False), (256, 2, True),
+                                                     (1000, 1, True)])
+def test_filter_groups_equal(ctx, samples, iterations, clip):
+    m = _mesh(res=40, quads=4000, size=0.03)
+    gm = ctx.upload_mesh(m)
+    vs = scenes.finest_voxel_size(m, 140 if samples <= 100 else 90)
+    p = r2.filter_params(vs, samples, iterations, clip_rays=clip, seed=4)
+    rec, g = ctx.filter_lod(gm, p)
+    flat = rec.reshape(-1, 32)
+    assert ctx.filter_stats()["active_voxels"] > (16 * 4096 if samples <= 64 else 4 * 4096)
+    dens = flat[:, :4].copy().view(np.float32)[:, 0]
+    full = np.nonzero(dens != 0)[0].astype(np.uint32)
+    rng = np.random.default_rng(samples)
+    for n in (1, 3, 4095, 2 * 4096 + 5, min(5 * 4096 + 11, full.size)):
+        ids = np.concatenate([rng.choice(full, n - n // 8, replace=False),
+                              rng.integers(0, flat.shape[0], n // 8).astype(np.uint32)])
+        assert np.array_equal(ctx.filter_voxels(gm, p, ids), flat[ids]), n
+    ids = rng.choice(full, 400 if samples <= 100 else 60, replace=False)
+    of = O.MeshFilter(m)
+    ref = of.run(of.setup(vs), samples, iterations, seed=4, clip_rays=clip, ids=ids)
+    assert np.array_equal(flat[ids], ref)
