@@ -21,6 +21,73 @@ int hip_fail(r2_ctx* ctx, hipError_t e, const char* what) {
   if (ctx) ctx->err = std::string(what) + ": " + hipGetErrorString(e);
   return e == hipErrorOutOfMemory ? R2_ERR_OOM : R2_ERR_HIP;
 }
+hipError_t DevCache::get(size_t bytes, void** out, size_t* got) {
+  *out = nullptr;
+  bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    size_t best = free_.size();
+    for (size_t i = 0; i < free_.size(); ++i) {
+      const size_t n = free_[i].second;
+      if (n >= bytes && n <= bytes + bytes / 8 + 4096 && (best == free_.size() || n < free_[best].second)) best = i;
+    }
+    if (best < free_.size()) {
+      *out = free_[best].first;
+      *got = free_[best].second;
+      held_ -= *got;
+      free_.erase(free_.begin() + best);
+      return hipSuccess;
+    }
+  }
+  hipError_t e = hipMalloc(out, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    trim();
+    e = hipMalloc(out, bytes);
+  }
+  *got = bytes;
+  return e;
+}
+void DevCache::put(void* p, size_t bytes) {
+  if (!p) return;
+  std::vector<void*> gone;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (bytes > kCap) {
+      gone.push_back(p);
+    } else {
+      free_.push_back({p, bytes});
+      held_ += bytes;
+      while (held_ > kCap) {
+        gone.push_back(free_.front().first);
+        held_ -= free_.front().second;
+        free_.erase(free_.begin());
+      }
+    }
+  }
+  for (void* q : gone) (void)hipFree(q);
+}
+void DevCache::trim() {
+  std::vector<std::pair<void*, size_t>> all;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    all.swap(free_);
+    held_ = 0;
+  }
+  for (auto& b : all) (void)hipFree(b.first);
+}
+
+// hipMalloc that gives the context's cached blocks back before it fails
+static hipError_t malloc_trimmed(r2_ctx* ctx, void** out, size_t bytes) {
+  hipError_t e = hipMalloc(out, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->cache.trim();
+    e = hipMalloc(out, bytes);
+  }
+  return e;
+}
+
 int ensure_scratch(r2_ctx* ctx, size_t bytes) {
   if (ctx->scratch_bytes >= bytes) return R2_OK;
   if (ctx->scratch) {
@@ -29,7 +96,7 @@ int ensure_scratch(r2_ctx* ctx, size_t bytes) {
     ctx->scratch = nullptr;
     ctx->scratch_bytes = 0;
   }
-  R2_HIP(ctx, hipMalloc(&ctx->scratch, bytes));
+  R2_HIP(ctx, malloc_trimmed(ctx, &ctx->scratch, bytes));
   ctx->scratch_bytes = bytes;
   return R2_OK;
 }
@@ -48,7 +115,7 @@ hipError_t pool_get(r2_ctx* ctx, int slot, size_t bytes, void** out) {
     }
     // grow by 1/8 to absorb small size changes between calls
     const size_t want = bytes + bytes / 8;
-    const hipError_t e = hipMalloc(&ctx->pool[slot], want);
+    const hipError_t e = malloc_trimmed(ctx, &ctx->pool[slot], want);
     if (e != hipSuccess) return e;
     ctx->pool_bytes[slot] = want;
   }
@@ -360,6 +427,7 @@ int r2_destroy(r2_ctx* c) {
   if (c->side) (void)hipStreamSynchronize(c->side);
   if (c->scratch) (void)hipFree(c->scratch);
   if (c->d_scene) (void)hipFree(c->d_scene);
+  c->cache.trim();
   for (int i = 0; i < r2_ctx::kPoolSlots; ++i)
     if (c->pool[i]) (void)hipFree(c->pool[i]);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -384,6 +452,7 @@ int r2_grid_upload(r2_ctx* ctx, const r2_grid_desc* d, r2_grid** out) {
   (void)hipSetDevice(ctx->device);
   r2_grid* g = new (std::nothrow) r2_grid();
   if (!g) return R2_ERR_OOM;
+  g->device = ctx->device;
   const int rc = grid_build(ctx, d, g);
   if (rc) {
     r2_grid_free(ctx, g);
@@ -396,8 +465,15 @@ int r2_grid_upload(r2_ctx* ctx, const r2_grid_desc* d, r2_grid** out) {
 int r2_grid_free(r2_ctx* ctx, r2_grid* g) {
   if (!g) return R2_OK;
   if (ctx) (void)hipStreamSynchronize(ctx->stream);
-  for (void* p : g->allocs)
-    if (p) (void)hipFree(p);
+  // the blocks go to the context's cache once the whole device is done with them, as
+  // hipFree waits for it (another stream, a server's or another context's, may have
+  // rendered the grid); a grid of another device goes back to the driver
+  const bool keep = ctx && ctx->device == g->device && hipSetDevice(ctx->device) == hipSuccess &&
+                    hipDeviceSynchronize() == hipSuccess;
+  for (auto& b : g->allocs) {
+    if (keep) ctx->cache.put(b.first, b.second);
+    else (void)hipFree(b.first);
+  }
   delete g;
   return R2_OK;
 }
@@ -586,17 +662,13 @@ static int render_common(r2_ctx* ctx, const r2_render_params* p, float* out, int
   if (rc) return rc;
   const size_t bytes = (size_t)p->width * p->height * 3 * sizeof(float);
   float* d_out = out;
-  void* tmp = nullptr;
-  if (!out_on_device) {
-    R2_HIP(ctx, hipMalloc(&tmp, bytes));
-    d_out = (float*)tmp;
-  }
+  TmpBlocks tmp(ctx->cache, ctx->stream);
+  if (!out_on_device) R2_HIP(ctx, tmp.get(&d_out, bytes));
   rc = launch_render_ex(ctx, s, d_out, (p->flags & R2_FLAG_FP64_ACCUM) != 0, o);
   if ((rc == R2_OK || rc == R2_ERR_CANCELLED) && !out_on_device) {
     hipError_t e = hipMemcpy(out, d_out, bytes, hipMemcpyDeviceToHost);
     if (e != hipSuccess) rc = hip_fail(ctx, e, "hipMemcpy(framebuffer)");
   }
-  if (tmp) (void)hipFree(tmp);
   ctx->stats.last_total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return rc;
 }

@@ -6,6 +6,7 @@
 // Restates: COpenvdbBackend::setValues (raytracer/src/filtering/openvdb_backend.cpp:108-132),
 // CNVDBMedium::init / getMaxValue (raytracer/src/medium/nvdb_medium.cu:130-173,308-323),
 // CHostBrickGrid::CHostBrickGrid (raytracer/src/grid_brick/host_grid_brick.cpp:61-152).
+#include <hipcub/hipcub.hpp>
 #include "r2_internal.hpp"
 #include "r2_volume.hpp"
 #include <algorithm>
@@ -26,12 +27,17 @@ __device__ __forceinline__ uint32_t float_key(float f) {
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-// wave, then block reduction of a thread's extrema and active box, published
-// with one set of atomics per block (same-address atomics from every wavefront
-// serialise in L2): max_bits[0] = max active density (float bits), max_bits[1] =
-// order key of the minimum, bbox = active index box
-__device__ __forceinline__ void publish_extrema(float lmax, float lmin, int lo[3], int hi[3], int* __restrict__ bbox,
-                                                uint32_t* __restrict__ max_bits) {
+// Extrema and active box of a set of voxels: max_key = max active density (float
+// bits, at least 0), min_key = order key of the minimum, lo / hi = active index box.
+struct Extrema {
+  int lo[3], hi[3];
+  uint32_t max_key, min_key;
+};
+// wave, then block reduction of a thread's extrema and active box, written as the
+// block's entry of a list that k_counts reduces (2048 blocks' atomics on the same
+// eight words took 150 of the 230 us of k_active at 256^3)
+__device__ __forceinline__ void publish_extrema(float lmax, float lmin, int lo[3], int hi[3],
+                                                Extrema* __restrict__ out) {
   for (int off = 32; off > 0; off >>= 1) {
     lmax = fmaxf(lmax, __shfl_xor(lmax, off));
     lmin = fminf(lmin, __shfl_xor(lmin, off));
@@ -56,47 +62,96 @@ __device__ __forceinline__ void publish_extrema(float lmax, float lmin, int lo[3
       lmin = fminf(lmin, s_min[w]);
       for (int a = 0; a < 3; ++a) lo[a] = min(lo[a], s_lo[w][a]), hi[a] = max(hi[a], s_hi[w][a]);
     }
-    atomicMax(max_bits, __float_as_uint(fmaxf(lmax, 0.f)));
-    atomicMin(max_bits + 1, float_key(lmin));
-    for (int a = 0; a < 3; ++a) {
-      atomicMin(&bbox[a], lo[a]);
-      atomicMax(&bbox[3 + a], hi[a]);
-    }
+    Extrema e;
+    for (int a = 0; a < 3; ++a) e.lo[a] = lo[a], e.hi[a] = hi[a];
+    e.max_key = __float_as_uint(fmaxf(lmax, 0.f));
+    e.min_key = float_key(lmin);
+    out[blockIdx.x] = e;
   }
 }
 
-// dense records: the active rule (density > 0, or a corner of the index box),
-// leaf occupancy, and the extrema and active box over all voxels (inactive ones
-// reading 0 for the minimum, the brick grid's minorant)
-__global__ void k_active(const uint4* __restrict__ rec, int nx, int ny, int nz, uint8_t* __restrict__ active,
-                         uint32_t* __restrict__ leaf_flag, int nlx, int nly, int* __restrict__ bbox,
-                         uint32_t* __restrict__ max_bits) {
-  const size_t n = (size_t)nx * ny * nz;
-  const bool small = n <= 0xFFFFFFFFull;  // 32-bit index arithmetic (the common case)
+// dense records: the active rule (density > 0, or a corner of the index box), and the
+// extrema and active box over all voxels (inactive ones reading 0 for the minimum,
+// the brick grid's minorant).  One wavefront per 8^3 leaf: flag[leaf] says whether
+// the leaf holds an active voxel, dens[leaf * 512 + v] the density as the brick grid
+// sees it (0 for inactive voxels and beyond the box), so that the brick passes read
+// 4 bytes per voxel instead of records 32 bytes apart.  Bound by the read of the
+// records (256^3: 512 MB).
+__global__ __launch_bounds__(256) void k_active(const uint4* __restrict__ rec, int nx, int ny, int nz, int nlx, int nly,
+                                                int nlz, uint32_t* __restrict__ flag, float* __restrict__ dens,
+                                                Extrema* __restrict__ ext) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t nleaf = (uint32_t)nlx * (uint32_t)nly * (uint32_t)nlz;
+  const uint32_t wave0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+  const uint32_t nwave = (gridDim.x * blockDim.x) >> 6;
   float lmax = 0.f, lmin = FLT_MAX;
   int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    int x, y, z;
-    if (small) {
-      const uint32_t i32 = (uint32_t)i, r = i32 / (uint32_t)nx;
-      x = (int)(i32 - r * (uint32_t)nx);
-      y = (int)(r % (uint32_t)ny);
-      z = (int)(r / (uint32_t)ny);
-    } else {
-      x = (int)(i % nx), y = (int)((i / nx) % ny), z = (int)(i / ((size_t)nx * ny));
+  for (uint32_t li = wave0; li < nleaf; li += nwave) {
+    const int lx = (int)(li % (uint32_t)nlx), ly = (int)(li / (uint32_t)nlx % (uint32_t)nly),
+              lz = (int)(li / ((uint32_t)nlx * (uint32_t)nly));
+    const int x = lx * 8 + (lane & 7), y = ly * 8 + (lane >> 3);
+    float d[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int z = lz * 8 + k;
+      const bool in = x < nx && y < ny && z < nz;
+      const size_t i = ((size_t)(in ? z : 0) * ny + (in ? y : 0)) * nx + (in ? x : 0);
+      d[k] = __uint_as_float(rec[2 * i].x);
     }
-    const float d = __uint_as_float(rec[2 * i].x);
-    const bool a = (d > 0.f) || is_corner(x, y, z, nx, ny, nz);
-    active[i] = a ? 1 : 0;
-    lmin = fminf(lmin, a ? d : 0.f);
-    if (a) {
-      leaf_flag[((size_t)(z >> 3) * nly + (y >> 3)) * nlx + (x >> 3)] = 1u;
-      lmax = fmaxf(lmax, d);
-      lo[0] = min(lo[0], x); lo[1] = min(lo[1], y); lo[2] = min(lo[2], z);
-      hi[0] = max(hi[0], x); hi[1] = max(hi[1], y); hi[2] = max(hi[2], z);
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int z = lz * 8 + k;
+      const bool in = x < nx && y < ny && z < nz;
+      const bool a = in && (d[k] > 0.f || is_corner(x, y, z, nx, ny, nz));
+      const float v = a ? d[k] : 0.f;
+      dens[(size_t)li * kLeafVoxels + k * 64 + lane] = v;
+      if (in) lmin = fminf(lmin, v);
+      if (a) {
+        any = true;
+        lmax = fmaxf(lmax, v);
+        lo[0] = min(lo[0], x); lo[1] = min(lo[1], y); lo[2] = min(lo[2], z);
+        hi[0] = max(hi[0], x); hi[1] = max(hi[1], y); hi[2] = max(hi[2], z);
+      }
+    }
+    const bool used = __ballot(any) != 0ull;
+    if (lane == 0) flag[li] = used ? 1u : 0u;
+  }
+  publish_extrema(lmax, lmin, lo, hi, ext);
+}
+
+// what the host needs to go on: extrema and active box (of the blocks' list), leaves
+// and non-empty bricks (the last entry of each exclusive scan plus the last flag)
+struct BuildCounts {
+  Extrema ext;
+  uint32_t n_leaves, n_bricks;
+};
+__global__ __launch_bounds__(256) void k_counts(BuildCounts* __restrict__ c, const Extrema* __restrict__ ext, int n_ext,
+                                                const uint32_t* __restrict__ flag,
+                                                const uint32_t* __restrict__ leaf_slot, size_t n_leaf,
+                                                const uint32_t* __restrict__ nonempty,
+                                                const uint32_t* __restrict__ brick_slot, size_t n_brick) {
+  __shared__ Extrema s_e[256];
+  Extrema e{{INT32_MAX, INT32_MAX, INT32_MAX}, {INT32_MIN, INT32_MIN, INT32_MIN}, 0u, 0xFFFFFFFFu};
+  auto merge = [&](const Extrema& o) {
+    for (int a = 0; a < 3; ++a) e.lo[a] = min(e.lo[a], o.lo[a]), e.hi[a] = max(e.hi[a], o.hi[a]);
+    e.max_key = max(e.max_key, o.max_key);
+    e.min_key = min(e.min_key, o.min_key);
+  };
+  for (int i = threadIdx.x; i < n_ext; i += 256) merge(ext[i]);
+  s_e[threadIdx.x] = e;
+  for (int h = 128; h > 0; h >>= 1) {
+    __syncthreads();
+    if ((int)threadIdx.x < h) {
+      merge(s_e[threadIdx.x + h]);
+      s_e[threadIdx.x] = e;
     }
   }
-  publish_extrema(lmax, lmin, lo, hi, bbox, max_bits);
+  if (threadIdx.x == 0) {
+    c->ext = e;
+    c->n_leaves = leaf_slot ? leaf_slot[n_leaf - 1] + flag[n_leaf - 1] : 0u;
+    c->n_bricks = brick_slot[n_brick - 1] + nonempty[n_brick - 1];
+  }
 }
 
 // sparse records: leaf k of the caller's list becomes pool slot k; a voxel is
@@ -105,7 +160,7 @@ __global__ void k_active(const uint4* __restrict__ rec, int nx, int ny, int nz, 
 // active box over the voxels of the leaves
 __global__ void k_sparse_leaves(const uint4* __restrict__ rec, const uint8_t* __restrict__ masks,
                                 const int32_t* __restrict__ origins, int64_t n_leaves, int nx, int ny, int nz,
-                                uint4* __restrict__ leaves, int* __restrict__ bbox, uint32_t* __restrict__ max_bits) {
+                                uint4* __restrict__ leaves, Extrema* __restrict__ ext) {
   float lmax = 0.f, lmin = FLT_MAX;
   int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
   for (int64_t li = blockIdx.x; li < n_leaves; li += gridDim.x) {
@@ -131,30 +186,42 @@ __global__ void k_sparse_leaves(const uint4* __restrict__ rec, const uint8_t* __
       leaves[2 * i + 1] = b;
     }
   }
-  publish_extrema(lmax, lmin, lo, hi, bbox, max_bits);
+  publish_extrema(lmax, lmin, lo, hi, ext);
 }
 
-// scatter records into the leaf pool; inactive voxels of an allocated leaf hold the background record
-__global__ void k_leaves(const uint4* __restrict__ rec, const uint8_t* __restrict__ active, int nx, int ny, int nz,
-                         const int32_t* __restrict__ leaf_table, int nlx, int nly, int nlz, uint4* __restrict__ leaves) {
+// copy records into the leaf pool, and the leaf table: slot of each occupied leaf, -1
+// elsewhere; inactive voxels of an allocated leaf hold the background record
+__global__ __launch_bounds__(256) void k_leaves(const uint4* __restrict__ rec, int nx, int ny, int nz,
+                                                const uint32_t* __restrict__ flag, const uint32_t* __restrict__ leaf_slot,
+                                                int nlx, int nly, int nlz, int32_t* __restrict__ leaf_table,
+                                                uint4* __restrict__ leaves) {
   const size_t nleaf_total = (size_t)nlx * nly * nlz;
   for (size_t li = blockIdx.x; li < nleaf_total; li += gridDim.x) {
-    const int32_t slot = leaf_table[li];
-    if (slot < 0) continue;
+    const bool used = flag[li] != 0u;
+    const uint32_t slot = leaf_slot[li];
+    if (threadIdx.x == 0) leaf_table[li] = used ? (int32_t)slot : -1;
+    if (!used) continue;
     const int lx = (int)(li % nlx), ly = (int)((li / nlx) % nly), lz = (int)(li / ((size_t)nlx * nly));
-    for (int v = threadIdx.x; v < kLeafVoxels; v += blockDim.x) {
+    // two lanes per record: consecutive 16-byte words of a row of eight records
+    uint4 w[4];
+    const int h = threadIdx.x & 1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int v = (int)(threadIdx.x >> 1) + 128 * k;
       const int x = lx * 8 + (v & 7), y = ly * 8 + ((v >> 3) & 7), z = lz * 8 + (v >> 6);
-      uint4 a = make_uint4(0u, 0u, 0u, 0u), b = make_uint4(0u, 0u, 0u, 0x3C00u);
-      if (x < nx && y < ny && z < nz) {
-        const size_t i = ((size_t)z * ny + y) * nx + x;
-        if (active[i]) {
-          a = rec[2 * i];
-          b = rec[2 * i + 1];
-        }
-      }
-      uint4* dst = leaves + ((size_t)slot * kLeafVoxels + v) * 2;
-      dst[0] = a;
-      dst[1] = b;
+      const bool in = x < nx && y < ny && z < nz;
+      const size_t i = ((size_t)(in ? z : 0) * ny + (in ? y : 0)) * nx + (in ? x : 0);
+      w[k] = rec[2 * i + h];
+    }
+    uint4* dst = leaves + (size_t)slot * kLeafVoxels * 2;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int v = (int)(threadIdx.x >> 1) + 128 * k;
+      const int x = lx * 8 + (v & 7), y = ly * 8 + ((v >> 3) & 7), z = lz * 8 + (v >> 6);
+      // the record's density is in the first word, which the pair's even lane holds
+      const float d = __uint_as_float((uint32_t)__shfl((int)w[k].x, (int)(threadIdx.x & 62u)));
+      const bool act = x < nx && y < ny && z < nz && (d > 0.f || is_corner(x, y, z, nx, ny, nz));
+      dst[2 * v + h] = act ? w[k] : make_uint4(0u, 0u, 0u, h ? 0x3C00u : 0u);
     }
   }
 }
@@ -229,16 +296,56 @@ struct PoolDens {
   const int32_t* table;
   const uint4* leaves;
   int nx, ny, nz, nlx, nly;
+  __device__ __forceinline__ bool leaf(size_t i) const { return table[i] >= 0; }
   __device__ __forceinline__ float operator()(int x, int y, int z) const {
     if ((unsigned)x >= (unsigned)nx || (unsigned)y >= (unsigned)ny || (unsigned)z >= (unsigned)nz) return 0.f;
     const int32_t leaf = table[((size_t)(z >> 3) * nly + (y >> 3)) * nlx + (x >> 3)];
     if (leaf < 0) return 0.f;
     return __uint_as_float(leaves[((size_t)leaf * kLeafVoxels + (((z & 7) << 6) | ((y & 7) << 3) | (x & 7))) * 2].x);
   }
+  // the densities of voxels 8 bx .. 8 bx + 7 of row (y, z), and the one before and after
+  __device__ __forceinline__ void row(int bx, int y, int z, float v[8]) const {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = (*this)(bx * 8 + k, y, z);
+  }
+  __device__ __forceinline__ void ends(int bx, int y, int z, float v[2]) const {
+    v[0] = (*this)(bx * 8 - 1, y, z);
+    v[1] = (*this)(bx * 8 + 8, y, z);
+  }
+};
+
+// the same from k_active's densities by leaf (dense records)
+struct LeafDens {
+  const float* dens;
+  const uint32_t* flag;
+  int nx, ny, nz, nlx, nly;
+  __device__ __forceinline__ bool leaf(size_t i) const { return flag[i] != 0u; }
+  __device__ __forceinline__ void row(int bx, int y, int z, float v[8]) const {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = 0.f;
+    if (bx * 8 >= nx || (unsigned)y >= (unsigned)ny || (unsigned)z >= (unsigned)nz) return;
+    const float4* p = reinterpret_cast<const float4*>(at(bx, y, z));
+    const float4 a = p[0], b = p[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+  __device__ __forceinline__ void ends(int bx, int y, int z, float v[2]) const {
+    v[0] = v[1] = 0.f;
+    if ((unsigned)y >= (unsigned)ny || (unsigned)z >= (unsigned)nz) return;
+    if (bx > 0 && bx * 8 - 1 < nx) v[0] = at(bx - 1, y, z)[7];
+    if (bx * 8 + 8 < nx) v[1] = at(bx + 1, y, z)[0];
+  }
+
+ private:
+  // the row of leaf column bx that holds (y, z): 32-byte aligned
+  __device__ __forceinline__ const float* at(int bx, int y, int z) const {
+    return dens + (((size_t)(z >> 3) * nly + (y >> 3)) * nlx + bx) * kLeafVoxels + (((z & 7) << 6) | ((y & 7) << 3));
+  }
 };
 
 // one wavefront per brick: min/max over the dilated 10^3 neighbourhood
-__global__ void k_brick_range(PoolDens dens, int nbx, int nby, int nbz, uint32_t* __restrict__ range,
+template <typename Dens>
+__global__ void k_brick_range(Dens dens, int nbx, int nby, int nbz, uint32_t* __restrict__ range,
                               uint32_t* __restrict__ nonempty) {
   const size_t wave = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
@@ -252,7 +359,7 @@ __global__ void k_brick_range(PoolDens dens, int nbx, int nby, int nbz, uint32_t
     const int lx = bx + lane % 3 - 1, ly = by + (lane / 3) % 3 - 1, lz = bz + lane / 9 - 1;
     const int nlx = (dens.nx + 7) >> 3, nly = (dens.ny + 7) >> 3, nlz = (dens.nz + 7) >> 3;
     if ((unsigned)lx < (unsigned)nlx && (unsigned)ly < (unsigned)nly && (unsigned)lz < (unsigned)nlz)
-      leaf = dens.table[((size_t)lz * nly + ly) * nlx + lx] >= 0;
+      leaf = dens.leaf(((size_t)lz * nly + ly) * nlx + lx);
   }
   if (__ballot(leaf) == 0ull) {
     if (lane == 0) {
@@ -262,11 +369,18 @@ __global__ void k_brick_range(PoolDens dens, int nbx, int nby, int nbz, uint32_t
     return;
   }
   float lo = FLT_MAX, hi = -FLT_MAX;
-  for (int k = lane; k < 1000; k += 64) {
-    const int x = k % 10 - 1, y = (k / 10) % 10 - 1, z = k / 100 - 1;
-    const float d = dens(bx * 8 + x, by * 8 + y, bz * 8 + z);
-    lo = fminf(lo, d);
-    hi = fmaxf(hi, d);
+  for (int k = lane; k < 100; k += 64) {  // a lane takes rows of ten voxels
+    const int y = by * 8 + k % 10 - 1, z = bz * 8 + k / 10 - 1;
+    float v[8], e[2];
+    dens.row(bx, y, z, v);
+    dens.ends(bx, y, z, e);
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      lo = fminf(lo, v[x]);
+      hi = fmaxf(hi, v[x]);
+    }
+    lo = fminf(lo, fminf(e[0], e[1]));
+    hi = fmaxf(hi, fmaxf(e[0], e[1]));
   }
   for (int off = 32; off > 0; off >>= 1) {
     lo = fminf(lo, __shfl_xor(lo, off));
@@ -278,8 +392,10 @@ __global__ void k_brick_range(PoolDens dens, int nbx, int nby, int nbz, uint32_t
   }
 }
 
-// one wavefront per brick: quantise the 512 voxels of every non-empty brick
-__global__ void k_brick_atlas(PoolDens dens, int nbx, int nby, int nbz, const uint32_t* __restrict__ range, const uint32_t* __restrict__ slot,
+// one wavefront per brick: quantise the 512 voxels of every non-empty brick, a row of
+// eight per lane and store
+template <typename Dens>
+__global__ void k_brick_atlas(Dens dens, int nbx, int nby, int nbz, const uint32_t* __restrict__ range, const uint32_t* __restrict__ slot,
                               const uint32_t* __restrict__ nonempty, uint2* __restrict__ bricks,
                               uint8_t* __restrict__ atlas, float* __restrict__ maj0) {
   const size_t wave = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -296,10 +412,12 @@ __global__ void k_brick_atlas(PoolDens dens, int nbx, int nby, int nbz, const ui
   if (!ne) return;
   const float lo = range_lo(r), hi = range_hi(r);
   uint8_t* dst = atlas + (size_t)slot[wave] * 512;
-  for (int v = lane; v < 512; v += 64) {
-    const int x = v & 7, y = (v >> 3) & 7, z = v >> 6;
-    dst[v] = encode_voxel(dens(bx * 8 + x, by * 8 + y, bz * 8 + z), lo, hi);
-  }
+  float d[8];
+  dens.row(bx, by * 8 + (lane & 7), bz * 8 + (lane >> 3), d);
+  uint32_t w[2] = {0u, 0u};
+#pragma unroll
+  for (int x = 0; x < 8; ++x) w[x >> 2] |= (uint32_t)encode_voxel(d[x], lo, hi) << (8 * (x & 3));
+  *reinterpret_cast<uint2*>(dst + lane * 8) = make_uint2(w[0], w[1]);
 }
 
 // min/max mip level from the level below (range encoded), plus its decoded max
@@ -342,89 +460,53 @@ __global__ void k_lookup(DGrid g, int n, const int32_t* __restrict__ xyz, uint4*
 template <typename T>
 int dmalloc(r2_ctx* ctx, r2_grid* g, T** p, size_t n) {
   void* q = nullptr;
-  hipError_t e = hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T));
+  size_t got = 0;
+  hipError_t e = ctx->cache.get(std::max<size_t>(n, 1) * sizeof(T), &q, &got);
   if (e != hipSuccess) return r2host::hip_fail(ctx, e, "hipMalloc(grid)");
-  g->allocs.push_back(q);
+  g->allocs.push_back({q, got});
   *p = (T*)q;
   return R2_OK;
 }
+// parts of one device block, each 256-byte aligned
+struct Carve {
+  size_t size = 0;
+  size_t add(size_t bytes) {
+    const size_t at = size;
+    size += (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+    return at;
+  }
+};
 
 }  // namespace
 
 namespace r2host {
 
+// The layout passes run on the stream without the host until the leaf and brick
+// counts are known (one wait), then the leaf pool and the atlas are allocated and
+// filled.  256^3 dense records in device memory, blocks at hand: 0.46 ms, 0.31 of it
+// k_active and k_leaves (4.4 and 6.0 TB/s); with two tables through the host, an
+// allocation per array and the brick passes on the 32-byte records it took 0.94, and
+// the freeing of the temporaries and of the grid 0.26.
 int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   using namespace r2;
   const int nx = desc->nx, ny = desc->ny, nz = desc->nz;
   const bool sparse = desc->n_leaves > 0;
   hipStream_t st = ctx->stream;
   int rc;
-  struct Tmp {
-    std::vector<void*> p;
-    ~Tmp() { for (void* q : p) (void)hipFree(q); }
-  } tmp;
-  auto tmalloc = [&](void** q, size_t bytes) -> hipError_t {
-    hipError_t e = hipMalloc(q, std::max<size_t>(bytes, 1));
-    if (e == hipSuccess) tmp.p.push_back(*q);
-    return e;
-  };
+  TmpBlocks tmp(ctx->cache, st);
   const int nlx = (nx + 7) / 8, nly = (ny + 7) / 8, nlz = (nz + 7) / 8;
   const size_t nleaf_total = (size_t)nlx * nly * nlz;
   // records staged in device memory: nx*ny*nz dense records, or n_leaves leaves of 512
   const size_t nrec = sparse ? (size_t)desc->n_leaves * kLeafVoxels : (size_t)nx * ny * nz;
-  const uint4* d_rec = nullptr;
-  if (desc->records_on_device) {
-    d_rec = (const uint4*)desc->records;
-  } else {
-    void* staged = nullptr;
-    R2_HIP(ctx, tmalloc(&staged, nrec * 32));
-    R2_HIP(ctx, hipMemcpyAsync(staged, desc->records, nrec * 32, hipMemcpyHostToDevice, st));
-    d_rec = (const uint4*)staged;
-  }
-  int* d_bbox = nullptr;
-  uint32_t* d_max = nullptr;
-  R2_HIP(ctx, tmalloc((void**)&d_bbox, 6 * 4));
-  R2_HIP(ctx, tmalloc((void**)&d_max, 8));
-  const int bbox_init[6] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN, INT32_MIN};
-  R2_HIP(ctx, hipMemcpyAsync(d_bbox, bbox_init, sizeof(bbox_init), hipMemcpyHostToDevice, st));
-  const uint32_t mm_init[2] = {0u, 0xFFFFFFFFu};
-  R2_HIP(ctx, hipMemcpyAsync(d_max, mm_init, 8, hipMemcpyHostToDevice, st));
-
-  std::vector<int32_t> table(nleaf_total, -1);
-  int64_t nleaves = 0;
-  const uint8_t* d_dense_active = nullptr;  // dense path: the active flags for the leaf scatter
-  uint4* d_leaves = nullptr;
-  bool covers_all = true;  // every voxel of the index box lies in a leaf (else some voxel reads 0)
-  int bbox[6];
-  uint32_t mm[2] = {0u, 0u};
-  if (!sparse) {
-    // dense: the active rule per voxel, leaves allocated in table order
-    const size_t nv = nrec;
-    uint8_t* d_active = nullptr;
-    uint32_t* d_leaf_flag = nullptr;
-    R2_HIP(ctx, tmalloc((void**)&d_active, nv));
-    R2_HIP(ctx, tmalloc((void**)&d_leaf_flag, nleaf_total * 4));
-    R2_HIP(ctx, hipMemsetAsync(d_leaf_flag, 0, nleaf_total * 4, st));
-    // grid-stride over the voxels: 8 blocks per CU are enough to stream the records
-    const int blocks = (int)std::min<size_t>((nv + 255) / 256, 2048);
-    hipLaunchKernelGGL(k_active, dim3(blocks), dim3(256), 0, st, d_rec, nx, ny, nz, d_active, d_leaf_flag, nlx, nly,
-                       d_bbox, d_max);
-    R2_HIP(ctx, hipGetLastError());
-    std::vector<uint32_t> flags(nleaf_total);
-    R2_HIP(ctx, hipMemcpyAsync(flags.data(), d_leaf_flag, nleaf_total * 4, hipMemcpyDeviceToHost, st));
-    R2_HIP(ctx, hipMemcpyAsync(bbox, d_bbox, sizeof(bbox), hipMemcpyDeviceToHost, st));
-    R2_HIP(ctx, hipMemcpyAsync(mm, d_max, 8, hipMemcpyDeviceToHost, st));
-    R2_HIP(ctx, hipStreamSynchronize(st));
-    for (size_t i = 0; i < nleaf_total; ++i) table[i] = flags[i] ? (int32_t)(nleaves++) : -1;
-    if (nleaves == 0) return fail(ctx, R2_ERR_INVALID, "grid has no active voxel");
-    if ((rc = dmalloc(ctx, g, &d_leaves, (size_t)nleaves * kLeafVoxels * 2))) return rc;
-    d_dense_active = d_active;
-  } else {
-    // sparse: the caller's leaves in their order
-    nleaves = desc->n_leaves;
+  // the caller's sparse leaves: their table and whether they cover the index box (else
+  // some voxel reads 0)
+  std::vector<int32_t> table;
+  bool covers_all = true;
+  if (sparse) {
     if (!desc->leaf_origins) return fail(ctx, R2_ERR_INVALID, "grid: sparse records without leaf origins");
+    table.assign(nleaf_total, -1);
     uint64_t covered = 0;
-    for (int64_t k = 0; k < nleaves; ++k) {
+    for (int64_t k = 0; k < desc->n_leaves; ++k) {
       const int32_t* o = desc->leaf_origins + 3 * k;
       if ((o[0] | o[1] | o[2]) & 7 || o[0] < 0 || o[1] < 0 || o[2] < 0 || o[0] >= nx || o[1] >= ny || o[2] >= nz)
         return fail(ctx, R2_ERR_INVALID, "grid: leaf origin " + std::to_string(k) +
@@ -435,26 +517,115 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
       covered += (uint64_t)std::min(8, nx - o[0]) * std::min(8, ny - o[1]) * std::min(8, nz - o[2]);
     }
     covers_all = covered == (uint64_t)nx * ny * nz;
-    int32_t* d_orig = nullptr;
-    uint8_t* d_mask = nullptr;
-    R2_HIP(ctx, tmalloc((void**)&d_orig, (size_t)nleaves * 12));
-    R2_HIP(ctx, hipMemcpyAsync(d_orig, desc->leaf_origins, (size_t)nleaves * 12, hipMemcpyHostToDevice, st));
-    if (desc->leaf_masks) {
-      R2_HIP(ctx, tmalloc((void**)&d_mask, (size_t)nleaves * 64));
-      R2_HIP(ctx, hipMemcpyAsync(d_mask, desc->leaf_masks, (size_t)nleaves * 64, hipMemcpyHostToDevice, st));
-    }
-    if ((rc = dmalloc(ctx, g, &d_leaves, (size_t)nleaves * kLeafVoxels * 2))) return rc;
-    hipLaunchKernelGGL(k_sparse_leaves, dim3((unsigned)std::min<int64_t>(nleaves, 65536)), dim3(256), 0, st, d_rec,
-                       d_mask, d_orig, nleaves, nx, ny, nz, d_leaves, d_bbox, d_max);
-    R2_HIP(ctx, hipGetLastError());
-    R2_HIP(ctx, hipMemcpyAsync(bbox, d_bbox, sizeof(bbox), hipMemcpyDeviceToHost, st));
-    R2_HIP(ctx, hipMemcpyAsync(mm, d_max, 8, hipMemcpyDeviceToHost, st));
-    R2_HIP(ctx, hipStreamSynchronize(st));
-    if (bbox[0] > bbox[3]) return fail(ctx, R2_ERR_INVALID, "grid has no active voxel");
   }
-  // read the copied extrema only after the stream has finished the copies
-  const uint32_t maxbits = mm[0];
-  uint32_t minbits = (mm[1] & 0x80000000u) ? (mm[1] & 0x7FFFFFFFu) : ~mm[1];
+  int nb[3];
+  const int n3[3] = {nx, ny, nz};
+  for (int a = 0; a < 3; ++a) {
+    const int b = (int)ceilf((float)n3[a] / 8.f);
+    nb[a] = (int)ceilf((float)b / 8.f) * 8;
+    if (nb[a] >= 1024) return fail(ctx, R2_ERR_UNSUPPORTED, "exceeded max brick count of 1024 per axis");
+  }
+  const size_t nbt = (size_t)nb[0] * nb[1] * nb[2];
+
+  const uint4* d_rec = nullptr;
+  if (desc->records_on_device) {
+    d_rec = (const uint4*)desc->records;
+  } else {
+    void* staged = nullptr;
+    R2_HIP(ctx, tmp.get(&staged, nrec * 32));
+    R2_HIP(ctx, hipMemcpyAsync(staged, desc->records, nrec * 32, hipMemcpyHostToDevice, st));
+    d_rec = (const uint4*)staged;
+  }
+  // arrays of known size that the grid keeps: leaf table, brick entries, level-0
+  // ranges, the four majorant levels in one buffer (level l, nbt / 8^l texels, nbt a
+  // multiple of 512, starts at (nbt / 64) x {0, 64, 72, 73}[l], so that a lookup finds
+  // its level's table by arithmetic) and the three mips
+  Carve kc;
+  const size_t o_table = kc.add(nleaf_total * 4), o_bricks = kc.add(nbt * 8), o_range = kc.add(nbt * 4),
+               o_maj = kc.add((nbt + nbt / 8 + nbt / 64 + nbt / 512) * 4), o_mip0 = kc.add(nbt / 8 * 4),
+               o_mip1 = kc.add(nbt / 64 * 4), o_mip2 = kc.add(nbt / 512 * 4);
+  char* kept = nullptr;
+  if ((rc = dmalloc(ctx, g, &kept, kc.size))) return rc;
+  int32_t* d_table = (int32_t*)(kept + o_table);
+  uint2* d_bricks = (uint2*)(kept + o_bricks);
+  uint32_t* d_range = (uint32_t*)(kept + o_range);
+  float* d_maj[4] = {(float*)(kept + o_maj), nullptr, nullptr, nullptr};
+  d_maj[1] = d_maj[0] + nbt;
+  d_maj[2] = d_maj[1] + nbt / 8;
+  d_maj[3] = d_maj[2] + nbt / 64;
+  uint32_t* d_mip[3] = {(uint32_t*)(kept + o_mip0), (uint32_t*)(kept + o_mip1), (uint32_t*)(kept + o_mip2)};
+  // and of the build alone
+  size_t scan_bytes = 0, sb = 0;
+  R2_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr, (int)nbt, st));
+  if (!sparse) {
+    R2_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, sb, (uint32_t*)nullptr, (uint32_t*)nullptr, (int)nleaf_total, st));
+    scan_bytes = std::max(scan_bytes, sb);
+  }
+  // blocks of the pass over the records: a wavefront takes about four leaves of a 256^3
+  // grid, 8 blocks per CU stream the records
+  const unsigned rec_blocks = (unsigned)std::min<size_t>(sparse ? (size_t)desc->n_leaves : (nleaf_total + 3) / 4,
+                                                         (size_t)num_cus(ctx) * 8);
+  Carve tc;
+  const size_t o_ext = tc.add(rec_blocks * sizeof(Extrema));
+  const size_t o_counts = tc.add(sizeof(BuildCounts)), o_nonempty = tc.add(nbt * 4), o_slot = tc.add(nbt * 4),
+               o_scan = tc.add(scan_bytes), o_flag = tc.add(sparse ? 0 : nleaf_total * 4),
+               o_lslot = tc.add(sparse ? 0 : nleaf_total * 4),
+               o_dens = tc.add(sparse ? 0 : nleaf_total * kLeafVoxels * 4),
+               o_orig = tc.add(sparse ? (size_t)desc->n_leaves * 12 : 0),
+               o_mask = tc.add(sparse && desc->leaf_masks ? (size_t)desc->n_leaves * 64 : 0);
+  char* work = nullptr;
+  R2_HIP(ctx, tmp.get(&work, tc.size));
+  BuildCounts* d_counts = (BuildCounts*)(work + o_counts);
+  uint32_t *d_nonempty = (uint32_t*)(work + o_nonempty), *d_slot = (uint32_t*)(work + o_slot);
+  uint32_t *d_flag = (uint32_t*)(work + o_flag), *d_lslot = (uint32_t*)(work + o_lslot);
+  float* d_dens = (float*)(work + o_dens);
+  void* d_scan = work + o_scan;
+  Extrema* d_ext = (Extrema*)(work + o_ext);
+  BuildCounts counts{};
+
+  uint4* d_leaves = nullptr;
+  const dim3 brick_blocks((unsigned)((nbt * 64 + 255) / 256));
+  const LeafDens ldens{d_dens, d_flag, nx, ny, nz, nlx, nly};
+  if (!sparse) {
+    hipLaunchKernelGGL(k_active, dim3(rec_blocks), dim3(256), 0, st, d_rec, nx, ny, nz, nlx, nly, nlz, d_flag, d_dens,
+                       d_ext);
+    R2_HIP(ctx, hipGetLastError());
+    sb = scan_bytes;
+    R2_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(d_scan, sb, d_flag, d_lslot, (int)nleaf_total, st));
+    hipLaunchKernelGGL(k_brick_range<LeafDens>, brick_blocks, dim3(256), 0, st, ldens, nb[0], nb[1], nb[2], d_range,
+                       d_nonempty);
+    R2_HIP(ctx, hipGetLastError());
+  } else {
+    // the caller's leaves in their order
+    int32_t* d_orig = (int32_t*)(work + o_orig);
+    uint8_t* d_mask = nullptr;
+    R2_HIP(ctx, hipMemcpyAsync(d_table, table.data(), nleaf_total * 4, hipMemcpyHostToDevice, st));
+    R2_HIP(ctx, hipMemcpyAsync(d_orig, desc->leaf_origins, (size_t)desc->n_leaves * 12, hipMemcpyHostToDevice, st));
+    if (desc->leaf_masks) {
+      d_mask = (uint8_t*)(work + o_mask);
+      R2_HIP(ctx, hipMemcpyAsync(d_mask, desc->leaf_masks, (size_t)desc->n_leaves * 64, hipMemcpyHostToDevice, st));
+    }
+    if ((rc = dmalloc(ctx, g, &d_leaves, (size_t)desc->n_leaves * kLeafVoxels * 2))) return rc;
+    hipLaunchKernelGGL(k_sparse_leaves, dim3(rec_blocks), dim3(256), 0, st, d_rec, d_mask, d_orig, desc->n_leaves, nx, ny,
+                       nz, d_leaves, d_ext);
+    R2_HIP(ctx, hipGetLastError());
+    hipLaunchKernelGGL(k_brick_range<PoolDens>, brick_blocks, dim3(256), 0, st,
+                       PoolDens{d_table, d_leaves, nx, ny, nz, nlx, nly}, nb[0], nb[1], nb[2], d_range, d_nonempty);
+    R2_HIP(ctx, hipGetLastError());
+  }
+  sb = scan_bytes;
+  R2_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(d_scan, sb, d_nonempty, d_slot, (int)nbt, st));
+  hipLaunchKernelGGL(k_counts, dim3(1), dim3(256), 0, st, d_counts, d_ext, (int)rec_blocks, d_flag,
+                     sparse ? nullptr : d_lslot, nleaf_total, d_nonempty, d_slot, nbt);
+  R2_HIP(ctx, hipGetLastError());
+  R2_HIP(ctx, hipMemcpyAsync(&counts, d_counts, sizeof(counts), hipMemcpyDeviceToHost, st));
+  R2_HIP(ctx, hipStreamSynchronize(st));
+  const int64_t nleaves = sparse ? desc->n_leaves : (int64_t)counts.n_leaves;
+  const uint32_t nne = counts.n_bricks;
+  const Extrema& ext = counts.ext;
+  if (nleaves == 0 || ext.lo[0] > ext.hi[0]) return fail(ctx, R2_ERR_INVALID, "grid has no active voxel");
+  const uint32_t maxbits = ext.max_key;
+  uint32_t minbits = (ext.min_key & 0x80000000u) ? (ext.min_key & 0x7FFFFFFFu) : ~ext.min_key;
   if (!covers_all) {
     float mn;
     memcpy(&mn, &minbits, 4);
@@ -465,14 +636,21 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   d.nx = nx; d.ny = ny; d.nz = nz;
   d.nlx = nlx; d.nly = nly; d.nlz = nlz;
   d.precision = desc->precision;
-  int32_t* d_table = nullptr;
-  if ((rc = dmalloc(ctx, g, &d_table, nleaf_total))) return rc;
-  R2_HIP(ctx, hipMemcpyAsync(d_table, table.data(), nleaf_total * 4, hipMemcpyHostToDevice, st));
+  uint8_t* d_atlas = nullptr;
+  if ((rc = dmalloc(ctx, g, &d_atlas, (size_t)std::max<uint32_t>(nne, 1) * 512))) return rc;
   if (!sparse) {
-    hipLaunchKernelGGL(k_leaves, dim3((unsigned)std::min<size_t>(nleaf_total, 65536)), dim3(256), 0, st, d_rec,
-                       d_dense_active, nx, ny, nz, d_table, nlx, nly, nlz, d_leaves);
+    if ((rc = dmalloc(ctx, g, &d_leaves, (size_t)nleaves * kLeafVoxels * 2))) return rc;
+    hipLaunchKernelGGL(k_leaves, dim3((unsigned)std::min<size_t>(nleaf_total, 65536)), dim3(256), 0, st, d_rec, nx, ny,
+                       nz, d_flag, d_lslot, nlx, nly, nlz, d_table, d_leaves);
     R2_HIP(ctx, hipGetLastError());
+    hipLaunchKernelGGL(k_brick_atlas<LeafDens>, brick_blocks, dim3(256), 0, st, ldens, nb[0], nb[1], nb[2], d_range,
+                       d_slot, d_nonempty, d_bricks, d_atlas, d_maj[0]);
+  } else {
+    hipLaunchKernelGGL(k_brick_atlas<PoolDens>, brick_blocks, dim3(256), 0, st,
+                       PoolDens{d_table, d_leaves, nx, ny, nz, nlx, nly}, nb[0], nb[1], nb[2], d_range, d_slot,
+                       d_nonempty, d_bricks, d_atlas, d_maj[0]);
   }
+  R2_HIP(ctx, hipGetLastError());
   d.leaf_table = d_table;
   d.leaves = d_leaves;
   d.leaves_packed = nullptr;
@@ -489,66 +667,15 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
     d.leaves_packed = d_hot;
     d.leaves_cold = d_cold;
   }
-  const PoolDens pool{d_table, d_leaves, nx, ny, nz, nlx, nly};
-
-  // brick grid
-  int nb[3];
-  const int n3[3] = {nx, ny, nz};
-  for (int a = 0; a < 3; ++a) {
-    const int b = (int)ceilf((float)n3[a] / 8.f);
-    nb[a] = (int)ceilf((float)b / 8.f) * 8;
-    if (nb[a] >= 1024) return fail(ctx, R2_ERR_UNSUPPORTED, "exceeded max brick count of 1024 per axis");
-  }
-  const size_t nbt = (size_t)nb[0] * nb[1] * nb[2];
-  uint32_t *d_range = nullptr, *d_nonempty = nullptr, *d_slot = nullptr;
-  R2_HIP(ctx, tmalloc((void**)&d_range, nbt * 4));
-  R2_HIP(ctx, tmalloc((void**)&d_nonempty, nbt * 4));
-  R2_HIP(ctx, tmalloc((void**)&d_slot, nbt * 4));
-  {
-    const size_t threads = nbt * 64;
-    hipLaunchKernelGGL(k_brick_range, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, pool, nb[0], nb[1],
-                       nb[2], d_range, d_nonempty);
-    R2_HIP(ctx, hipGetLastError());
-  }
-  std::vector<uint32_t> ne(nbt), slot(nbt);
-  R2_HIP(ctx, hipMemcpyAsync(ne.data(), d_nonempty, nbt * 4, hipMemcpyDeviceToHost, st));
-  R2_HIP(ctx, hipStreamSynchronize(st));
-  uint32_t nne = 0;
-  for (size_t i = 0; i < nbt; ++i) slot[i] = ne[i] ? nne++ : 0u;
-  R2_HIP(ctx, hipMemcpyAsync(d_slot, slot.data(), nbt * 4, hipMemcpyHostToDevice, st));
-  uint2* d_bricks = nullptr;
-  uint8_t* d_atlas = nullptr;
-  float* d_maj[4] = {nullptr, nullptr, nullptr, nullptr};
-  uint32_t* d_mip[3] = {nullptr, nullptr, nullptr};
-  if ((rc = dmalloc(ctx, g, &d_bricks, nbt))) return rc;
-  if ((rc = dmalloc(ctx, g, &d_atlas, (size_t)std::max<uint32_t>(nne, 1) * 512))) return rc;
-  // the four majorant levels in one buffer: level l (nbt / 8^l texels, nbt a
-  // multiple of 512) starts at (nbt / 64) x {0, 64, 72, 73}[l], so that a lookup
-  // finds its level's table by arithmetic
-  if ((rc = dmalloc(ctx, g, &d_maj[0], nbt + nbt / 8 + nbt / 64 + nbt / 512))) return rc;
-  d_maj[1] = d_maj[0] + nbt;
-  d_maj[2] = d_maj[1] + nbt / 8;
-  d_maj[3] = d_maj[2] + nbt / 64;
-  {
-    const size_t threads = nbt * 64;
-    hipLaunchKernelGGL(k_brick_atlas, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, pool, nb[0], nb[1],
-                       nb[2], d_range, d_slot, d_nonempty, d_bricks, d_atlas, d_maj[0]);
-    R2_HIP(ctx, hipGetLastError());
-  }
   for (int l = 0; l < 3; ++l) {
     const int sx = nb[0] >> (l + 1), sy = nb[1] >> (l + 1), sz = nb[2] >> (l + 1);
     const int px = nb[0] >> l, py = nb[1] >> l;
     const size_t cnt = (size_t)sx * sy * sz;
-    if ((rc = dmalloc(ctx, g, &d_mip[l], cnt))) return rc;
     const uint32_t* src = l == 0 ? d_range : d_mip[l - 1];
     hipLaunchKernelGGL(k_brick_mip, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st, src, px, py, d_mip[l], sx, sy,
                        sz, d_maj[l + 1]);
     R2_HIP(ctx, hipGetLastError());
   }
-  // keep the level-0 ranges for the parity probe (d_range is temporary)
-  uint32_t* d_range_keep = nullptr;
-  if ((rc = dmalloc(ctx, g, &d_range_keep, nbt))) return rc;
-  R2_HIP(ctx, hipMemcpyAsync(d_range_keep, d_range, nbt * 4, hipMemcpyDeviceToDevice, st));
   d.bricks = d_bricks;
   d.atlas = d_atlas;
   for (int l = 0; l < 4; ++l) d.maj[l] = d_maj[l];
@@ -558,8 +685,8 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   // transforms (CNVDBMedium::init, nvdb_medium.cu:152-170)
   r2_grid_info& info = g->info;
   for (int a = 0; a < 3; ++a) {
-    info.ibb_min[a] = bbox[a];
-    info.size[a] = bbox[3 + a] - bbox[a] + 1;
+    info.ibb_min[a] = ext.lo[a];
+    info.size[a] = ext.hi[a] - ext.lo[a] + 1;
     info.n_bricks[a] = nb[a];
     d.ibb_min[a] = info.ibb_min[a];
     d.size[a] = info.size[a];
@@ -631,42 +758,37 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   }
   g->voxel_size_filtering = desc->voxel_size_filtering;
   // level-0 ranges and mip buffers stay reachable for r2_grid_download_bricks
-  g->range0 = d_range_keep;
+  g->range0 = d_range;
   for (int l = 0; l < 3; ++l) g->mip[l] = d_mip[l];
   return R2_OK;
 }
 
 int grid_lookup(r2_ctx* ctx, const r2_grid* g, int n, const int32_t* coords, uint8_t* out) {
-  void *dc = nullptr, *dout = nullptr;
-  struct F {
-    void** q[2];
-    ~F() { for (auto x : q) if (*x) (void)hipFree(*x); }
-  } f{{&dc, &dout}};
-  R2_HIP(ctx, hipMalloc(&dc, (size_t)n * 12));
-  R2_HIP(ctx, hipMalloc(&dout, (size_t)n * 32));
-  R2_HIP(ctx, hipMemcpy(dc, coords, (size_t)n * 12, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_lookup, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, g->dev, n, (const int32_t*)dc,
-                     (uint4*)dout);
+  hipStream_t st = ctx->stream;
+  TmpBlocks tmp(ctx->cache, st);
+  int32_t* dc = nullptr;
+  uint4* dout = nullptr;
+  R2_HIP(ctx, tmp.get(&dc, (size_t)n * 12));
+  R2_HIP(ctx, tmp.get(&dout, (size_t)n * 32));
+  R2_HIP(ctx, hipMemcpyAsync(dc, coords, (size_t)n * 12, hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_lookup, dim3((n + 255) / 256), dim3(256), 0, st, g->dev, n, dc, dout);
   R2_HIP(ctx, hipGetLastError());
-  R2_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  R2_HIP(ctx, hipMemcpy(out, dout, (size_t)n * 32, hipMemcpyDeviceToHost));
+  R2_HIP(ctx, hipMemcpyAsync(out, dout, (size_t)n * 32, hipMemcpyDeviceToHost, st));
+  R2_HIP(ctx, hipStreamSynchronize(st));
   return R2_OK;
 }
 
 int grid_sample(r2_ctx* ctx, const r2_grid* g, int n, const float* pos, float* out) {
-  void *dp = nullptr, *dout = nullptr;
-  struct F {
-    void** q[2];
-    ~F() { for (auto x : q) if (*x) (void)hipFree(*x); }
-  } f{{&dp, &dout}};
-  R2_HIP(ctx, hipMalloc(&dp, (size_t)n * 12));
-  R2_HIP(ctx, hipMalloc(&dout, (size_t)n * 17 * 4));
-  R2_HIP(ctx, hipMemcpy(dp, pos, (size_t)n * 12, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_sample, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, g->dev, n, (const float*)dp,
-                     (float*)dout);
+  hipStream_t st = ctx->stream;
+  TmpBlocks tmp(ctx->cache, st);
+  float *dp = nullptr, *dout = nullptr;
+  R2_HIP(ctx, tmp.get(&dp, (size_t)n * 12));
+  R2_HIP(ctx, tmp.get(&dout, (size_t)n * 17 * 4));
+  R2_HIP(ctx, hipMemcpyAsync(dp, pos, (size_t)n * 12, hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_sample, dim3((n + 255) / 256), dim3(256), 0, st, g->dev, n, dp, dout);
   R2_HIP(ctx, hipGetLastError());
-  R2_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  R2_HIP(ctx, hipMemcpy(out, dout, (size_t)n * 17 * 4, hipMemcpyDeviceToHost));
+  R2_HIP(ctx, hipMemcpyAsync(out, dout, (size_t)n * 17 * 4, hipMemcpyDeviceToHost, st));
+  R2_HIP(ctx, hipStreamSynchronize(st));
   return R2_OK;
 }
 

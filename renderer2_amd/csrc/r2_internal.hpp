@@ -1,13 +1,63 @@
 // Internal host-side declarations shared by the translation units of the library.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 #include "../../include/r2.h"
 #include "r2_types.hpp"
 
+namespace r2host {
+// Device blocks that a context's finished calls and freed grids leave for the next
+// ones.  A program that loads one volume after another otherwise pays for fresh
+// memory each time: once as much memory as the device has had been allocated and
+// freed, every new 512 MB block cost 14 ms (the driver clears it), ten times the work
+// of laying out a 256^3 volume.  A block is put here only when nothing on the device
+// uses it any more.  At most kCap bytes are kept (the oldest go first), all are given
+// back when an allocation fails and when the context is destroyed.  A request takes
+// the smallest block that fits with at most an eighth to spare.
+class DevCache {
+ public:
+  static constexpr size_t kCap = size_t(8) << 30;
+  hipError_t get(size_t bytes, void** out, size_t* got);
+  void put(void* p, size_t bytes);
+  void trim();
+
+ private:
+  std::mutex mu_;
+  std::vector<std::pair<void*, size_t>> free_;  // oldest first
+  size_t held_ = 0;
+};
+// device blocks of one call, put back when it ends (after a wait for the stream)
+struct TmpBlocks {
+  DevCache& cache;
+  hipStream_t stream;
+  std::vector<std::pair<void*, size_t>> p;
+  TmpBlocks(DevCache& c, hipStream_t s) : cache(c), stream(s) {}
+  ~TmpBlocks() {
+    if (p.empty()) return;
+    const bool idle = hipStreamSynchronize(stream) == hipSuccess;
+    for (auto& b : p) {
+      if (idle) cache.put(b.first, b.second);
+      else (void)hipFree(b.first);
+    }
+  }
+  template <typename T>
+  hipError_t get(T** out, size_t bytes) {
+    void* q = nullptr;
+    size_t n = 0;
+    const hipError_t e = cache.get(bytes, &q, &n);
+    if (e == hipSuccess) p.push_back({q, n});
+    *out = (T*)q;
+    return e;
+  }
+};
+}  // namespace r2host
+
 struct r2_ctx {
   int device = 0;
+  r2host::DevCache cache;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // second stream for work that overlaps the main one (the filter's record fill),
@@ -36,7 +86,8 @@ struct r2_ctx {
 struct r2_grid {
   r2::DGrid dev{};            // device view (pointers into `allocs`)
   r2_grid_info info{};
-  std::vector<void*> allocs;  // owned device allocations
+  std::vector<std::pair<void*, size_t>> allocs;  // owned device blocks
+  int device = 0;
   uint32_t* range0 = nullptr;  // level-0 brick ranges (also in allocs)
   uint32_t* mip[3] = {nullptr, nullptr, nullptr};
   float voxel_size_filtering = 0.f;

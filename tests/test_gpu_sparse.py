@@ -134,3 +134,47 @@ def test_sparse_large_extent(ctx):
     print(f"2048^3 sparse extent: relMSE against the dense 56^3 grid {e:.2e}, "
           f"{np.mean(np.all(fa == fb, axis=2)):.4f} of pixels identical")
     assert e < 2e-3
+
+
+# grids made and freed one after another share the context's device blocks, which hold
+# the last grid's bytes: each of a run of sizes (sides that are no multiple of the leaf,
+# a single voxel, one leaf row, half of the volume empty) equals the same grid in a
+# context of its own, and its lookups the records
+@pytest.mark.parametrize("form", ["dense", "sparse", "packed"])
+def test_reused_blocks_give_fresh_grids(ctx, form):
+    import renderer2_amd as r2
+
+    rng = np.random.default_rng(5)
+    for shape in ((40, 33, 57), (41, 32, 56), (1, 1, 1), (8, 8, 200), (130, 70, 9), (40, 33, 57)):
+        nz, ny, nx = shape
+        rec = np.zeros((*shape, 32), np.uint8)
+        rec[..., 4:28] = rng.integers(0, 256, (*shape, 24))
+        rec[..., 28:30] = np.frombuffer(np.float16(1.4).tobytes(), np.uint8)
+        dens = rng.random(shape, dtype=np.float32) * 3
+        dens[:, :, nx // 2:] = 0
+        rec[..., :4] = dens[..., None].view(np.uint8)
+        g = dict(records=rec, shape=shape, map_mat=(0.1, 0, 0, 0, 0.1, 0, 0, 0, 0.1), map_vec=(0, 0, 0),
+                 sigma_a=(0.1,) * 3, sigma_s=(0.9,) * 3, voxel_size_filtering=0.1)
+        if form == "sparse":
+            g.update(_leaves(rec))
+        if form == "packed":
+            g["precision"] = "packed"
+        fresh = r2.Context(0)
+        a, b = ctx.upload_grid(g), fresh.upload_grid(g)
+        assert all(np.array_equal(v, b.info()[k]) for k, v in a.info().items())
+        (ra, ua, ma), (rb, ub, mb) = a.download_bricks(), b.download_bricks()
+        assert np.array_equal(ra, rb) and np.array_equal(ua, ub)
+        assert all(np.array_equal(x, y) for x, y in zip(ma, mb))
+        la = _all_lookups(a, shape)
+        assert np.array_equal(la, _all_lookups(b, shape))
+        pos = rng.random((200, 3), dtype=np.float32)
+        assert np.array_equal(a.sample(pos).view(np.uint32), b.sample(pos).view(np.uint32))
+        want = np.zeros((nz + 2, ny + 2, nx + 2, 32), np.uint8)
+        want[..., 29] = 0x3C
+        act = dens > 0
+        act[np.ix_((0, nz - 1), (0, ny - 1), (0, nx - 1))] = True
+        want[1:-1, 1:-1, 1:-1][act] = rec[act]
+        assert np.array_equal(la, want.reshape(-1, 32))
+        a.free()
+        b.free()
+        fresh.close()
