@@ -17,7 +17,7 @@ namespace {
 using namespace r2;
 
 __device__ __forceinline__ bool is_corner(int x, int y, int z, int nx, int ny, int nz) {
-  return (x == 0 || x == nx - 1) && (y == 0 || y == ny - 1) && (z == 0 || z == nz - 1);
+  return ((x == 0) | (x == nx - 1)) & ((y == 0) | (y == ny - 1)) & ((z == 0) | (z == nz - 1));
 }
 
 // effective density (active rule) + leaf occupancy + bbox + max density
@@ -220,8 +220,11 @@ __global__ __launch_bounds__(256) void k_leaves(const uint4* __restrict__ rec, i
       const int x = lx * 8 + (v & 7), y = ly * 8 + ((v >> 3) & 7), z = lz * 8 + (v >> 6);
       // the record's density is in the first word, which the pair's even lane holds
       const float d = __uint_as_float((uint32_t)__shfl((int)w[k].x, (int)(threadIdx.x & 62u)));
-      const bool act = x < nx && y < ny && z < nz && (d > 0.f || is_corner(x, y, z, nx, ny, nz));
-      dst[2 * v + h] = act ? w[k] : make_uint4(0u, 0u, 0u, h ? 0x3C00u : 0u);
+      // by masks: hipcc compiled the choice between two uint4 under this condition wrongly
+      // (three of the four words of a corner voxel of density 0 became background)
+      const bool act = (x < nx) & (y < ny) & (z < nz) & ((d > 0.f) | is_corner(x, y, z, nx, ny, nz));
+      const uint32_t m = act ? 0xFFFFFFFFu : 0u, ior = h ? 0x3C00u : 0u;
+      dst[2 * v + h] = make_uint4(w[k].x & m, w[k].y & m, w[k].z & m, (w[k].w & m) | (ior & ~m));
     }
   }
 }
