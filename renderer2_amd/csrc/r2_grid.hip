@@ -804,7 +804,7 @@ __global__ void k_scene_intersect(const r2::DScene* __restrict__ sp, const float
   const r2::DScene& s = r2::kconst(sp);
   const float* q = rays + 7 * (size_t)i;
   r2::Ray r = r2::mkray(r2::mk(q[0], q[1], q[2]), r2::mk(q[3], q[4], q[5]), q[6], -1);
-  const r2::Hit h = r2::scene_intersect<true, false>(s, r);
+  const r2::Hit h = r2::scene_intersect<true, r2::kAnyInst>(s, r);
   float* o = out + 4 * (size_t)i;
   o[0] = (float)h.hit;
   o[1] = h.t;

@@ -116,9 +116,9 @@ struct BatchEntry {
 #define R2K_DECLARE(NS)                                                                                              \
   namespace NS {                                                                                                     \
   void launch_sm(hipStream_t st, int blocks, int lanes, const r2::DScene* d_scene, uint64_t* counter, uint64_t total, \
-                 int chunk, void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp, const int32_t* ps, \
+                 int chunk, void* partial, bool fp64, int inst, bool surf, bool count, const int32_t* pp, const int32_t* ps, \
                  float* po, uint32_t* pc);                                                                           \
-  void launch_batch_group(hipStream_t st, int blocks, const void* ents, int n, uint64_t* counters, bool single,      \
+  void launch_batch_group(hipStream_t st, int blocks, const void* ents, int n, uint64_t* counters, int inst,         \
                           bool surf, bool fp64);                                                                     \
   void launch_reduce_k(hipStream_t st, const void* partial, bool fp64, int nchunks, uint32_t n3, float* out);        \
   }
@@ -187,9 +187,14 @@ struct BatchSlice {
   void* d_partial;
   uint64_t first, count;
   int chunk;
-  bool single, surf, fp64, packed;
+  int inst;  // r2::kOneInst, kFewInst or kAnyInst
+  bool surf, fp64, packed;
 };
 constexpr int kMaxBatchEntries = 256;
+// the kernels' form for a scene
+inline int inst_form(const r2::DScene& s) {
+  return s.n_inst == 1 ? r2::kOneInst : (s.n_bvh == 0 ? r2::kFewInst : r2::kAnyInst);
+}
 void render_chunking(const r2::DScene& scene, int* chunk, int* nchunks);
 int launch_reduce(hipStream_t st, const void* partial, bool fp64, int nchunks, uint32_t n3, float* out);
 // d_ents: kMaxBatchEntries entries of device scratch, d_counters: as many u64

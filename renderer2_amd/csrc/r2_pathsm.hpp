@@ -196,9 +196,9 @@ __device__ __forceinline__ void dead_walk(PathLane& p) {
 
 // --------------------------------------------------------------- traversal --
 // Prologue of sampleDDA / sampleInternal / trDDA / trInternal on instance k.
-template <bool kSingle>
+template <int kInst>
 __device__ __forceinline__ void start_traversal(const DScene& s, PathLane& p, int k, const Ray& rw, int kind) {
-  const int ki = kSingle ? 0 : k;
+  const int ki = kInst == kOneInst ? 0 : k;
   const DInstance& in = inst_at(s, ki);
   const DGrid& g = s.grid[in.grid];
   const Ray rm = ray_transform2(rw, in.w2m);
@@ -227,9 +227,9 @@ __device__ __forceinline__ void start_traversal(const DScene& s, PathLane& p, in
 
 // One step of the traversal loop body.  Returns true when the traversal ended;
 // p.tres = 1 for a real collision of a free flight.
-template <bool kSingle, bool kCount>
+template <int kInst, bool kCount>
 __device__ __forceinline__ bool traversal_step(const DScene& s, PathLane& p, Cnt& cnt) {
-  const int ki = kSingle ? 0 : p.tinst;
+  const int ki = kInst == kOneInst ? 0 : p.tinst;
   const DInstance& in = inst_at(s, ki);
   const DGrid& g = s.grid[in.grid];
   const float ratio = in.ratio;
@@ -301,9 +301,9 @@ __device__ __forceinline__ bool traversal_step(const DScene& s, PathLane& p, Cnt
 
 // Collision tail of sampleDDA / sampleInternal + CMediumInstance::sample's
 // transform back to world space: returns the albedo, fills the scatter record.
-template <bool kSingle, bool kCount>
+template <int kInst, bool kCount>
 __device__ __forceinline__ v3 flight_collision(const DScene& s, const PathLane& p, Scatter& sc, Cnt& cnt) {
-  const int ki = kSingle ? 0 : p.tinst;
+  const int ki = kInst == kOneInst ? 0 : p.tinst;
   const DInstance& in = inst_at(s, ki);
   const DGrid& g = s.grid[in.grid];
   Rec fd;
@@ -332,19 +332,19 @@ __device__ __forceinline__ v3 flight_collision(const DScene& s, const PathLane& 
   return alb;
 }
 
-template <bool kSingle>
+template <int kInst>
 __device__ __forceinline__ Ray lane_move_to_voxel_border(const DScene& s, int k, const Ray& r) {
-  return inst_move_to_voxel_border(s, kSingle ? 0 : k, r);
+  return inst_move_to_voxel_border(s, kInst == kOneInst ? 0 : k, r);
 }
 
 // a ray spawned at a scatter point along dir, its origin offset along `off` (the
 // voxel normal for shadow rays, the unnormalised sample for the continuation),
 // moved to the voxel border (the tails of direct() and of Li's bounce)
-template <bool kSingle>
+template <int kInst>
 __device__ __forceinline__ Ray spawn_at_scatter(const DScene& s, const Scatter& sc, v3 dir, v3 off) {
   Ray r = mkray(sc.pos, dir, kDefaultTmax, sc.inst);
   ray_offset(r, off);
-  return lane_move_to_voxel_border<kSingle>(s, sc.inst, r);
+  return lane_move_to_voxel_border<kInst>(s, sc.inst, r);
 }
 
 // -------------------------------------------------------------------- walk --
@@ -410,7 +410,7 @@ __device__ __forceinline__ void cont_nohit(PathLane& p) {
 // then the transmittance traversal of the segment if it lies inside a medium.
 // Both roles share one scene intersection and one traversal set-up, so a pass
 // whose lanes hold both kinds of ray runs each once.
-template <bool kSingle, bool kSurf>
+template <int kInst, bool kSurf>
 __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
   dead_traversal(p);  // read by the step that ended the last traversal
   const bool dda = (s.flags & 1u) != 0u;
@@ -427,7 +427,7 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
   }
   const int cur = p.ray.medium;
   Ray r = cont ? p.ray : spawn_ray(p.ray.o, p.ray.d, cur);
-  const Hit h = scene_intersect<kSurf, kSingle>(s, r);  // shortens r.tmax to the hit, as the reference's intersect does
+  const Hit h = scene_intersect<kSurf, kInst>(s, r);  // shortens r.tmax to the hit, as the reference's intersect does
   Ray tr = r;  // the ray of the traversal to start
   // a second intersection that both roles may need is made once for all lanes
   Ray r2;
@@ -479,7 +479,7 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
     }
   }
   if (again) {
-    const Hit se = scene_intersect<kSurf, kSingle>(s, r2);
+    const Hit se = scene_intersect<kSurf, kInst>(s, r2);
     if (cont) {
       if (!se.hit) {
         cont_nohit(p);
@@ -495,15 +495,15 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
     }
   }
   const int kind = cont ? (dda ? TK_FLIGHT_DDA : TK_FLIGHT_DELTA) : (dda ? TK_TR_DDA : TK_TR_RATIO);
-  start_traversal<kSingle>(s, p, tr.medium, tr, kind);
+  start_traversal<kInst>(s, p, tr.medium, tr, kind);
 }
 
 // A lane inside a traversal (ST_TRAV): one DDA / tracking step; at the end
 // of the traversal the continuation has collided (next vertex) or leaves the
 // medium box, and a shadow ray's segment ends at a box face.
-template <bool kSingle, bool kCount>
+template <int kInst, bool kCount>
 __device__ __forceinline__ void trav_step(const DScene& s, PathLane& p, Cnt& cnt) {
-  if (!traversal_step<kSingle, kCount>(s, p, cnt)) return;
+  if (!traversal_step<kInst, kCount>(s, p, cnt)) return;
   if (p.role == RL_CONT) {
     if (p.tres) cont_done(p, CR_COLLIDED);
     else cont_nohit(p);
@@ -523,7 +523,7 @@ __device__ __forceinline__ void trav_step(const DScene& s, PathLane& p, Cnt& cnt
 // The scatter vertex k (k >= 1) of a path at a collision: direct()'s two
 // strategies up to their shadow walks, Li's continuation and Russian roulette,
 // in the reference's order of draws from the vertex's own stream.
-template <bool kSingle, bool kCount>
+template <int kInst, bool kCount>
 __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, const Scatter& sc, Cnt& cnt) {
   ++p.k;
   p.rng.init(p.rng.c0, p.rng.c1, 4u * (uint32_t)p.k);
@@ -538,7 +538,7 @@ __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, cons
   const v3 Le = env_sample<kCount>(s.env, p.rng, ldir, lpdf, cnt);
   if (lpdf > 0.f) {
     const v3 dl = normalize(ldir);
-    const Ray r = spawn_at_scatter<kSingle>(s, sc, dl, sc.n);
+    const Ray r = spawn_at_scatter<kInst>(s, sc, dl, sc.n);
     p.ray.o = r.o;  // walked first: straight to the walk registers (wo is taken)
     p.ray.d = r.o + r.tmax * r.d;
     p.ray.medium = r.medium;
@@ -554,7 +554,7 @@ __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, cons
     const float ph = phase_sample(sc.S, sc.n, sc.ior, wo, wi, p.rng);
     if (ph > 0.f) {
       const v3 dw = normalize(wi);
-      const Ray r = spawn_at_scatter<kSingle>(s, sc, dw, sc.n);
+      const Ray r = spawn_at_scatter<kInst>(s, sc, dw, sc.n);
       p.c.lb0 = r.o;
       p.c.lb1 = r.o + r.tmax * r.d;
       p.c.lb_med = r.medium;
@@ -570,7 +570,7 @@ __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, cons
   {
     v3 wi;
     (void)phase_sample(sc.S, sc.n, sc.ior, wo, wi, p.rng);
-    const Ray r = spawn_at_scatter<kSingle>(s, sc, normalize(wi), wi);
+    const Ray r = spawn_at_scatter<kInst>(s, sc, normalize(wi), wi);
     p.c.c_o = r.o;
     p.c.c_d = r.d;
     p.c.c_tmax = r.tmax;

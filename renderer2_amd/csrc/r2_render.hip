@@ -48,14 +48,14 @@ static LaunchShape launch_shape(r2_ctx* ctx, uint64_t items) {
 }
 
 static void launch_sm(r2_ctx* ctx, int prec, const LaunchShape& sh, uint64_t* counter, uint64_t total,
-                      int chunk, void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp,
+                      int chunk, void* partial, bool fp64, int inst, bool surf, bool count, const int32_t* pp,
                       const int32_t* ps, float* po, uint32_t* pc) {
   if (prec == 1)
     r2k_packed::launch_sm(ctx->stream, sh.blocks, sh.lanes, ctx->d_scene, counter, total, chunk, partial, fp64,
-                          single, surf, count, pp, ps, po, pc);
+                          inst, surf, count, pp, ps, po, pc);
   else
     r2k_fp32::launch_sm(ctx->stream, sh.blocks, sh.lanes, ctx->d_scene, counter, total, chunk, partial, fp64,
-                        single, surf, count, pp, ps, po, pc);
+                        inst, surf, count, pp, ps, po, pc);
 }
 
 size_t batch_entry_bytes() { return sizeof(r2::BatchEntry); }
@@ -80,16 +80,16 @@ int launch_reduce(hipStream_t st, const void* partial, bool fp64, int nchunks, u
 int launch_batch(r2_ctx* ctx, hipStream_t st, const std::vector<BatchSlice>& items, void* d_ents, uint64_t* d_counters) {
   using namespace r2;
   if (items.empty()) return R2_OK;
-  // one launch per (single instance, surfaces, accumulator type, record precision) group
+  // one launch per (instance form, surfaces, accumulator type, record precision) group
   std::vector<BatchEntry> host(items.size());
   int off = 0;
-  for (int g = 0; g < 16; ++g) {
-    const bool single = (g & 1) != 0, fp64 = (g & 2) != 0, packed = (g & 4) != 0, surf = (g & 8) != 0;
-    if (single && surf) continue;  // surface scenes run the general-instance form, whatever their instance count
+  for (int g = 0; g < 24; ++g) {
+    const int inst = g >> 3;
+    const bool fp64 = (g & 1) != 0, packed = (g & 2) != 0, surf = (g & 4) != 0;
     const int first = off;
     uint64_t total = 0;
     for (const BatchSlice& b : items) {
-      if (b.surf != surf || (!surf && b.single != single) || b.fp64 != fp64 || b.packed != packed || b.count == 0)
+      if (b.surf != surf || b.inst != inst || b.fp64 != fp64 || b.packed != packed || b.count == 0)
         continue;
       BatchEntry& e = host[off++];
       e.scene = b.d_scene;
@@ -106,8 +106,8 @@ int launch_batch(r2_ctx* ctx, hipStream_t st, const std::vector<BatchSlice>& ite
     R2_HIP(ctx, hipMemcpyAsync(de, &host[first], sizeof(BatchEntry) * n, hipMemcpyHostToDevice, st));
     R2_HIP(ctx, hipMemsetAsync(d_counters + first, 0, sizeof(uint64_t) * n, st));
     const int blocks = (int)std::min<uint64_t>((uint64_t)num_cus(ctx) * kBlocksPerCu, (total + 255) / 256);
-    if (packed) r2k_packed::launch_batch_group(st, blocks, de, n, d_counters + first, single, surf, fp64);
-    else r2k_fp32::launch_batch_group(st, blocks, de, n, d_counters + first, single, surf, fp64);
+    if (packed) r2k_packed::launch_batch_group(st, blocks, de, n, d_counters + first, inst, surf, fp64);
+    else r2k_fp32::launch_batch_group(st, blocks, de, n, d_counters + first, inst, surf, fp64);
     R2_HIP(ctx, hipGetLastError());
   }
   return R2_OK;
@@ -119,10 +119,10 @@ int launch_batch(r2_ctx* ctx, hipStream_t st, const std::vector<BatchSlice>& ite
 // sample chunk, like the reference's one launch per sample: a launch takes the
 // items [first, total) by starting the shared item counter at `first`.  Each item
 // writes its own chunk sum, so the frame is the same bit for bit either way.
-static int launch_items(r2_ctx* ctx, int prec, bool single, bool surf, bool fp64, uint64_t* counter, uint64_t first,
+static int launch_items(r2_ctx* ctx, int prec, int inst, bool surf, bool fp64, uint64_t* counter, uint64_t first,
                         uint64_t total, int chunk, void* partial) {
   const LaunchShape sh = launch_shape(ctx, total - first);
-  launch_sm(ctx, prec, sh, counter, total, chunk, partial, fp64, single, surf, false, nullptr, nullptr, nullptr,
+  launch_sm(ctx, prec, sh, counter, total, chunk, partial, fp64, inst, surf, false, nullptr, nullptr, nullptr,
             nullptr);
   R2_HIP(ctx, hipGetLastError());
   return R2_OK;
@@ -155,7 +155,8 @@ int launch_render_ex(r2_ctx* ctx, const HostScene& hs, float* d_out, bool fp64, 
   }
   const uint64_t total = (uint64_t)nchunks * npix;
   hipStream_t st = ctx->stream;
-  const bool single = scene.n_inst == 1, surf = scene.n_surf > 0;
+  const int inst = inst_form(scene);
+  const bool surf = scene.n_surf > 0;
   const int prec = hs.precision;
   if (prec < 0) return fail(ctx, R2_ERR_UNSUPPORTED, "render: instances mix FP32 and packed grids");
   {
@@ -167,7 +168,7 @@ int launch_render_ex(r2_ctx* ctx, const HostScene& hs, float* d_out, bool fp64, 
   int done_chunks = nchunks;
   int launches = 1;
   if (!o.progress) {
-    int rc = launch_items(ctx, prec, single, surf, fp64, counter, 0, total, chunk, partial);
+    int rc = launch_items(ctx, prec, inst, surf, fp64, counter, 0, total, chunk, partial);
     if (rc) return rc;
   } else {
     // one launch per sample chunk, with up to two in flight; the callback runs
@@ -187,7 +188,7 @@ int launch_render_ex(r2_ctx* ctx, const HostScene& hs, float* d_out, bool fp64, 
         const uint64_t first = (uint64_t)queued * npix;
         R2_HIP(ctx, hipMemsetD32Async((hipDeviceptr_t)counter,
                                       (int)(uint32_t)first, 1, st));
-        rc = launch_items(ctx, prec, single, surf, fp64, counter, first, first + npix, chunk, partial);
+        rc = launch_items(ctx, prec, inst, surf, fp64, counter, first, first + npix, chunk, partial);
         if (rc) break;
         R2_HIP(ctx, hipEventRecord(evs[queued & 1], st));
         ++queued;
@@ -280,7 +281,7 @@ int launch_paths(r2_ctx* ctx, const HostScene& hs, int n, const int32_t* d_pix, 
     const int rc = upload_scene(ctx, hs, true);
     if (rc) return rc;
   }
-  launch_sm(ctx, prec, launch_shape(ctx, (uint64_t)n), scene_counter(ctx, hs), (uint64_t)n, 1, nullptr, false, scene.n_inst == 1, scene.n_surf > 0, true, d_pix, d_smp,
+  launch_sm(ctx, prec, launch_shape(ctx, (uint64_t)n), scene_counter(ctx, hs), (uint64_t)n, 1, nullptr, false, inst_form(scene), scene.n_surf > 0, true, d_pix, d_smp,
             d_out, d_cnt);
   R2_HIP(ctx, hipGetLastError());
   R2_HIP(ctx, hipStreamSynchronize(st));

@@ -120,14 +120,14 @@ __device__ __forceinline__ void finish_path(const DScene& s, PathLane& p, Cnt& c
 // next scatter vertex, a surface hit the next surface vertex; an escaped camera
 // ray sees the environment; anything else ends the path), and for a path that
 // ends the start of the item's next sample (vertex 0: the camera ray).
-template <bool kSingle, bool kSurf, bool kCount, typename Acc>
+template <int kInst, bool kSurf, bool kCount, typename Acc>
 __device__ __forceinline__ void shade(const DScene& s, PathLane& p, Cnt& cnt, uint32_t npix, int chunk,
                                       Acc* __restrict__ partial, const int32_t* __restrict__ probe_pix,
                                       float* __restrict__ probe_out, uint32_t* __restrict__ probe_cnt) {
   bool scatter = false;
   Scatter sc;
   if (p.cres == CR_COLLIDED) {
-    p.thr = p.thr * flight_collision<kSingle, kCount>(s, p, sc, cnt);
+    p.thr = p.thr * flight_collision<kInst, kCount>(s, p, sc, cnt);
     scatter = !any_zero(p.thr);
   } else if (p.cres == CR_ESCAPED) {
     float lpdf = 0.f;
@@ -140,7 +140,7 @@ __device__ __forceinline__ void shade(const DScene& s, PathLane& p, Cnt& cnt, ui
   dead(p.sh_Tr);
   dead(p.si_hit);
   if (scatter) {
-    shade_scatter<kSingle, kCount>(s, p, sc, cnt);
+    shade_scatter<kInst, kCount>(s, p, sc, cnt);
     return;
   }
   if (kSurf && p.cres == CR_SURFACE) {
@@ -240,7 +240,7 @@ constexpr short kPrioTrav = 2, kPrioSeg = 1;
 #ifndef R2_SEG_RATIO
 #define R2_SEG_RATIO 2
 #endif
-template <bool kSingle, bool kSurf, bool kCount, typename Acc, typename Fetch>
+template <int kInst, bool kSurf, bool kCount, typename Acc, typename Fetch>
 __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cnt, int lane, uint32_t npix,
                                            Acc* __restrict__ partial, const int32_t* __restrict__ probe_pix,
                                            float* __restrict__ probe_out, uint32_t* __restrict__ probe_cnt,
@@ -259,7 +259,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
     SM_STAT(1, 1);
     SM_STAT(2, __popcll(__ballot(p.stage == ST_SHADE)));
     if (p.stage == ST_SHADE)
-      shade<kSingle, kSurf, kCount, Acc>(s, p, cnt, npix, fetch.chunk_len(), partial, probe_pix, probe_out, probe_cnt);
+      shade<kInst, kSurf, kCount, Acc>(s, p, cnt, npix, fetch.chunk_len(), partial, probe_pix, probe_out, probe_cnt);
 #ifdef R2_SM_STATS
     SM_STAT(5, SM_CLOCK() - t0);
 #endif
@@ -270,7 +270,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
     __builtin_amdgcn_s_setprio(kPrioSeg);
     if (p.stage == ST_SEG) {
       p.rng.top_up();
-      seg_step<kSingle, kSurf>(s, p);
+      seg_step<kInst, kSurf>(s, p);
     }
     __builtin_amdgcn_s_setprio(0);
   } else if (ns * 64 >= R2_SEG_MIN * live || ns >= R2_SEG_RATIO * nt) {
@@ -279,7 +279,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
     __builtin_amdgcn_s_setprio(kPrioSeg);
     if (at_seg) {
       p.rng.top_up();
-      seg_step<kSingle, kSurf>(s, p);
+      seg_step<kInst, kSurf>(s, p);
     }
     __builtin_amdgcn_s_setprio(0);
 #ifdef R2_SM_STATS
@@ -291,7 +291,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
     __builtin_amdgcn_s_setprio(kPrioTrav);
     if (at_trav) {
       p.rng.top_up();
-      trav_step<kSingle, kCount>(s, p, cnt);
+      trav_step<kInst, kCount>(s, p, cnt);
     }
     __builtin_amdgcn_s_setprio(0);
 #ifdef R2_SM_STATS
@@ -304,7 +304,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
 #ifndef R2_SM_WAVES
 #define R2_SM_WAVES 4  // wavefronts per SIMD the register budget is sized for
 #endif
-template <bool kSingle, bool kSurf, bool kCount, typename Acc>
+template <int kInst, bool kSurf, bool kCount, typename Acc>
 __global__ void __launch_bounds__(256, R2_SM_WAVES) k_paths_sm(const DScene* __restrict__ sp, uint64_t* __restrict__ counter,
                                                   int lanes, uint64_t total, int chunk, Acc* __restrict__ partial,
                                                   const int32_t* __restrict__ probe_pix,
@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(256, R2_SM_WAVES) k_paths_sm(const DScene* __r
   stats_begin();
   for (uint32_t guard = 0; guard < (1u << 30); ++guard) {
     SM_STAT(0, 1);
-    if (!sched_step<kSingle, kSurf, kCount, Acc>(s, p, cnt, lane, npix, partial, probe_pix, probe_out, probe_cnt, fetch))
+    if (!sched_step<kInst, kSurf, kCount, Acc>(s, p, cnt, lane, npix, partial, probe_pix, probe_out, probe_cnt, fetch))
       break;
   }
   stats_end();
@@ -368,7 +368,7 @@ struct BatchFetch {
   }
 };
 
-template <bool kSingle, bool kSurf, typename Acc>
+template <int kInst, bool kSurf, typename Acc>
 __global__ void __launch_bounds__(256, R2_SM_WAVES) k_paths_batch(const BatchEntry* __restrict__ ents, int n_ent,
                                                                   uint64_t* __restrict__ counters) {
   const int lane = threadIdx.x & 63;
@@ -392,7 +392,7 @@ __global__ void __launch_bounds__(256, R2_SM_WAVES) k_paths_batch(const BatchEnt
     p.cres = CR_START;
     const BatchFetch fetch{&E, &counters[e]};
     for (uint32_t guard = 0; guard < (1u << 30); ++guard) {
-      if (!sched_step<kSingle, kSurf, false, Acc>(s, p, cnt, lane, npix, partial, nullptr, nullptr, nullptr, fetch))
+      if (!sched_step<kInst, kSurf, false, Acc>(s, p, cnt, lane, npix, partial, nullptr, nullptr, nullptr, fetch))
         break;
     }
   }
@@ -423,46 +423,60 @@ __global__ void k_reduce(const Acc* __restrict__ partial, int nchunks, uint32_t 
 
 
 
-// host-side launchers of this instantiation.  Scenes with analytic surfaces run
-// the general-instance form with the surface code; the others the forms without.
+// host-side launchers of this instantiation.  Compensated FP64 sums and the lookup
+// counters of the probe run a few instances in the general form, and surface scenes
+// of those two all in it (kernel_form; the same for a standalone and a batched frame).
+static int kernel_form(int inst, bool surf, bool fp64, bool count) {
+  if (fp64 || count) return surf || inst != kOneInst ? kAnyInst : kOneInst;
+  return inst;
+}
 void launch_sm(hipStream_t st, int blocks, int lanes, const DScene* d_scene, uint64_t* counter, uint64_t total,
-               int chunk, void* partial, bool fp64, bool single, bool surf, bool count, const int32_t* pp,
+               int chunk, void* partial, bool fp64, int inst, bool surf, bool count, const int32_t* pp,
                const int32_t* ps, float* po, uint32_t* pc) {
 #define R2K_LAUNCH(S, F, C, A)                                                                                  \
   hipLaunchKernelGGL((k_paths_sm<S, F, C, A>), dim3(blocks), dim3(256), 0, st, d_scene, counter, lanes, total, \
                      chunk, (A*)partial, pp, ps, po, pc)
-  if (surf) {
-    if (count) R2K_LAUNCH(false, true, true, float);
-    else if (fp64) R2K_LAUNCH(false, true, false, double);
-    else R2K_LAUNCH(false, true, false, float);
-  } else if (count) {
-    if (single) R2K_LAUNCH(true, false, true, float);
-    else R2K_LAUNCH(false, false, true, float);
+  const int f = kernel_form(inst, surf, fp64, count);
+  if (count) {
+    if (surf) R2K_LAUNCH(kAnyInst, true, true, float);
+    else if (f == kOneInst) R2K_LAUNCH(kOneInst, false, true, float);
+    else R2K_LAUNCH(kAnyInst, false, true, float);
   } else if (fp64) {
-    if (single) R2K_LAUNCH(true, false, false, double);
-    else R2K_LAUNCH(false, false, false, double);
+    if (surf) R2K_LAUNCH(kAnyInst, true, false, double);
+    else if (f == kOneInst) R2K_LAUNCH(kOneInst, false, false, double);
+    else R2K_LAUNCH(kAnyInst, false, false, double);
+  } else if (surf) {
+    if (f == kOneInst) R2K_LAUNCH(kOneInst, true, false, float);
+    else if (f == kFewInst) R2K_LAUNCH(kFewInst, true, false, float);
+    else R2K_LAUNCH(kAnyInst, true, false, float);
   } else {
-    if (single) R2K_LAUNCH(true, false, false, float);
-    else R2K_LAUNCH(false, false, false, float);
+    if (f == kOneInst) R2K_LAUNCH(kOneInst, false, false, float);
+    else if (f == kFewInst) R2K_LAUNCH(kFewInst, false, false, float);
+    else R2K_LAUNCH(kAnyInst, false, false, float);
   }
 #undef R2K_LAUNCH
 }
 
-void launch_batch_group(hipStream_t st, int blocks, const void* ents, int n, uint64_t* counters, bool single,
-                        bool surf, bool fp64) {
+void launch_batch_group(hipStream_t st, int blocks, const void* ents, int n, uint64_t* counters, int inst, bool surf,
+                        bool fp64) {
   const BatchEntry* de = (const BatchEntry*)ents;
-  if (surf && fp64)
-    hipLaunchKernelGGL((k_paths_batch<false, true, double>), dim3(blocks), dim3(256), 0, st, de, n, counters);
-  else if (surf)
-    hipLaunchKernelGGL((k_paths_batch<false, true, float>), dim3(blocks), dim3(256), 0, st, de, n, counters);
-  else if (single && fp64)
-    hipLaunchKernelGGL((k_paths_batch<true, false, double>), dim3(blocks), dim3(256), 0, st, de, n, counters);
-  else if (single)
-    hipLaunchKernelGGL((k_paths_batch<true, false, float>), dim3(blocks), dim3(256), 0, st, de, n, counters);
-  else if (fp64)
-    hipLaunchKernelGGL((k_paths_batch<false, false, double>), dim3(blocks), dim3(256), 0, st, de, n, counters);
-  else
-    hipLaunchKernelGGL((k_paths_batch<false, false, float>), dim3(blocks), dim3(256), 0, st, de, n, counters);
+#define R2K_LAUNCH(S, F, A) \
+  hipLaunchKernelGGL((k_paths_batch<S, F, A>), dim3(blocks), dim3(256), 0, st, de, n, counters)
+  const int f = kernel_form(inst, surf, fp64, false);
+  if (fp64) {
+    if (surf) R2K_LAUNCH(kAnyInst, true, double);
+    else if (f == kOneInst) R2K_LAUNCH(kOneInst, false, double);
+    else R2K_LAUNCH(kAnyInst, false, double);
+  } else if (surf) {
+    if (f == kOneInst) R2K_LAUNCH(kOneInst, true, float);
+    else if (f == kFewInst) R2K_LAUNCH(kFewInst, true, float);
+    else R2K_LAUNCH(kAnyInst, true, float);
+  } else {
+    if (f == kOneInst) R2K_LAUNCH(kOneInst, false, float);
+    else if (f == kFewInst) R2K_LAUNCH(kFewInst, false, float);
+    else R2K_LAUNCH(kAnyInst, false, float);
+  }
+#undef R2K_LAUNCH
 }
 
 void launch_reduce_k(hipStream_t st, const void* partial, bool fp64, int nchunks, uint32_t n3, float* out) {

@@ -53,7 +53,8 @@ struct SrvReq {
   const r2::DScene& scene = hs.s;
   std::vector<unsigned char> scene_img;  // host image of the device copy (kept until the request ends)
   int chunk = 1, nchunks = 1;
-  bool fp64 = false, single = true, surf = false, packed = false;
+  int form = r2::kOneInst;  // the instance form of the kernels
+  bool fp64 = false, surf = false, packed = false;
   uint64_t total_items = 0, next_item = 0;  // items in all, items handed to slices
   uint64_t done_items = 0;                   // items of completed slices
   int inflight = 0;                          // slices on the GPU that hold items of this request
@@ -319,7 +320,7 @@ void scheduler(r2_server* s) {
           extra -= more * (uint64_t)r.chunk;
           items = (items + 63) & ~(uint64_t)63;
           items = std::min<uint64_t>(items, left);
-          slice.push_back(r2host::BatchSlice{r.d_scene, r.d_partial, r.next_item, items, r.chunk, r.single, r.surf,
+          slice.push_back(r2host::BatchSlice{r.d_scene, r.d_partial, r.next_item, items, r.chunk, r.form, r.surf,
                                              r.fp64, r.packed});
           sl.took.push_back({r.id, items});
           r.next_item += items;
@@ -435,7 +436,7 @@ extern "C" int64_t r2_server_submit(r2_server* s, const r2_request* req) {
   r->fp64 = (r->params.flags & R2_FLAG_FP64_ACCUM) != 0;
   // scenes with surfaces run the general-instance form of the batched kernel
   r->surf = r->scene.n_surf > 0;
-  r->single = r->scene.n_inst == 1 && !r->surf;
+  r->form = r2host::inst_form(r->scene);
   if (r->hs.precision < 0) return R2_ERR_UNSUPPORTED;  // instances mix FP32 and packed grids
   r->packed = r->hs.precision == 1;
   const uint64_t npix = (uint64_t)r->scene.W * r->scene.H;

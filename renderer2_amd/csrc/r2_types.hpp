@@ -11,6 +11,11 @@ namespace r2 {
 constexpr int kMaxGrids = 16;
 constexpr int kMaxInstances = 1 << 20;
 constexpr int kLinearInstances = 8;
+// The kernels' forms by scene: one instance (its fields are wave-uniform scalar
+// loads), a scan over a few, and any number (a scan or the hierarchy).  The
+// hierarchy's walk costs registers: with it, scenes of two to eight instances ran
+// 1 to 5 % slower, so they have a form without.
+enum : int { kOneInst = 0, kFewInst = 1, kAnyInst = 2 };
 constexpr int kLeafDim = 8;            // NanoVDB leaf node: 8^3 voxels
 constexpr int kLeafVoxels = 512;
 constexpr float kDefaultTmax = 1e12f;  // CRay::DEFAULT_TMAX (ray.hpp:12)

@@ -830,7 +830,7 @@ __device__ __forceinline__ void bvh_closest(const DScene& s, const float o[3], c
 // (kSurf) the analytic surfaces through __intersection__surface (:170-189);
 // closest accepted hit wins, the lowest instance index among equal t (the order
 // of a linear scan, which the hierarchy walk reproduces).
-template <bool kSurf = false, bool kSingle = false>
+template <bool kSurf = false, int kInst = kAnyInst>
 __device__ __forceinline__ Hit scene_intersect(const DScene& s, Ray& ray) {
   Hit h;
   h.hit = 0; h.t = 0.f; h.medium = -1; h.pos = mk(0.f, 0.f, 0.f);
@@ -839,8 +839,8 @@ __device__ __forceinline__ Hit scene_intersect(const DScene& s, Ray& ray) {
   const float o[3] = {ray.o.x, ray.o.y, ray.o.z};
   const float inv[3] = {1.f / ray.d.x, 1.f / ray.d.y, 1.f / ray.d.z};
   const int sg0 = inv[0] < 0.f, sg1 = inv[1] < 0.f, sg2 = inv[2] < 0.f;
-  if (kSingle || s.n_bvh == 0) {
-    const int n = kSingle ? 1 : s.n_inst;
+  if (kInst != kAnyInst || s.n_bvh == 0) {
+    const int n = kInst == kOneInst ? 1 : s.n_inst;
     for (int k = 0; k < n; ++k) {
       const DInstance& in = inst_at(s, k);
       float t;
