@@ -219,13 +219,9 @@ struct FrameFetch {
 // waiting at it, chosen from ballots so that the costly blocks run with many
 // lanes: shading once at least R2_SHADE_MIN lanes wait for it (or nothing else
 // is left), followed by segment starts for the lanes at them; else segment
-// starts once at least R2_SEG_MIN of 64 lanes, or R2_SEG_RATIO times as many
-// lanes as are in traversals, wait for them; else a traversal step.  The segment
-// threshold is a share of the lanes that still hold a path: at the end of a launch,
-// and in one of few paths, half of the lanes left do not wait for the others (with
-// the fixed 32 a 333 x 217 x 16 frame took 790 us, now 746; a share for the shading
-// too costs more passes of the largest block: 830).  Returns false when every lane
-// is idle.
+// starts once at least R2_SEG_MIN lanes, or R2_SEG_RATIO times as many lanes as
+// are in traversals, wait for them; else a traversal step.  Returns false when
+// every lane is idle.
 #ifndef R2_SHADE_MIN
 #define R2_SHADE_MIN 48
 #endif
@@ -249,8 +245,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
   const bool at_seg = p.stage == ST_SEG;
   const bool at_trav = p.stage == ST_TRAV;
   const int nh = __popcll(__ballot(at_shade)), ns = __popcll(__ballot(at_seg)), nt = __popcll(__ballot(at_trav));
-  const int live = nh + ns + nt;
-  if (live == 0) return false;
+  if (nh + ns + nt == 0) return false;
 #ifdef R2_SM_STATS
   const uint64_t t0 = SM_CLOCK();
 #endif
@@ -273,7 +268,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
       seg_step<kInst, kSurf>(s, p);
     }
     __builtin_amdgcn_s_setprio(0);
-  } else if (ns * 64 >= R2_SEG_MIN * live || ns >= R2_SEG_RATIO * nt) {
+  } else if (ns >= R2_SEG_MIN || ns >= R2_SEG_RATIO * nt) {
     SM_STAT(3, 1);
     SM_STAT(4, ns);
     __builtin_amdgcn_s_setprio(kPrioSeg);
@@ -423,11 +418,12 @@ __global__ void k_reduce(const Acc* __restrict__ partial, int nchunks, uint32_t 
 
 
 
-// host-side launchers of this instantiation.  Compensated FP64 sums and the lookup
-// counters of the probe run a few instances in the general form, and surface scenes
-// of those two all in it (kernel_form; the same for a standalone and a batched frame).
+// host-side launchers of this instantiation.  The lookup counters of the probe run a
+// few instances in the general form, and surface scenes with them or with
+// compensated FP64 sums all in it (kernel_form; the same for a standalone and a
+// batched frame).
 static int kernel_form(int inst, bool surf, bool fp64, bool count) {
-  if (fp64 || count) return surf || inst != kOneInst ? kAnyInst : kOneInst;
+  if (count || (fp64 && surf)) return surf || inst != kOneInst ? kAnyInst : kOneInst;
   return inst;
 }
 void launch_sm(hipStream_t st, int blocks, int lanes, const DScene* d_scene, uint64_t* counter, uint64_t total,
@@ -444,6 +440,7 @@ void launch_sm(hipStream_t st, int blocks, int lanes, const DScene* d_scene, uin
   } else if (fp64) {
     if (surf) R2K_LAUNCH(kAnyInst, true, false, double);
     else if (f == kOneInst) R2K_LAUNCH(kOneInst, false, false, double);
+    else if (f == kFewInst) R2K_LAUNCH(kFewInst, false, false, double);
     else R2K_LAUNCH(kAnyInst, false, false, double);
   } else if (surf) {
     if (f == kOneInst) R2K_LAUNCH(kOneInst, true, false, float);
@@ -466,6 +463,7 @@ void launch_batch_group(hipStream_t st, int blocks, const void* ents, int n, uin
   if (fp64) {
     if (surf) R2K_LAUNCH(kAnyInst, true, double);
     else if (f == kOneInst) R2K_LAUNCH(kOneInst, false, double);
+    else if (f == kFewInst) R2K_LAUNCH(kFewInst, false, double);
     else R2K_LAUNCH(kAnyInst, false, double);
   } else if (surf) {
     if (f == kOneInst) R2K_LAUNCH(kOneInst, true, float);
