@@ -91,7 +91,7 @@ static_assert(sizeof(ColdLane) == 39 * 4, "ColdLane must keep an odd dword strid
 #ifndef R2_RNG_AHEAD
 #define R2_RNG_AHEAD 4
 #endif
-static_assert(R2_RNG_AHEAD >= 1 && R2_RNG_AHEAD <= 5, "the ring holds two blocks");
+static_assert(R2_RNG_AHEAD >= 4 && R2_RNG_AHEAD <= 5, "a traversal step draws four words in hand; the ring holds two blocks");
 struct PathRng {
   const uint32_t k0, k1;  // launch-uniform: kept in scalar registers
   uint32_t c0, c1, c3;
@@ -132,6 +132,23 @@ struct PathRng {
     return ring[n++ & 7u];
   }
   __device__ __forceinline__ float uni() { return (float)(next_u32() >> 8) * 5.9604644775390625e-08f; }
+  // one of the R2_RNG_AHEAD draws after top_up(): the word is in hand
+  __device__ __forceinline__ float uni_in_hand() { return (float)(ring[n++ & 7u] >> 8) * 5.9604644775390625e-08f; }
+};
+// The draws after a top_up(): the first R2_RNG_AHEAD come without the test for an
+// empty ring and its copy of the block function (inlined at every draw, eleven copies
+// made up half of the traversal step's code).  `left` is known at compile time where
+// the draws are straight-line code.
+struct RngInHand {
+  PathRng& r;
+  int left = R2_RNG_AHEAD;
+  __device__ __forceinline__ float uni() {
+    if (left > 0) {
+      --left;
+      return r.uni_in_hand();
+    }
+    return r.uni();
+  }
 };
 
 struct PathLane {
@@ -214,7 +231,7 @@ __device__ __forceinline__ void start_traversal(const DScene& s, PathLane& p, in
     p.td = ir.d;
     p.ttmax = ir.tmax;
     p.tri = mk(1.f / ir.d.x, 1.f / ir.d.y, 1.f / ir.d.z);
-    p.ttau = -logf(1.f - p.rng.uni());
+    p.ttau = -logf(1.f - p.rng.uni_in_hand());  // sched_step tops up before a segment
     p.tmip = 3.f;
   } else {
     const Ray ir = ray_transform2(rm, g.m2i);
@@ -249,9 +266,10 @@ __device__ __forceinline__ bool traversal_step(const DScene& s, PathLane& p, Cnt
     if (p.ttau > 0.f) return false;
     p.tt += p.ttau / (maj * g.sigma_t);
     if (p.tt >= p.ttmax) return true;
-    const float u0 = p.rng.uni(), u1 = p.rng.uni(), u2 = p.rng.uni();
+    // four draws in hand (sched_step tops up before the step)
+    const float u0 = p.rng.uni_in_hand(), u1 = p.rng.uni_in_hand(), u2 = p.rng.uni_in_hand();
     const float d = lookup_density<kCount>(g, p.to + p.tt * p.td, mk(u0, u1, u2), cnt);
-    if (p.rng.uni() * maj < d * ratio) {
+    if (p.rng.uni_in_hand() * maj < d * ratio) {
       if (p.tk == TK_FLIGHT_DDA) {
         p.tres = 1;
         return true;
@@ -277,11 +295,11 @@ __device__ __forceinline__ bool traversal_step(const DScene& s, PathLane& p, Cnt
   ++p.tsteps;
   count<kCount>(cnt, kCntFlight);
   const float inv_max = 1.f / (ratio / g.inv_max_density);
-  p.tt -= div_sigma_t(g, logf(1.f - p.rng.uni()) * inv_max);
+  p.tt -= div_sigma_t(g, logf(1.f - p.rng.uni_in_hand()) * inv_max);
   if (p.tt >= p.ttmax) return true;
   const Rec fd = filtered_data<kCount>(g, p.to + p.tt * p.td, cnt);
   if (p.tk == TK_FLIGHT_DELTA) {
-    if (ratio * fd.density * inv_max > p.rng.uni()) {
+    if (ratio * fd.density * inv_max > p.rng.uni_in_hand()) {
       p.tres = 1;
       return true;
     }
@@ -290,7 +308,7 @@ __device__ __forceinline__ bool traversal_step(const DScene& s, PathLane& p, Cnt
   p.ttr *= 1.f - gmax(0.f, ratio * fd.density * inv_max);
   if (p.ttr < 1.f) {
     const float pr = 1.f - p.ttr;
-    if (p.rng.uni() < pr) {
+    if (p.rng.uni_in_hand() < pr) {
       p.ttr = 0.f;
       return true;
     }
@@ -535,14 +553,15 @@ __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, cons
   // direct(): light sample, its shadow ray and the phase function toward it
   v3 ldir;
   float lpdf = 0.f;
-  const v3 Le = env_sample<kCount>(s.env, p.rng, ldir, lpdf, cnt);
+  RngInHand rng{p.rng};
+  const v3 Le = env_sample<kCount>(s.env, rng, ldir, lpdf, cnt);
   if (lpdf > 0.f) {
     const v3 dl = normalize(ldir);
     const Ray r = spawn_at_scatter<kInst>(s, sc, dl, sc.n);
     p.ray.o = r.o;  // walked first: straight to the walk registers (wo is taken)
     p.ray.d = r.o + r.tmax * r.d;
     p.ray.medium = r.medium;
-    const float ph = phase_p(sc.S, sc.n, sc.ior, wo, dl, p.rng);
+    const float ph = phase_p(sc.S, sc.n, sc.ior, wo, dl, rng);
     const float mis = (1.f * lpdf) / (1.f * lpdf + 1.f * ph);
     p.c.nee_a = p.thr * ((Le * (mis * ph)) / lpdf);
     flags |= FL_LIGHT;
@@ -551,7 +570,8 @@ __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, cons
   // direct(): phase sample, its shadow ray and the environment along it
   {
     v3 wi;
-    const float ph = phase_sample(sc.S, sc.n, sc.ior, wo, wi, p.rng);
+    RngInHand rng{p.rng};
+    const float ph = phase_sample(sc.S, sc.n, sc.ior, wo, wi, rng);
     if (ph > 0.f) {
       const v3 dw = normalize(wi);
       const Ray r = spawn_at_scatter<kInst>(s, sc, dw, sc.n);
@@ -569,7 +589,8 @@ __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, cons
   // Li: continuation direction; its ray is offset along the unnormalised sample
   {
     v3 wi;
-    (void)phase_sample(sc.S, sc.n, sc.ior, wo, wi, p.rng);
+    RngInHand rng{p.rng};
+    (void)phase_sample(sc.S, sc.n, sc.ior, wo, wi, rng);
     const Ray r = spawn_at_scatter<kInst>(s, sc, normalize(wi), wi);
     p.c.c_o = r.o;
     p.c.c_d = r.d;

@@ -154,7 +154,9 @@ __device__ __forceinline__ void shade(const DScene& s, PathLane& p, Cnt& cnt, ui
   // vertex 0 of the item's next sample: the camera ray
   dead_walk(p);
   p.rng.init(p.rng.c0, p.rng.c1, 0u);
-  const Ray r = camera_ray(s, (int)(p.rng.c0 % (uint32_t)s.W), (int)(p.rng.c0 / (uint32_t)s.W), p.rng);
+  p.rng.top_up();
+  RngInHand rng{p.rng};
+  const Ray r = camera_ray(s, (int)(p.rng.c0 % (uint32_t)s.W), (int)(p.rng.c0 / (uint32_t)s.W), rng);
   p.c.c_o = r.o;
   p.c.c_d = r.d;
   p.c.c_tmax = r.tmax;
