@@ -245,8 +245,8 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
                                            const Fetch& fetch) {
   const bool at_shade = p.stage == ST_SHADE || p.stage == ST_FETCH;
   const bool at_seg = p.stage == ST_SEG;
-  const bool at_trav = p.stage == ST_TRAV;
-  const int nh = __popcll(__ballot(at_shade)), ns = __popcll(__ballot(at_seg)), nt = __popcll(__ballot(at_trav));
+  const int nh = __popcll(__ballot(at_shade)), ns = __popcll(__ballot(at_seg)),
+            nt = __popcll(__ballot(p.stage == ST_TRAV));
   if (nh + ns + nt == 0) return false;
 #ifdef R2_SM_STATS
   const uint64_t t0 = SM_CLOCK();
@@ -283,13 +283,22 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
     SM_STAT(6, SM_CLOCK() - t0);
 #endif
   } else {
-    SM_STAT(7, 1);
-    SM_STAT(8, nt);
+    // traversal steps run in a loop of their own while the rule above keeps choosing
+    // them: around the outer loop the compiler moves the lane's state between the
+    // registers of the three blocks, some 80 moves a step
     __builtin_amdgcn_s_setprio(kPrioTrav);
-    if (at_trav) {
-      p.rng.top_up();
-      trav_step<kInst, kCount>(s, p, cnt);
-    }
+    int mh, ms, mt;
+    do {
+      SM_STAT(7, 1);
+      SM_STAT(8, __popcll(__ballot(p.stage == ST_TRAV)));
+      if (p.stage == ST_TRAV) {
+        p.rng.top_up();
+        trav_step<kInst, kCount>(s, p, cnt);
+      }
+      mh = __popcll(__ballot(p.stage == ST_SHADE || p.stage == ST_FETCH));
+      ms = __popcll(__ballot(p.stage == ST_SEG));
+      mt = __popcll(__ballot(p.stage == ST_TRAV));
+    } while (mt > 0 && mh < R2_SHADE_MIN && ms < R2_SEG_MIN && ms < R2_SEG_RATIO * mt);
     __builtin_amdgcn_s_setprio(0);
 #ifdef R2_SM_STATS
     SM_STAT(9, SM_CLOCK() - t0);
