@@ -5,10 +5,10 @@
 //   1. k_tri_prep   per triangle: world AABB -> conservative range of voxels whose
 //                   ray region (the clip sphere, or the voxel plus one ray length)
 //                   can reach it, split into 64-voxel tasks.
-//   2. k_pairs      one wave per task, one voxel per lane: exact point/triangle
-//                   distance against the voxel's reach radius; passing (voxel, tri)
-//                   pairs are counted (with the task's lane mask), then emitted
-//                   from the masks as 64-bit keys voxel<<32 | tri.
+//   2. k_pairs      the (task, voxel) pairs of a block packed onto its lanes: exact
+//                   point/triangle distance against the voxel's reach radius; passing
+//                   (voxel, tri) pairs are counted (with the task's lane mask), then
+//                   emitted from the masks as 64-bit keys voxel<<32 | tri.
 //   3. radix sort + run-length encode: sorted candidate list per active voxel.
 //   4. k_filter     one wave per group of active voxels; voxel by voxel the 64 lanes
 //                   are the voxel's rays.  Every lane tests every candidate
