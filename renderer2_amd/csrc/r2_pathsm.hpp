@@ -365,6 +365,20 @@ __device__ __forceinline__ Ray spawn_at_scatter(const DScene& s, const Scatter& 
   return lane_move_to_voxel_border<kInst>(s, sc.inst, r);
 }
 
+// a ray along n (normalised) from o to no end, its origin moved along off by d
+__device__ __forceinline__ Ray ray_from(v3 o, v3 n, int medium, v3 off, float d) {
+  const v3 end = o + kDefaultTmax * n, po = offset_point(o, off, d);
+  return mkray(po, n, length_x(end - po), medium);
+}
+// CRay::spawnRay (ray.hpp:62-69); n is the normalised end - start
+__device__ __forceinline__ Ray spawn_ray(v3 start, v3 end, v3 n, int medium) {
+  v3 dir = end - start;
+  const v3 off = offset_point(start, n, offset_x(n));
+  const float t = length_x(end - off);
+  dir = dir / t;
+  return mkray(off, dir, t, medium);
+}
+
 // -------------------------------------------------------------------- walk --
 // Begin the walk of the vertex's ray `role`: the light-sample shadow ray is in
 // the walk registers already, the others wait in the lane's LDS slots.
@@ -408,14 +422,15 @@ __device__ __forceinline__ void cont_done(PathLane& p, int cr) {
 // the bounce loop's no-scatter branch: the environment for an escaped camera
 // ray (looked up by the next shading pass), the end of the path on a miss,
 // else a pass-through: the ray continues from the box it hit without a bounce
+template <bool kSeg>
 __device__ __forceinline__ void cont_nohit(PathLane& p) {
   if (!p.si_hit) {
     cont_done(p, p.b == 0 ? CR_ESCAPED : CR_END);
     return;
   }
-  Ray nr = mkray(p.si_pos, normalize(p.ray.d), kDefaultTmax, p.ray.medium < 0 ? p.si_medium : -1);
-  ray_offset(nr, p.ray.d);
-  p.ray = nr;
+  const v3 d = p.ray.d;
+  p.ray = ray_from(p.si_pos, kSeg ? normalize_x(d) : normalize_y(d), p.ray.medium < 0 ? p.si_medium : -1, d,
+                   kSeg ? offset_x(d) : offset_y(d));
   p.stage = ST_SEG;
 }
 // A lane at the start of a segment (ST_SEG).  For the continuation this is the
@@ -444,7 +459,7 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
     return;
   }
   const int cur = p.ray.medium;
-  Ray r = cont ? p.ray : spawn_ray(p.ray.o, p.ray.d, cur);
+  Ray r = cont ? p.ray : spawn_ray(p.ray.o, p.ray.d, normalize_y(p.ray.d - p.ray.o), cur);
   const Hit h = scene_intersect<kSurf, kInst>(s, r);  // shortens r.tmax to the hit, as the reference's intersect does
   Ray tr = r;  // the ray of the traversal to start
   // a second intersection that both roles may need is made once for all lanes
@@ -462,7 +477,7 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
         cont_done(p, CR_SURFACE);
         return;
       }
-      cont_nohit(p);
+      cont_nohit<true>(p);
       return;
     }
     if (r.medium >= 0) {
@@ -471,8 +486,7 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
         return;
       }
     } else {
-      r2 = mkray(h.pos, normalize(r.d), kDefaultTmax, h.medium);
-      ray_offset(r2, r.d);
+      r2 = ray_from(h.pos, normalize_x(r.d), h.medium, r.d, offset_x(r.d));
       again = true;
     }
   } else {
@@ -492,7 +506,7 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
     // same result); when it meets nothing (si_hit = 2 through the traversal),
     // the traversal's last step ends the walk without another segment pass.
     if (p.sh_seg < 64 + inst_extra(s)) {
-      r2 = spawn_ray(p.ray.o, p.ray.d, p.ray.medium);
+      r2 = spawn_ray(p.ray.o, p.ray.d, normalize_x(p.ray.d - p.ray.o), p.ray.medium);
       again = true;
     }
   }
@@ -500,7 +514,7 @@ __device__ __forceinline__ void seg_step(const DScene& s, PathLane& p) {
     const Hit se = scene_intersect<kSurf, kInst>(s, r2);
     if (cont) {
       if (!se.hit) {
-        cont_nohit(p);
+        cont_nohit<true>(p);
         return;
       }
       if (se.medium >= 0 && h.medium != se.medium) {
@@ -524,7 +538,7 @@ __device__ __forceinline__ void trav_step(const DScene& s, PathLane& p, Cnt& cnt
   if (!traversal_step<kInst, kCount>(s, p, cnt)) return;
   if (p.role == RL_CONT) {
     if (p.tres) cont_done(p, CR_COLLIDED);
-    else cont_nohit(p);
+    else cont_nohit<false>(p);
   } else {
     p.sh_Tr *= p.ttr;  // intersectTr continues from the box face
     if (p.si_hit == 2) {  // the next segment, intersected already, meets nothing
@@ -573,7 +587,7 @@ __device__ __forceinline__ void shade_scatter(const DScene& s, PathLane& p, cons
     RngInHand rng{p.rng};
     const float ph = phase_sample(sc.S, sc.n, sc.ior, wo, wi, rng);
     if (ph > 0.f) {
-      const v3 dw = normalize(wi);
+      const v3 dw = normalize_y(wi);
       const Ray r = spawn_at_scatter<kInst>(s, sc, dw, sc.n);
       p.c.lb0 = r.o;
       p.c.lb1 = r.o + r.tmax * r.d;

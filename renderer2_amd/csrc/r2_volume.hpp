@@ -54,9 +54,9 @@ __device__ __forceinline__ float next_dn(float v) {
   u = (v > 0.f) ? u - 1u : u + 1u;
   return u2f(u);
 }
-// CRay::offsetRayOrigin (ray.hpp:71-84)
-__device__ __forceinline__ v3 offset_point(v3 p, v3 dir) {
-  const float d = fabsf(dir.x) * kRayOffset + fabsf(dir.y) * kRayOffset + fabsf(dir.z) * kRayOffset;
+// CRay::offsetRayOrigin (ray.hpp:71-84): p moved along dir by d, the length of dir
+// in the sum norm times the ray offset
+__device__ __forceinline__ v3 offset_point(v3 p, v3 dir, float d) {
   const v3 off = dir * d;
   v3 po = p + off;
   po.x = off.x > 0.f ? next_up(po.x) : (off.x < 0.f ? next_dn(po.x) : po.x);
@@ -64,18 +64,32 @@ __device__ __forceinline__ v3 offset_point(v3 p, v3 dir) {
   po.z = off.z > 0.f ? next_up(po.z) : (off.z < 0.f ? next_dn(po.z) : po.z);
   return po;
 }
+__device__ __forceinline__ v3 offset_point(v3 p, v3 dir) {
+  return offset_point(p, dir, fabsf(dir.x) * kRayOffset + fabsf(dir.y) * kRayOffset + fabsf(dir.z) * kRayOffset);
+}
 __device__ __forceinline__ void ray_offset(Ray& r, v3 dir) {
   const v3 end = r.o + r.tmax * r.d;
   r.o = offset_point(r.o, dir);
   r.tmax = length(end - r.o);
 }
-// CRay::spawnRay (ray.hpp:62-69)
-__device__ __forceinline__ Ray spawn_ray(v3 start, v3 end, int medium) {
-  v3 dir = end - start;
-  const v3 off = offset_point(start, normalize(end - start));
-  const float t = length(end - off);
-  dir = dir / t;
-  return mkray(off, dir, t, medium);
+
+// Sums of three products with the fused products written out: _x fuses the x product
+// into the rounded y product, _y the other way round.  Left to the compiler, a * a +
+// b * b is fused by its own order of operands, which follows the blocks around the sum:
+// changes of the control flow alone turned the last bits of these directions, and
+// with them single paths (frames differed by up to 1e-3).
+__device__ __forceinline__ v3 normalize_x(v3 a) {
+  return a * (1.f / sqrtf(fmaf(a.z, a.z, fmaf(a.x, a.x, a.y * a.y))));
+}
+__device__ __forceinline__ v3 normalize_y(v3 a) {
+  return a * (1.f / sqrtf(fmaf(a.z, a.z, fmaf(a.y, a.y, a.x * a.x))));
+}
+__device__ __forceinline__ float length_x(v3 a) { return sqrtf(fmaf(a.z, a.z, fmaf(a.x, a.x, a.y * a.y))); }
+__device__ __forceinline__ float offset_x(v3 a) {
+  return fmaf(fabsf(a.z), kRayOffset, fmaf(fabsf(a.x), kRayOffset, fabsf(a.y) * kRayOffset));
+}
+__device__ __forceinline__ float offset_y(v3 a) {
+  return fmaf(fabsf(a.z), kRayOffset, fmaf(fabsf(a.y), kRayOffset, fabsf(a.x) * kRayOffset));
 }
 
 // ------------------------------------------------------------ records --
@@ -859,7 +873,7 @@ __device__ __forceinline__ Hit scene_intersect(const DScene& s, Ray& ray) {
       if (!surface_hit(s.surf[j], ray, h.hit ? h.t : best, t, n) || (h.hit && !(t < h.t))) continue;
       h.hit = 1; h.t = t; h.medium = -1; h.surf = j; h.normal = n;
     }
-    if (h.surf >= 0) h.normal = normalize(h.normal);
+    if (h.surf >= 0) h.normal = normalize_x(h.normal);
   }
   if (h.hit) {
     h.pos = mk(ray.o.x + h.t * ray.d.x, ray.o.y + h.t * ray.d.y, ray.o.z + h.t * ray.d.z);
