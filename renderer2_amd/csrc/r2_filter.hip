@@ -27,6 +27,7 @@
 #include <cmath>
 #include <cstring>
 #include <vector>
+#include "r2_filter_lds.hpp"
 #include "r2_internal.hpp"
 #include "r2_codec.hpp"
 #include "r2_detmath.hpp"
@@ -57,9 +58,7 @@ struct r2_mesh {
 
 namespace {
 
-constexpr int kRow = 68;  // LDS row of one value over a batch's hits: 16-byte aligned, rows 4 banks apart
-constexpr int kWaves = 4;  // waves per 256-thread block
-constexpr int kVals = 17;  // per-ray sums: S6, diffuse3, specular3, normal3, ior, distance
+using namespace r2::filter_lds;
 constexpr uint32_t kTag = 0xF17Eu;
 
 struct FConst {
@@ -661,12 +660,6 @@ __device__ __forceinline__ float quad_add_in_order(float e, float v) {
 // of voxels with many candidates spreads over waves (consecutive ones: 4.6 ms there).
 // kTex: the mesh has texture coordinates or material textures (alpha test,
 // textured colours, normal maps); without, the kernel carries none of that code.
-constexpr int kGroup = 16;        // voxels of a wave's density pass, four lanes each
-constexpr int kTsFloats = 1024;   // clip distances a wave's group may hold (kGroup * 64; a voxel has up to 1000)
-constexpr int kStage = 32;        // candidate triangles staged at a time (9 float4 each)
-static_assert(kStage * 9 * 4 <= kVals * kRow, "the staged triangles share the space of the per-hit values");
-static_assert(kTsFloats <= kVals * kRow, "so do the exp terms of the density iteration");
-constexpr int kSumRow = 19;       // per voxel: the kVals sums, the hit count; odd, so that rows fall on distinct banks
 template <bool kTex>
 __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __restrict__ work, uint32_t n_work,
                                                 int direct, const uint32_t* __restrict__ act,
@@ -675,7 +668,7 @@ __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __rest
                                                 const float4* __restrict__ tri, const int32_t* __restrict__ tidx,
                                                 const float* __restrict__ nrm, const int32_t* __restrict__ tmat,
                                                 const float* __restrict__ matf, uint4* __restrict__ out,
-                                                int ts_cap, int group, int vshift, uint32_t n_waves) {
+                                                int cap, int group, int vshift, uint32_t n_waves) {
   extern __shared__ __align__(16) float lds[];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + (uint32_t)wave));
@@ -683,9 +676,9 @@ __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __rest
   const int ng = (int)((n_work - 1u - w0) / n_waves) + 1;  // voxels w0 + g n_waves < n_work
   // [kVals][kRow] per-hit values of a ray batch, value-major, hits compacted in
   // ray order; before that the staged triangles of the batch
-  float* V = lds + wave * (kVals * kRow + group * (ts_cap + kSumRow));
-  float* TSG = V + kVals * kRow;            // [group][ts_cap] clip distances of the hits, in ray order
-  float* SUM = TSG + group * ts_cap;        // [group][kSumRow]
+  float* V = lds + wave * wave_floats(group, cap);
+  float* TSG = V + kVals * kRow;            // [group][cap] clip distances of the hits, in ray order
+  float* SUM = TSG + group * cap;        // [group][kSumRow]
 
   uint32_t vid = 0, beg = 0, nc = 0;
   int ix = 0, iy = 0, iz = 0;
@@ -717,7 +710,7 @@ __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __rest
                    gnc = (uint32_t)lane_i((int)nc, g);
     const float gx = (float)lane_i(ix, g), gy = (float)lane_i(iy, g), gz = (float)lane_i(iz, g);
     const v3 gctr = mk(lane_f(ctr.x, g), lane_f(ctr.y, g), lane_f(ctr.z, g));
-    float* TS = TSG + g * ts_cap;
+    float* TS = TSG + g * cap;
     float acc = 0.f;  // lane q < kVals: running sum of quantity q over the hit rays, in ray order
     uint32_t hits = 0;
     for (int r0 = 0; r0 < c.n_samples; r0 += 64) {
@@ -850,7 +843,7 @@ __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __rest
   uint32_t wout[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0x3C00u};
   if (hits > 0) {
     // estimateDensity (mesh_filter.hpp:182-204, 216-226)
-    const float* TS = TSG + g * ts_cap;
+    const float* TS = TSG + g * cap;
     const float avg = sum[16] / (float)hits;
     const float P = (float)hits / (float)c.n_samples;
     float dens = -det_logf(1.f - P) / (avg * c.sigma_t);
@@ -865,7 +858,7 @@ __global__ __launch_bounds__(256) void k_filter(FConst c, const uint32_t* __rest
             e = quad_add_in_order(e, h + (uint32_t)j < hits ? det_expf(-dens * c.sigma_t * TS[h + j]) : 0.f);
         } else {
           // few voxels: more lanes share the terms, which every lane then adds from LDS
-          float* E = V + g * ts_cap;
+          float* E = V + g * cap;
           for (uint32_t h = (uint32_t)j; h < hits; h += 1u << vshift) E[h] = det_expf(-dens * c.sigma_t * TS[h]);
           wave_sync();
           uint32_t h = 0;
@@ -1144,13 +1137,13 @@ int launch_filter(r2_ctx* ctx, const r2_mesh* m, const FConst& c, const Binning&
     *kernel_ms = 0.f;
     return R2_OK;
   }
-  const int ts_cap = ((c.n_samples + 63) / 64) * 64;
+  const int cap = ts_cap(c.n_samples);
   // voxels per wave: as many as the LDS for clip distances and the density pass's
   // lanes allow, fewer when there are not 16 waves per CU to make of them
   const uint32_t fill = (uint32_t)r2host::num_cus(ctx) * 16u;
   const int group = (int)std::max<uint32_t>(
-      1u, std::min<uint32_t>(std::min<uint32_t>(kGroup, (uint32_t)(kTsFloats / ts_cap)), n_work / fill));
-  const size_t lds = sizeof(float) * kWaves * (kVals * kRow + group * (ts_cap + kSumRow));
+      1u, std::min<uint32_t>((uint32_t)max_group(cap), n_work / fill));
+  const size_t lds = sizeof(float) * kWaves * wave_floats(group, cap);
   int vshift = 6;  // 2^vshift lanes per voxel of the density pass
   while ((group << vshift) > 64) --vshift;
   const uint32_t n_waves = (n_work + (uint32_t)group - 1u) / (uint32_t)group;
@@ -1158,11 +1151,11 @@ int launch_filter(r2_ctx* ctx, const r2_mesh* m, const FConst& c, const Binning&
   R2F_HIP(hipEventRecord(ctx->ev0, ctx->stream), "filter: event");
   if (c.uv || c.mtex)
     hipLaunchKernelGGL(k_filter<true>, dim3(blocks), dim3(256), lds, ctx->stream, c, work, n_work, direct ? 1 : 0,
-                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, ts_cap, group,
+                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, cap, group,
                        vshift, n_waves);
   else
     hipLaunchKernelGGL(k_filter<false>, dim3(blocks), dim3(256), lds, ctx->stream, c, work, n_work, direct ? 1 : 0,
-                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, ts_cap, group,
+                       B.act, B.off, B.cnt, B.n_act, B.cand, m->tri, m->idx, m->nrm, m->mat, m->matf, out, cap, group,
                        vshift, n_waves);
   R2F_HIP(hipGetLastError(), "filter: k_filter");
   R2F_HIP(hipEventRecord(ctx->ev1, ctx->stream), "filter: event");
