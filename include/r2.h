@@ -58,6 +58,9 @@ const char* r2_last_error(const r2_ctx* ctx);
 int r2_version(void);
 /* The HIP stream the context launches on (a hipStream_t). */
 void* r2_stream(r2_ctx* ctx);
+/* Give the device memory that the context keeps for its next grids and calls back to the
+ * driver, for other allocators of the process.  May be called from any thread. */
+int r2_trim(r2_ctx* ctx);
 
 /* ---------------------------------------------------------------- grid -- */
 /* A filtered volume: NanoVDB-layout record tree + brick majorant grid.
@@ -99,6 +102,9 @@ typedef struct {
 } r2_grid_info;
 
 int r2_grid_upload(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid** out);
+/* The grid's device blocks stay with the context for the next grid (at most 8 GiB, the
+ * oldest go first).  Any allocation of this library on the device that fails takes them
+ * back; r2_trim and r2_destroy do as well. */
 int r2_grid_free(r2_ctx* ctx, r2_grid* grid);
 int r2_grid_get_info(const r2_grid* grid, r2_grid_info* out);
 /* Parity probe: copy the brick grid back.  range: nb^3 u32 (half min | half max << 16),

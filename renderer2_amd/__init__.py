@@ -141,6 +141,10 @@ class Context:
         except Exception:
             pass
 
+    def trim(self):
+        """Give the device memory kept for the next grids back to the driver."""
+        self._check(capi.lib().r2_trim(self.h))
+
     def _check(self, rc):
         return capi.check(rc, self.h)
 

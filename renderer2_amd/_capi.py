@@ -199,6 +199,7 @@ SIGNATURES = [
     ("r2_last_error", C.c_char_p, [C.c_void_p]),
     ("r2_version", C.c_int, []),
     ("r2_stream", C.c_void_p, [C.c_void_p]),
+    ("r2_trim", C.c_int, [C.c_void_p]),
     ("r2_grid_upload", C.c_int, [C.c_void_p, C.POINTER(GridDesc), C.POINTER(C.c_void_p)]),
     ("r2_grid_free", C.c_int, [C.c_void_p, C.c_void_p]),
     ("r2_grid_get_info", C.c_int, [C.c_void_p, C.POINTER(GridInfo)]),

@@ -39,14 +39,8 @@ hipError_t DevCache::get(size_t bytes, void** out, size_t* got) {
       return hipSuccess;
     }
   }
-  hipError_t e = hipMalloc(out, bytes);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    trim();
-    e = hipMalloc(out, bytes);
-  }
   *got = bytes;
-  return e;
+  return dev_malloc(out, bytes);
 }
 void DevCache::put(void* p, size_t bytes) {
   if (!p) return;
@@ -77,15 +71,41 @@ void DevCache::trim() {
   for (auto& b : all) (void)hipFree(b.first);
 }
 
-// hipMalloc that gives the context's cached blocks back before it fails
-static hipError_t malloc_trimmed(r2_ctx* ctx, void** out, size_t bytes) {
-  hipError_t e = hipMalloc(out, bytes);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    ctx->cache.trim();
-    e = hipMalloc(out, bytes);
+// The caches of all contexts, linked through next_, for dev_malloc.  This lock is taken
+// before a cache's own; it is never destroyed, contexts may outlive the statics.
+static std::mutex& caches_mu() {
+  static std::mutex* m = new std::mutex;
+  return *m;
+}
+static DevCache* g_caches = nullptr;
+
+void DevCache::open(int device) {
+  std::lock_guard<std::mutex> lk(caches_mu());
+  device_ = device;
+  next_ = g_caches;
+  g_caches = this;
+}
+DevCache::~DevCache() {
+  if (device_ >= 0) {
+    std::lock_guard<std::mutex> lk(caches_mu());
+    DevCache** c = &g_caches;
+    while (*c != this) c = &(*c)->next_;
+    *c = next_;
   }
-  return e;
+  trim();
+}
+hipError_t dev_malloc(void** out, size_t bytes) {
+  hipError_t e = hipMalloc(out, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  int device = -1;
+  (void)hipGetDevice(&device);
+  {
+    std::lock_guard<std::mutex> lk(caches_mu());
+    for (DevCache* c = g_caches; c; c = c->next_)
+      if (c->device_ == device) c->trim();
+  }
+  return hipMalloc(out, bytes);
 }
 
 int ensure_scratch(r2_ctx* ctx, size_t bytes) {
@@ -96,7 +116,7 @@ int ensure_scratch(r2_ctx* ctx, size_t bytes) {
     ctx->scratch = nullptr;
     ctx->scratch_bytes = 0;
   }
-  R2_HIP(ctx, malloc_trimmed(ctx, &ctx->scratch, bytes));
+  R2_HIP(ctx, dev_malloc(&ctx->scratch, bytes));
   ctx->scratch_bytes = bytes;
   return R2_OK;
 }
@@ -115,7 +135,7 @@ hipError_t pool_get(r2_ctx* ctx, int slot, size_t bytes, void** out) {
     }
     // grow by 1/8 to absorb small size changes between calls
     const size_t want = bytes + bytes / 8;
-    const hipError_t e = malloc_trimmed(ctx, &ctx->pool[slot], want);
+    const hipError_t e = dev_malloc(&ctx->pool[slot], want);
     if (e != hipSuccess) return e;
     ctx->pool_bytes[slot] = want;
   }
@@ -271,7 +291,7 @@ int upload_scene(r2_ctx* ctx, const HostScene& hs, bool may_alloc) {
     (void)hipFree(ctx->d_scene);
     ctx->d_scene = nullptr;
     ctx->scene_cap = 0;
-    R2_HIP(ctx, hipMalloc((void**)&ctx->d_scene, need));
+    R2_HIP(ctx, dev_malloc(&ctx->d_scene, need));
     ctx->scene_cap = need;
   }
   // the image stays in the context until the next upload, past the stream's copy
@@ -402,12 +422,13 @@ int r2_create(r2_ctx** out, int device) {
   r2_ctx* c = new (std::nothrow) r2_ctx();
   if (!c) return R2_ERR_OOM;
   c->device = device;
+  c->cache.open(device);
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
       hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&c->side_done, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->main_mark, hipEventDisableTiming) != hipSuccess ||
-      hipMalloc((void**)&c->d_scene, scene_bytes_for(kCtxSceneInstances) + kSceneCounterBytes) != hipSuccess) {
+      dev_malloc(&c->d_scene, scene_bytes_for(kCtxSceneInstances) + kSceneCounterBytes) != hipSuccess) {
     r2_destroy(c);
     return R2_ERR_HIP;
   }
@@ -427,7 +448,6 @@ int r2_destroy(r2_ctx* c) {
   if (c->side) (void)hipStreamSynchronize(c->side);
   if (c->scratch) (void)hipFree(c->scratch);
   if (c->d_scene) (void)hipFree(c->d_scene);
-  c->cache.trim();
   for (int i = 0; i < r2_ctx::kPoolSlots; ++i)
     if (c->pool[i]) (void)hipFree(c->pool[i]);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -437,6 +457,12 @@ int r2_destroy(r2_ctx* c) {
   if (c->side) (void)hipStreamDestroy(c->side);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
+  return R2_OK;
+}
+
+int r2_trim(r2_ctx* ctx) {
+  if (!ctx) return R2_ERR_INVALID;
+  ctx->cache.trim();
   return R2_OK;
 }
 
@@ -617,7 +643,7 @@ int r2_env_upload(r2_ctx* ctx, const float* rgb, int32_t W, int32_t H, r2_env** 
   if (!e) return R2_ERR_OOM;
   auto up = [&](const void* src, size_t bytes) -> void* {
     void* d = nullptr;
-    if (hipMalloc(&d, bytes) != hipSuccess) return nullptr;
+    if (dev_malloc(&d, bytes) != hipSuccess) return nullptr;
     e->allocs.push_back(d);
     if (hipMemcpy(d, src, bytes, hipMemcpyHostToDevice) != hipSuccess) return nullptr;
     return d;
@@ -733,10 +759,10 @@ int r2_render_paths(r2_ctx* ctx, const r2_render_params* p, int32_t n, const int
     void** q[4];
     ~F() { for (auto x : q) if (*x) (void)hipFree(*x); }
   } f{{&dp, &ds, &dout, &dc}};
-  R2_HIP(ctx, hipMalloc(&dp, (size_t)n * 4));
-  R2_HIP(ctx, hipMalloc(&ds, (size_t)n * 4));
-  R2_HIP(ctx, hipMalloc(&dout, (size_t)n * 12));
-  if (counters) R2_HIP(ctx, hipMalloc(&dc, (size_t)n * kNumCnt * 4));
+  R2_HIP(ctx, dev_malloc(&dp, (size_t)n * 4));
+  R2_HIP(ctx, dev_malloc(&ds, (size_t)n * 4));
+  R2_HIP(ctx, dev_malloc(&dout, (size_t)n * 12));
+  if (counters) R2_HIP(ctx, dev_malloc(&dc, (size_t)n * kNumCnt * 4));
   R2_HIP(ctx, hipMemcpy(dp, pix, (size_t)n * 4, hipMemcpyHostToDevice));
   R2_HIP(ctx, hipMemcpy(ds, smp, (size_t)n * 4, hipMemcpyHostToDevice));
   rc = launch_paths(ctx, s, n, (const int32_t*)dp, (const int32_t*)ds, (float*)dout, (uint32_t*)dc);

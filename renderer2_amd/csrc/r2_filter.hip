@@ -1248,7 +1248,7 @@ extern "C" int r2_mesh_upload(r2_ctx* ctx, const r2_mesh_desc* d, r2_mesh** out)
     return r2host::hip_fail(ctx, e, what);
   };
   auto dalloc = [&](void** p, size_t bytes) {
-    const hipError_t e = hipMalloc(p, bytes);
+    const hipError_t e = r2host::dev_malloc(p, bytes);
     if (e == hipSuccess) m->allocs.push_back(*p);
     return e;
   };

@@ -836,9 +836,9 @@ int dda_cells(r2_ctx* ctx, int n, const float* rays, float sigma_t, int collide_
     ~F() { for (auto x : q) if (*x) (void)hipFree(*x); }
   } f{{&dr, &dc, &dn}};
   const size_t cbytes = (size_t)n * max_cells * 16;
-  R2_HIP(ctx, hipMalloc(&dr, (size_t)n * 28));
-  R2_HIP(ctx, hipMalloc(&dc, cbytes));
-  R2_HIP(ctx, hipMalloc(&dn, (size_t)n * 4));
+  R2_HIP(ctx, dev_malloc(&dr, (size_t)n * 28));
+  R2_HIP(ctx, dev_malloc(&dc, cbytes));
+  R2_HIP(ctx, dev_malloc(&dn, (size_t)n * 4));
   R2_HIP(ctx, hipMemcpy(dr, rays, (size_t)n * 28, hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_dda_cells, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, (const float*)dr, n, sigma_t,
                      collide_every, max_cells, (int32_t*)dc, (int32_t*)dn);

@@ -9,25 +9,46 @@
 #include "r2_types.hpp"
 
 namespace r2host {
+// hipMalloc on the current device.  When it fails, the blocks that all contexts of this
+// device keep (DevCache) are given back and it is tried once more: every allocation of
+// the library goes through here, so that none fails for memory that is only kept.
+hipError_t dev_malloc(void** out, size_t bytes);
+template <typename T>
+hipError_t dev_malloc(T** out, size_t bytes) {
+  void* p = nullptr;
+  const hipError_t e = dev_malloc(&p, bytes);
+  *out = (T*)p;
+  return e;
+}
 // Device blocks that a context's finished calls and freed grids leave for the next
 // ones.  A program that loads one volume after another otherwise pays for fresh
 // memory each time: once as much memory as the device has had been allocated and
 // freed, every new 512 MB block cost 14 ms (the driver clears it), ten times the work
 // of laying out a 256^3 volume.  A block is put here only when nothing on the device
-// uses it any more.  At most kCap bytes are kept (the oldest go first), all are given
-// back when an allocation fails and when the context is destroyed.  A request takes
-// the smallest block that fits with at most an eighth to spare.
+// uses it any more.  At most kCap bytes are kept (the oldest go first); all are given
+// back when an allocation of any context on the device fails, by r2_trim (for other
+// allocators of the process, which cannot ask) and when the context is destroyed.  A
+// request takes the smallest block that fits with at most an eighth to spare.
 class DevCache {
  public:
   static constexpr size_t kCap = size_t(8) << 30;
+  DevCache() = default;
+  DevCache(const DevCache&) = delete;
+  DevCache& operator=(const DevCache&) = delete;
+  ~DevCache();  // gives the blocks back
+  // the device of the context: failing allocations on it find this cache from now on
+  void open(int device);
   hipError_t get(size_t bytes, void** out, size_t* got);
   void put(void* p, size_t bytes);
   void trim();
 
  private:
+  int device_ = -1;
+  DevCache* next_ = nullptr;
   std::mutex mu_;
   std::vector<std::pair<void*, size_t>> free_;  // oldest first
   size_t held_ = 0;
+  friend hipError_t dev_malloc(void** out, size_t bytes);
 };
 // device blocks of one call, put back when it ends (after a wait for the stream)
 struct TmpBlocks {

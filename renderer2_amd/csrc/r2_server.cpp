@@ -392,9 +392,9 @@ extern "C" int r2_server_start(r2_ctx* ctx, const r2_server_config* cfg, r2_serv
     (void)hipStreamDestroy(s->shadow.stream);
     return r2host::fail(ctx, R2_ERR_HIP, "server: stream");
   }
-  if (hipMalloc(&s->d_ents, r2host::batch_entry_bytes() * r2host::kMaxBatchEntries) != hipSuccess ||
-      hipMalloc((void**)&s->d_counters, sizeof(uint64_t) * r2host::kMaxBatchEntries) != hipSuccess ||
-      hipMalloc(&s->d_pool, (size_t)s->cfg.hbm_budget_bytes) != hipSuccess) {
+  if (r2host::dev_malloc(&s->d_ents, r2host::batch_entry_bytes() * r2host::kMaxBatchEntries) != hipSuccess ||
+      r2host::dev_malloc(&s->d_counters, sizeof(uint64_t) * r2host::kMaxBatchEntries) != hipSuccess ||
+      r2host::dev_malloc(&s->d_pool, (size_t)s->cfg.hbm_budget_bytes) != hipSuccess) {
     (void)hipGetLastError();
     if (s->d_ents) (void)hipFree(s->d_ents);
     if (s->d_counters) (void)hipFree(s->d_counters);
