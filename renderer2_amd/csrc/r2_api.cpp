@@ -40,7 +40,9 @@ hipError_t DevCache::get(size_t bytes, void** out, size_t* got) {
     }
   }
   *got = bytes;
-  return dev_malloc(out, bytes);
+  // the blocks of a cache are its device's, whatever device the thread has current
+  const hipError_t e = hipSetDevice(device_);
+  return e == hipSuccess ? dev_malloc(out, bytes) : e;
 }
 void DevCache::put(void* p, size_t bytes) {
   if (!p) return;
@@ -550,12 +552,14 @@ int r2_grid_download_bricks(r2_ctx* ctx, const r2_grid* g, uint32_t* range, uint
 int r2_grid_lookup(r2_ctx* ctx, const r2_grid* g, int32_t n, const int32_t* coords, uint8_t* out) {
   if (!ctx || !g || n < 0 || (n > 0 && (!coords || !out))) return R2_ERR_INVALID;
   if (n == 0) return R2_OK;
+  (void)hipSetDevice(ctx->device);
   return grid_lookup(ctx, g, n, coords, out);
 }
 
 int r2_grid_sample(r2_ctx* ctx, const r2_grid* g, int32_t n, const float* pos, float* out) {
   if (!ctx || !g || n < 0 || (n > 0 && (!pos || !out))) return R2_ERR_INVALID;
   if (n == 0) return R2_OK;
+  (void)hipSetDevice(ctx->device);
   return grid_sample(ctx, g, n, pos, out);
 }
 

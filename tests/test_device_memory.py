@@ -96,3 +96,18 @@ fill_cache(other)
 other.close()
 assert fake.fake_hip_used(0) <= before + 4096
 """)
+
+
+def test_blocks_of_lookups_belong_to_the_context_s_device(fake):
+    # another device is the thread's current one when a context of device 0 answers
+    run(fake, """
+hip = C.CDLL(None)
+for call in (lambda: grid.lookup(np.zeros((70000, 3), np.int32)), lambda: grid.sample(np.zeros((70000, 3), np.float32))):
+    ctx.trim()
+    before = fake.fake_hip_used(0)
+    hip.hipSetDevice(1)
+    call()
+    assert fake.fake_hip_used(1) == 0
+    assert fake.fake_hip_used(0) > before  # kept for the next call
+    hip.hipSetDevice(0)
+""")
