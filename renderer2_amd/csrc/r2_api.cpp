@@ -46,22 +46,31 @@ hipError_t DevCache::get(size_t bytes, void** out, size_t* got) {
 }
 void DevCache::put(void* p, size_t bytes) {
   if (!p) return;
-  std::vector<void*> gone;
-  {
+  bool keep = bytes <= kCap;
+  if (keep) {
     std::lock_guard<std::mutex> lk(mu_);
-    if (bytes > kCap) {
-      gone.push_back(p);
-    } else {
+    try {
       free_.push_back({p, bytes});
       held_ += bytes;
-      while (held_ > kCap) {
-        gone.push_back(free_.front().first);
-        held_ -= free_.front().second;
-        free_.erase(free_.begin());
-      }
+    } catch (const std::bad_alloc&) {
+      keep = false;
     }
   }
-  for (void* q : gone) (void)hipFree(q);
+  if (!keep) {
+    (void)hipFree(p);
+    return;
+  }
+  for (;;) {  // the oldest go until the rest is within the bound
+    void* gone = nullptr;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (held_ <= kCap) return;
+      gone = free_.front().first;
+      held_ -= free_.front().second;
+      free_.erase(free_.begin());
+    }
+    (void)hipFree(gone);
+  }
 }
 void DevCache::trim() {
   std::vector<std::pair<void*, size_t>> all;

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <mutex>
+#include <new>
 #include <string>
 #include <utility>
 #include <vector>
@@ -68,6 +69,12 @@ struct TmpBlocks {
   hipError_t get(T** out, size_t bytes) {
     void* q = nullptr;
     size_t n = 0;
+    *out = nullptr;
+    try {
+      p.reserve(p.size() + 1);
+    } catch (const std::bad_alloc&) {
+      return hipErrorOutOfMemory;
+    }
     const hipError_t e = cache.get(bytes, &q, &n);
     if (e == hipSuccess) p.push_back({q, n});
     *out = (T*)q;

@@ -7,6 +7,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 
 namespace {
 std::mutex mu;
@@ -24,12 +25,24 @@ hipError_t done(hipError_t e) {
   return e;
 }
 char symbol[1 << 20];
+thread_local int new_fails_in = -1;
 }  // namespace
+
+// host memory that runs out: the n-th operator new from now on (and no other) throws
+void* operator new(size_t n) {
+  if (new_fails_in >= 0 && new_fails_in-- == 0) throw std::bad_alloc();
+  void* p = std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 // test controls
 size_t fake_hip_used(int device) { return used[device]; }
 void fake_hip_set_budget(int device, size_t bytes) { budget[device] = bytes; }
+void fake_hip_fail_new(int n) { new_fails_in = n; }
 int fake_hip_bad_frees() { return double_frees; }
 
 hipError_t hipMalloc(void** p, size_t n) {
@@ -38,7 +51,10 @@ hipError_t hipMalloc(void** p, size_t n) {
   if (used[current] + n > budget[current]) return done(hipErrorOutOfMemory);
   *p = std::calloc(n ? n : 1, 1);
   if (!*p) return done(hipErrorOutOfMemory);
+  const int keep = new_fails_in;
+  new_fails_in = -1;
   blocks[*p] = Block{n, current};
+  new_fails_in = keep;
   used[current] += n;
   return hipSuccess;
 }

@@ -111,3 +111,31 @@ for call in (lambda: grid.lookup(np.zeros((70000, 3), np.int32)), lambda: grid.s
     assert fake.fake_hip_used(0) > before  # kept for the next call
     hip.hipSetDevice(0)
 """)
+
+
+# host memory that runs out inside the bookkeeping of blocks is an error code or nothing at
+# all, never an exception through the C interface, and no device block is lost
+@pytest.mark.parametrize("call", ["free", "sample", "lookup"])
+def test_host_memory_running_out_ends_in_an_error_code(fake, call):
+    run(fake, f"""
+L = r2.capi.lib()
+for k in range(4):
+    ctx.trim()
+    before = fake.fake_hip_used(0)
+    g = sparse_grid(ctx, 40)
+    pos, out = np.zeros((9, 3), np.float32), np.zeros((9, 17), np.float32)
+    at, rec = np.zeros((9, 3), np.int32), np.zeros((9, 32), np.uint8)
+    fake.fake_hip_fail_new(k)
+    if "{call}" == "free":
+        rc, g.h = L.r2_grid_free(ctx.h, g.h), None
+    elif "{call}" == "sample":
+        rc = L.r2_grid_sample(ctx.h, g.h, 9, pos.ctypes.data, out.ctypes.data)
+    else:
+        rc = L.r2_grid_lookup(ctx.h, g.h, 9, at.ctypes.data, rec.ctypes.data)
+    fake.fake_hip_fail_new(-1)
+    assert rc in (0, -3, -4), rc
+    if g.h:
+        g.free()
+    ctx.trim()
+    assert fake.fake_hip_used(0) == before, (k, fake.fake_hip_used(0), before)
+""")
