@@ -6,6 +6,7 @@
 // r2_detmath.hpp so that the result does not depend on the device library.
 #include "r2_internal.hpp"
 #include "r2_detmath.hpp"
+#include <algorithm>
 #include <cfloat>
 
 namespace {
@@ -51,34 +52,37 @@ __device__ __forceinline__ float add_in_order(float a, const float* q, int n) {
 // chain of h additions (about 3 us for 1080) behind the double-evaluated logs of
 // one chunk; with one thread per column it was the load, log and addition of every
 // row in turn: 81 us for 1920 x 1080, now 14 us.  8 columns per block give 240
-// blocks at 1920 (fewer columns would cut a row's 96 bytes below a line).
-constexpr int kTmCols = 8, kTmRows = 512, kTmThreads = 1024;
+// blocks at 1920 (fewer columns would cut a row's 96 bytes below a line).  Frames wider
+// than kTmBlocks blocks take several turns of the grid: a launch holds fewer than 2^32
+// threads, and a frame may have 2^28 columns.
+constexpr int kTmCols = 8, kTmRows = 512, kTmThreads = 1024, kTmBlocks = 65536;
 constexpr int kTmStride = kTmRows + 4;  // columns 4 banks apart, 16-byte aligned
 __global__ __launch_bounds__(kTmThreads) void k_tm_columns(const float* __restrict__ hdr, int w, int h,
                                                            float* __restrict__ avg) {
   __shared__ __align__(16) float term[2][kTmCols * kTmStride];
-  const int x0 = blockIdx.x * kTmCols;
   const float divisor = (float)(h * w * 3);
   const int nchunk = (h + kTmRows - 1) / kTmRows;
   const int t = (int)threadIdx.x - 64;
-  float a = 0.f;
-  for (int c = 0; c <= nchunk; ++c) {
-    if (t >= 0) {
-      const int y0 = c * kTmRows, rows = min(kTmRows, h - y0);  // rows <= 0 past the last chunk
-      for (int i = t; i < rows * kTmCols; i += kTmThreads - 64) {
-        const int col = i % kTmCols, r = i / kTmCols, x = x0 + col;
-        if (x < w) {
-          const float* p = hdr + 3 * ((size_t)(y0 + r) * w + x);
-          term[c & 1][col * kTmStride + r] = det_logf(p[0] + p[1] + p[2] + FLT_MIN) / divisor;
+  for (int x0 = (int)blockIdx.x * kTmCols; x0 < w; x0 += (int)gridDim.x * kTmCols) {
+    float a = 0.f;
+    for (int c = 0; c <= nchunk; ++c) {
+      if (t >= 0) {
+        const int y0 = c * kTmRows, rows = min(kTmRows, h - y0);  // rows <= 0 past the last chunk
+        for (int i = t; i < rows * kTmCols; i += kTmThreads - 64) {
+          const int col = i % kTmCols, r = i / kTmCols, x = x0 + col;
+          if (x < w) {
+            const float* p = hdr + 3 * ((size_t)(y0 + r) * w + x);
+            term[c & 1][col * kTmStride + r] = det_logf(p[0] + p[1] + p[2] + FLT_MIN) / divisor;
+          }
         }
+      } else if (c > 0 && threadIdx.x < kTmCols) {
+        const int rows = min(kTmRows, h - (c - 1) * kTmRows);
+        a = add_in_order(a, term[(c - 1) & 1] + threadIdx.x * kTmStride, rows);
       }
-    } else if (c > 0 && threadIdx.x < kTmCols) {
-      const int rows = min(kTmRows, h - (c - 1) * kTmRows);
-      a = add_in_order(a, term[(c - 1) & 1] + threadIdx.x * kTmStride, rows);
+      __syncthreads();
     }
-    __syncthreads();
+    if (threadIdx.x < kTmCols && x0 + (int)threadIdx.x < w) avg[x0 + threadIdx.x] = a;
   }
-  if (threadIdx.x < kTmCols && x0 + (int)threadIdx.x < w) avg[x0 + threadIdx.x] = a;
 }
 
 // k = exp(sum_x avg[x]) - W H FLT_MIN  (computeGlobalTonemapping2): one chain of w
@@ -100,8 +104,9 @@ __global__ __launch_bounds__(kTmFactorThreads) void k_tm_factor(const float* __r
 }
 
 // applyTonemapping, correctGamma, fillByteFrame.  Bound by the double-evaluated
-// power (26 us at 1920 x 1080, 11 us of which the memory needs); a thread takes four values, so that the frame moves in 16-byte loads and
-// stores and the bytes in whole words where the pointers are aligned for it (kVec).
+// power (26 us at 1920 x 1080, 11 us of which the memory needs); a thread takes four
+// values, so that the frame moves in 16-byte loads and stores and the bytes in whole
+// words where the pointers are aligned for it (kVec).
 template <bool kVec>
 __global__ void k_tm_apply(const float* __restrict__ hdr, size_t n3, const float* __restrict__ factor, float inv_gamma,
                            float* __restrict__ ldr, uint8_t* __restrict__ bytes) {
@@ -162,7 +167,7 @@ extern "C" int r2_postprocess(r2_ctx* ctx, const float* hdr, int32_t w, int32_t 
     d_ldr = ldr ? outf : nullptr;
     d_bytes = bytes ? outb : nullptr;
   }
-  hipLaunchKernelGGL(k_tm_columns, dim3((w + kTmCols - 1) / kTmCols), dim3(kTmThreads), 0, st, d_hdr, w, h, avg);
+  hipLaunchKernelGGL(k_tm_columns, dim3(std::min((w + kTmCols - 1) / kTmCols, kTmBlocks)), dim3(kTmThreads), 0, st, d_hdr, w, h, avg);
   hipLaunchKernelGGL(k_tm_factor, dim3(1), dim3(kTmFactorThreads), 0, st, avg, w, h, factor);
   const dim3 ablk((unsigned)((n3 + 1023) / 1024));
   const bool vec = (((uintptr_t)d_hdr | (uintptr_t)d_ldr) & 15) == 0 && ((uintptr_t)d_bytes & 3) == 0;

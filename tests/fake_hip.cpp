@@ -3,6 +3,7 @@
 // kernels do nothing.  Tests of the library's memory handling use it.
 #define __HIP_PLATFORM_AMD__
 #include <hip/hip_runtime_api.h>
+#include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -130,10 +131,24 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
   a->type = hipMemoryTypeDevice;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+// a launch is refused, as by the runtime, when it is empty, when a block has more than
+// 1024 threads or when a grid has 2^32 threads or more in one dimension
+hipError_t hipLaunchKernel(const void*, dim3 g, dim3 b, void**, size_t, hipStream_t) {
+  const uint64_t n[3] = {uint64_t(g.x) * b.x, uint64_t(g.y) * b.y, uint64_t(g.z) * b.z};
+  if (uint64_t(b.x) * b.y * b.z > 1024) return done(hipErrorInvalidConfiguration);
+  for (uint64_t v : n)
+    if (v == 0 || v >= (uint64_t(1) << 32)) return done(hipErrorInvalidConfiguration);
+  return hipSuccess;
+}
+static thread_local dim3 pushed_grid, pushed_block;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t) {
+  pushed_grid = g;
+  pushed_block = b;
+  return hipSuccess;
+}
 hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* st) {
-  *g = *b = dim3();
+  *g = pushed_grid;
+  *b = pushed_block;
   *s = 0;
   *st = nullptr;
   return hipSuccess;

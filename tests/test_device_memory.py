@@ -1,8 +1,12 @@
 """The library's handling of device memory, on the CPU: the host code runs over a preloaded
-stand-in for the HIP runtime (fake_hip.cpp) whose device memory has a budget.
+stand-in for the HIP runtime (fake_hip.cpp) whose device memory has a budget and which refuses
+launches beyond the runtime's limits.
 
-Blocks that a context keeps for its next grid are not lost to anything else: whatever
-allocation fails, of any entry point and any context of the device, gets them back first."""
+* Blocks that a context keeps for its next grid are not lost to anything else: whatever
+  allocation fails, of any entry point and any context of the device, gets them back first;
+  they belong to the context's device.
+* Host memory that runs out is an error code.
+* Frames of every accepted shape can be post-processed."""
 import os
 import subprocess
 import sys
@@ -138,4 +142,14 @@ for k in range(4):
         g.free()
     ctx.trim()
     assert fake.fake_hip_used(0) == before, (k, fake.fake_hip_used(0), before)
+""")
+
+
+@pytest.mark.parametrize("w,h", [(1 << 28, 1), ((1 << 25) + 3, 7), (1, 1 << 28), (16384, 16384), (1, 1)])
+def test_postprocess_launches_every_accepted_shape(fake, w, h):
+    run(fake, f"""
+L = r2.capi.lib()
+p = C.create_string_buffer(64)  # kernels do nothing here: the frame is never read
+rc = L.r2_postprocess(ctx.h, C.addressof(p), {w}, {h}, C.c_float(2.2), C.addressof(p), C.addressof(p), 1)
+assert rc == 0, L.r2_last_error(ctx.h)
 """)

@@ -63,6 +63,18 @@ def test_postprocess_shapes_equal_the_oracle(ctx, h, w, shift):
     assert np.array_equal(host_ldr.view(np.uint32), ref_ldr.view(np.uint32)) and np.array_equal(host_by, ref_by)
 
 
+# more columns than one turn of the grid takes (65536 blocks of 8)
+def test_postprocess_wide_frame_equals_the_oracle(ctx):
+    w, h = 8 * 65536 * 2 + 13, 1
+    rng = np.random.default_rng(3)
+    hdr = rng.lognormal(0.0, 1.0, (h, w, 3)).astype(np.float32)
+    ref_ldr, ref_by = O.postprocess(hdr, 2.2)
+    ldr, by = np.zeros_like(hdr), np.zeros(hdr.shape, np.uint8)
+    capi.check(capi.lib().r2_postprocess(ctx.h, hdr.ctypes.data, w, h, C.c_float(2.2), ldr.ctypes.data, by.ctypes.data, 0),
+               ctx.h)
+    assert np.array_equal(ldr.view(np.uint32), ref_ldr.view(np.uint32)) and np.array_equal(by, ref_by)
+
+
 def write_obj(path: Path, mesh: dict):
     with open(path.with_suffix(".mtl"), "w") as f:
         for k in range(len(mesh["mat_ior"])):
