@@ -116,7 +116,9 @@ hipError_t dev_malloc(void** out, size_t bytes) {
     for (DevCache* c = g_caches; c; c = c->next_)
       if (c->device_ == device) c->trim();
   }
-  return hipMalloc(out, bytes);
+  e = hipMalloc(out, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();  // reported here, not again by a later check
+  return e;
 }
 
 int ensure_scratch(r2_ctx* ctx, size_t bytes) {

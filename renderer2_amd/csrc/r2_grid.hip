@@ -75,8 +75,10 @@ __device__ __forceinline__ void publish_extrema(float lmax, float lmin, int lo[3
 // the brick grid's minorant).  One wavefront per 8^3 leaf: flag[leaf] says whether
 // the leaf holds an active voxel, dens[leaf * 512 + v] the density as the brick grid
 // sees it (0 for inactive voxels and beyond the box), so that the brick passes read
-// 4 bytes per voxel instead of records 32 bytes apart.  Bound by the read of the
-// records (256^3: 512 MB).
+// 4 bytes per voxel instead of records 32 bytes apart (kDens; without it they read the
+// leaf pool, for grids so large that the densities do not fit beside it).  Bound by the
+// read of the records (256^3: 512 MB).
+template <bool kDens>
 __global__ __launch_bounds__(256) void k_active(const uint4* __restrict__ rec, int nx, int ny, int nz, int nlx, int nly,
                                                 int nlz, uint32_t* __restrict__ flag, float* __restrict__ dens,
                                                 Extrema* __restrict__ ext) {
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(256) void k_active(const uint4* __restrict__ rec, i
       const bool in = x < nx && y < ny && z < nz;
       const bool a = in && (d[k] > 0.f || is_corner(x, y, z, nx, ny, nz));
       const float v = a ? d[k] : 0.f;
-      dens[(size_t)li * kLeafVoxels + k * 64 + lane] = v;
+      if (kDens) dens[(size_t)li * kLeafVoxels + k * 64 + lane] = v;
       if (in) lmin = fminf(lmin, v);
       if (a) {
         any = true;
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(256) void k_counts(BuildCounts* __restrict__ c, con
   if (threadIdx.x == 0) {
     c->ext = e;
     c->n_leaves = leaf_slot ? leaf_slot[n_leaf - 1] + flag[n_leaf - 1] : 0u;
-    c->n_bricks = brick_slot[n_brick - 1] + nonempty[n_brick - 1];
+    c->n_bricks = brick_slot ? brick_slot[n_brick - 1] + nonempty[n_brick - 1] : 0u;
   }
 }
 
@@ -490,10 +492,15 @@ namespace r2host {
 // k_active and k_leaves (4.4 and 6.0 TB/s); with two tables through the host, an
 // allocation per array and the brick passes on the 32-byte records it took 0.94, and
 // the freeing of the temporaries and of the grid 0.26.
-int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
+//
+// by_leaf: the brick passes of dense records read k_active's densities (4 B per voxel of
+// temporaries).  Without, they read the leaf pool as for sparse records, after one more
+// wait, and the temporaries are the flags and scans alone.
+static int build_layout(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g, bool by_leaf) {
   using namespace r2;
   const int nx = desc->nx, ny = desc->ny, nz = desc->nz;
   const bool sparse = desc->n_leaves > 0;
+  by_leaf = by_leaf && !sparse;
   hipStream_t st = ctx->stream;
   int rc;
   TmpBlocks tmp(ctx->cache, st);
@@ -573,7 +580,7 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   const size_t o_counts = tc.add(sizeof(BuildCounts)), o_nonempty = tc.add(nbt * 4), o_slot = tc.add(nbt * 4),
                o_scan = tc.add(scan_bytes), o_flag = tc.add(sparse ? 0 : nleaf_total * 4),
                o_lslot = tc.add(sparse ? 0 : nleaf_total * 4),
-               o_dens = tc.add(sparse ? 0 : nleaf_total * kLeafVoxels * 4),
+               o_dens = tc.add(by_leaf ? nleaf_total * kLeafVoxels * 4 : 0),
                o_orig = tc.add(sparse ? (size_t)desc->n_leaves * 12 : 0),
                o_mask = tc.add(sparse && desc->leaf_masks ? (size_t)desc->n_leaves * 64 : 0);
   char* work = nullptr;
@@ -589,15 +596,40 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   uint4* d_leaves = nullptr;
   const dim3 brick_blocks((unsigned)((nbt * 64 + 255) / 256));
   const LeafDens ldens{d_dens, d_flag, nx, ny, nz, nlx, nly};
+  const auto counts_to_host = [&](const uint32_t* nonempty, const uint32_t* slot) -> int {
+    hipLaunchKernelGGL(k_counts, dim3(1), dim3(256), 0, st, d_counts, d_ext, (int)rec_blocks, d_flag,
+                       sparse ? nullptr : d_lslot, nleaf_total, nonempty, slot, nbt);
+    R2_HIP(ctx, hipGetLastError());
+    R2_HIP(ctx, hipMemcpyAsync(&counts, d_counts, sizeof(counts), hipMemcpyDeviceToHost, st));
+    R2_HIP(ctx, hipStreamSynchronize(st));
+    return R2_OK;
+  };
+  // the leaf pool of dense records, once their leaves are counted
+  const auto fill_leaves = [&]() -> int {
+    const int rl = dmalloc(ctx, g, &d_leaves, (size_t)counts.n_leaves * kLeafVoxels * 2);
+    if (rl) return rl;
+    hipLaunchKernelGGL(k_leaves, dim3((unsigned)std::min<size_t>(nleaf_total, 65536)), dim3(256), 0, st, d_rec, nx, ny,
+                       nz, d_flag, d_lslot, nlx, nly, nlz, d_table, d_leaves);
+    R2_HIP(ctx, hipGetLastError());
+    return R2_OK;
+  };
+  const char* none = "grid has no active voxel";
   if (!sparse) {
-    hipLaunchKernelGGL(k_active, dim3(rec_blocks), dim3(256), 0, st, d_rec, nx, ny, nz, nlx, nly, nlz, d_flag, d_dens,
+    const auto active = by_leaf ? k_active<true> : k_active<false>;
+    hipLaunchKernelGGL(active, dim3(rec_blocks), dim3(256), 0, st, d_rec, nx, ny, nz, nlx, nly, nlz, d_flag, d_dens,
                        d_ext);
     R2_HIP(ctx, hipGetLastError());
     sb = scan_bytes;
     R2_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(d_scan, sb, d_flag, d_lslot, (int)nleaf_total, st));
-    hipLaunchKernelGGL(k_brick_range<LeafDens>, brick_blocks, dim3(256), 0, st, ldens, nb[0], nb[1], nb[2], d_range,
-                       d_nonempty);
-    R2_HIP(ctx, hipGetLastError());
+    if (by_leaf) {
+      hipLaunchKernelGGL(k_brick_range<LeafDens>, brick_blocks, dim3(256), 0, st, ldens, nb[0], nb[1], nb[2], d_range,
+                         d_nonempty);
+      R2_HIP(ctx, hipGetLastError());
+    } else {
+      if ((rc = counts_to_host(nullptr, nullptr))) return rc;
+      if (counts.n_leaves == 0) return fail(ctx, R2_ERR_INVALID, none);
+      if ((rc = fill_leaves())) return rc;
+    }
   } else {
     // the caller's leaves in their order
     int32_t* d_orig = (int32_t*)(work + o_orig);
@@ -612,21 +644,19 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
     hipLaunchKernelGGL(k_sparse_leaves, dim3(rec_blocks), dim3(256), 0, st, d_rec, d_mask, d_orig, desc->n_leaves, nx, ny,
                        nz, d_leaves, d_ext);
     R2_HIP(ctx, hipGetLastError());
+  }
+  if (!by_leaf) {
     hipLaunchKernelGGL(k_brick_range<PoolDens>, brick_blocks, dim3(256), 0, st,
                        PoolDens{d_table, d_leaves, nx, ny, nz, nlx, nly}, nb[0], nb[1], nb[2], d_range, d_nonempty);
     R2_HIP(ctx, hipGetLastError());
   }
   sb = scan_bytes;
   R2_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(d_scan, sb, d_nonempty, d_slot, (int)nbt, st));
-  hipLaunchKernelGGL(k_counts, dim3(1), dim3(256), 0, st, d_counts, d_ext, (int)rec_blocks, d_flag,
-                     sparse ? nullptr : d_lslot, nleaf_total, d_nonempty, d_slot, nbt);
-  R2_HIP(ctx, hipGetLastError());
-  R2_HIP(ctx, hipMemcpyAsync(&counts, d_counts, sizeof(counts), hipMemcpyDeviceToHost, st));
-  R2_HIP(ctx, hipStreamSynchronize(st));
+  if ((rc = counts_to_host(d_nonempty, d_slot))) return rc;
   const int64_t nleaves = sparse ? desc->n_leaves : (int64_t)counts.n_leaves;
   const uint32_t nne = counts.n_bricks;
   const Extrema& ext = counts.ext;
-  if (nleaves == 0 || ext.lo[0] > ext.hi[0]) return fail(ctx, R2_ERR_INVALID, "grid has no active voxel");
+  if (nleaves == 0 || ext.lo[0] > ext.hi[0]) return fail(ctx, R2_ERR_INVALID, none);
   const uint32_t maxbits = ext.max_key;
   uint32_t minbits = (ext.min_key & 0x80000000u) ? (ext.min_key & 0x7FFFFFFFu) : ~ext.min_key;
   if (!covers_all) {
@@ -641,11 +671,8 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   d.precision = desc->precision;
   uint8_t* d_atlas = nullptr;
   if ((rc = dmalloc(ctx, g, &d_atlas, (size_t)std::max<uint32_t>(nne, 1) * 512))) return rc;
-  if (!sparse) {
-    if ((rc = dmalloc(ctx, g, &d_leaves, (size_t)nleaves * kLeafVoxels * 2))) return rc;
-    hipLaunchKernelGGL(k_leaves, dim3((unsigned)std::min<size_t>(nleaf_total, 65536)), dim3(256), 0, st, d_rec, nx, ny,
-                       nz, d_flag, d_lslot, nlx, nly, nlz, d_table, d_leaves);
-    R2_HIP(ctx, hipGetLastError());
+  if (by_leaf) {
+    if ((rc = fill_leaves())) return rc;
     hipLaunchKernelGGL(k_brick_atlas<LeafDens>, brick_blocks, dim3(256), 0, st, ldens, nb[0], nb[1], nb[2], d_range,
                        d_slot, d_nonempty, d_bricks, d_atlas, d_maj[0]);
   } else {
@@ -764,6 +791,19 @@ int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
   g->range0 = d_range;
   for (int l = 0; l < 3; ++l) g->mip[l] = d_mip[l];
   return R2_OK;
+}
+
+int grid_build(r2_ctx* ctx, const r2_grid_desc* desc, r2_grid* g) {
+  int rc = build_layout(ctx, desc, g, true);
+  if (rc == R2_ERR_OOM && desc->n_leaves <= 0) {
+    // again with everything of the first attempt given back and without the densities
+    (void)hipStreamSynchronize(ctx->stream);
+    for (auto& b : g->allocs) (void)hipFree(b.first);
+    g->allocs.clear();
+    ctx->cache.trim();
+    rc = build_layout(ctx, desc, g, false);
+  }
+  return rc;
 }
 
 int grid_lookup(r2_ctx* ctx, const r2_grid* g, int n, const int32_t* coords, uint8_t* out) {
