@@ -190,7 +190,9 @@ m44 get_rotation(v3 n) {
 // node: a range of instances is halved along the longest axis of its box centres
 // and both halves along the axis that is then the longest; a range of at most four
 // becomes the node's children themselves.  Instances are ordered by centre then
-// index, so the build is deterministic.
+// index, so the build is deterministic; a centre that is not a number comes last.  A
+// box with a side that is not a number is never rejected on that axis by a scan, so
+// the nodes that hold it are open there.
 static int bvh_levels(int n) {
   int l = 1;
   while ((1ll << (2 * l)) < n) ++l;
@@ -221,10 +223,14 @@ static void bvh_build(const std::vector<DInstance>& inst, std::vector<DBvhNode>&
       }
     }
     static int longest(const float e[3]) { return e[0] >= e[1] ? (e[0] >= e[2] ? 0 : 2) : (e[1] >= e[2] ? 1 : 2); }
+    float centre(int32_t i, int ax) const {
+      const float c = inst[i].bb_min[ax] + inst[i].bb_max[ax];
+      return c == c ? c : INFINITY;
+    }
     int halve(int lo, int hi, int ax) {
       const int mid = (lo + hi) / 2;
       std::nth_element(idx.begin() + lo, idx.begin() + mid, idx.begin() + hi, [&](int32_t x, int32_t y) {
-        const float cx = inst[x].bb_min[ax] + inst[x].bb_max[ax], cy = inst[y].bb_min[ax] + inst[y].bb_max[ax];
+        const float cx = centre(x, ax), cy = centre(y, ax);
         return cx < cy || (cx == cy && x < y);
       });
       return mid;
@@ -246,12 +252,15 @@ static void bvh_build(const std::vector<DInstance>& inst, std::vector<DBvhNode>&
       for (int k = 0; k < 4; ++k) {
         const int cnt = r[k + 1] - r[k];
         for (int a = 0; a < 3; ++a) {
-          nd.lo[a][k] = INFINITY;
-          nd.hi[a][k] = -INFINITY;
+          float lo_a = INFINITY, hi_a = -INFINITY;
           for (int i = r[k]; i < r[k + 1]; ++i) {
-            nd.lo[a][k] = std::min(nd.lo[a][k], inst[idx[i]].bb_min[a]);
-            nd.hi[a][k] = std::max(nd.hi[a][k], inst[idx[i]].bb_max[a]);
+            const float bmin = inst[idx[i]].bb_min[a], bmax = inst[idx[i]].bb_max[a];
+            const bool open = cnt > 1 && !(bmin <= bmax);
+            lo_a = cnt == 1 ? bmin : std::min(lo_a, open ? -INFINITY : bmin);
+            hi_a = cnt == 1 ? bmax : std::max(hi_a, open ? INFINITY : bmax);
           }
+          nd.lo[a][k] = lo_a;
+          nd.hi[a][k] = hi_a;
         }
         nd.child[k] = cnt == 0 ? kBvhEmpty : (cnt == 1 ? idx[r[k]] : kBvhInner);
         if (cnt > 1) run(level + 1, 4 * q + k, r[k], r[k + 1]);

@@ -95,3 +95,30 @@ def test_forest_server_matches_render(ctx, forest):
         srv.stop()
     assert np.array_equal(out, ref)
     assert np.isfinite(ref).all() and ref.mean() > 0
+
+
+def _check_intersections(ctx, w, rays, instances=None):
+    grids, env = _upload(ctx, w)
+    w = dict(w, instances=instances or w["instances"])
+    got = ctx.scene_intersect(w["render"], grids, w["instances"], env, rays)
+    sc = _oracle(w)
+    exp = np.zeros((len(rays), 4), np.float32)
+    for i, r in enumerate(rays):
+        hit, out = sc.intersect(r.astype(np.float32))
+        exp[i] = (hit, out[0] if hit else 0.0, out[4], out[5])
+    hits = exp[:, 0] > 0
+    assert np.array_equal(got[:, 0], exp[:, 0])
+    assert np.array_equal(got[:, 2], exp[:, 2]) and np.array_equal(got[:, 3], exp[:, 3])
+    assert np.array_equal(got[hits, 1], exp[hits, 1])
+    return exp
+
+
+# boxes at infinity or with sides that are not numbers end as they do in a scan
+def test_boxes_that_are_not_finite_match_the_scan(ctx):
+    w = scenes.forest_workload(50, ground=False)
+    inst = [dict(i) for i in w["instances"]]
+    for k, (axis, v) in enumerate([(0, np.inf), (1, -np.inf), (2, np.inf), (0, np.nan), (1, np.nan), (2, np.nan), (1, np.nan)]):
+        pos = list(inst[7 * k]["pos"])
+        pos[axis] = v
+        inst[7 * k]["pos"] = tuple(pos)
+    _check_intersections(ctx, w, _rays(4000, seed=9), inst)
