@@ -113,6 +113,32 @@ def _check_intersections(ctx, w, rays, instances=None):
     return exp
 
 
+# ragged hierarchies: empty children, instances beside nodes, levels of unequal depth, more
+# levels than a full tree of 256, a table that grows past 4096 instances
+@pytest.mark.parametrize("n", [9, 10, 13, 17, 33, 63, 65, 257, 1025, 5000])
+def test_ragged_hierarchies_match_the_scan(ctx, n):
+    exp = _check_intersections(ctx, scenes.forest_workload(n, ground=False), _rays(3000, seed=n))
+    assert (exp[:, 2] >= 0).mean() > 0.1
+
+
+# boxes that coincide (the lowest index wins, whatever the order of the visits), boxes inside
+# others, and a row of boxes with equal centres on two axes
+@pytest.mark.parametrize("kind", ["copies", "nested", "row"])
+def test_equal_boxes_keep_the_lowest_index(ctx, kind):
+    w = scenes.forest_workload(40, ground=False)
+    base = w["instances"]
+    if kind == "copies":
+        inst = [dict(base[k]) for k in np.random.default_rng(2).permutation(np.repeat(np.arange(40), 3))]
+    elif kind == "nested":
+        inst = [dict(base[k % 10], scaling=tuple(np.float32(v) * (1 + k // 10) for v in base[k % 10]["scaling"]))
+                for k in range(40)]
+    else:
+        inst = [dict(base[0], pos=(0.5 * (k // 2) - 4.0, 0.5, 0.0), orientation=(0, 1, 0), scaling=(0.5, 0.5, 0.5))
+                for k in range(37)]
+    exp = _check_intersections(ctx, w, _rays(3000, seed=4), inst)
+    assert (exp[:, 2] >= 0).mean() > 0.02
+
+
 # boxes at infinity or with sides that are not numbers end as they do in a scan
 def test_boxes_that_are_not_finite_match_the_scan(ctx):
     w = scenes.forest_workload(50, ground=False)
