@@ -12,6 +12,7 @@ The recording was made with the library of commit 77486b4, whose kernels ran eve
 more than one instance, and every scene with surfaces, in the general form:
     PYTHONPATH=.:oracle R2_LIB_PATH=<that librenderer2.so> python tests/test_gpu_frame_bits.py
 """
+import functools
 from pathlib import Path
 
 import numpy as np
@@ -25,21 +26,30 @@ SIDE = dict(width=32, height=24, spp=6)
 pytestmark = pytest.mark.gpu
 
 
+@functools.lru_cache(None)
+def _base(name):
+    if name == "one":
+        return scenes.make_workload("c2", n=32, **SIDE)
+    if name == "few":
+        from test_gpu_instances import multi_instance_workload
+
+        return multi_instance_workload(**SIDE)
+    return scenes.forest_workload(40, ground=name == "forest on its ground", **SIDE)
+
+
 def _one(packed=False, ground=False, **cfg):
-    w = scenes.make_workload("c2", n=32, **SIDE)
+    w = dict(_base("one"))
     if ground:
         w["render"] = dict(w["render"], cam_pos=(0.0, 0.7, 2.3), cam_look_at=(0.0, -0.15, 0.0))
     return _finish(w, packed, ground, -0.4, cfg)
 
 
 def _few(packed=False, ground=False, **cfg):
-    from test_gpu_instances import multi_instance_workload
-
-    return _finish(multi_instance_workload(**SIDE), packed, ground, -0.6, cfg)
+    return _finish(dict(_base("few")), packed, ground, -0.6, cfg)
 
 
 def _any(packed=False, ground=False, **cfg):
-    w = scenes.forest_workload(40, ground=ground, **SIDE)
+    w = dict(_base("forest on its ground" if ground else "forest"))
     return _finish(w, packed, False, 0.0, cfg)
 
 
@@ -83,6 +93,25 @@ def test_frames_keep_their_bits(ctx, form):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), \
         f"{form}: {np.mean(got != want):.4f} of the values differ, relative {np.linalg.norm(got - want) / np.linalg.norm(want):.1e}"
     assert np.array_equal(_frame(ctx, w, server=True).view(np.uint32), want.view(np.uint32)), f"{form}: server"
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_frames_are_the_sums_of_their_paths(ctx, form):
+    """A frame of one sample per item is the sum of its paths in sample order.  The path
+    probe, which the other tests compare with the oracle path by path, runs the counting
+    kernels (one or any number of instances); the frame runs the form of its scene."""
+    w = FORMS[form]()
+    cfg = w["render"]
+    grids, env = [ctx.upload_grid(g) for g in w["grids"]], ctx.upload_env(w["env"])
+    n, spp = cfg["width"] * cfg["height"], cfg["spp"]
+    pix = np.repeat(np.arange(n, dtype=np.int32), spp)
+    smp = np.tile(np.arange(spp, dtype=np.int32), n)
+    paths = ctx.render_paths(cfg, grids, w["instances"], env, pix, smp).reshape(n, spp, 3)
+    acc = np.zeros((n, 3), np.float64 if cfg.get("fp64_accum") else np.float32)
+    for s in range(spp):
+        acc += paths[:, s]
+    frame = ctx.render(cfg, grids, w["instances"], env).reshape(n, 3)
+    assert np.array_equal(acc.astype(np.float32), frame), form
 
 
 if __name__ == "__main__":
