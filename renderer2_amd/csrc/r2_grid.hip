@@ -20,8 +20,7 @@ __device__ __forceinline__ bool is_corner(int x, int y, int z, int nx, int ny, i
   return ((x == 0) | (x == nx - 1)) & ((y == 0) | (y == ny - 1)) & ((z == 0) | (z == nz - 1));
 }
 
-// effective density (active rule) + leaf occupancy + bbox + max density
-// order-preserving unsigned key of a float (for atomicMin over any sign)
+// order-preserving unsigned key of a float: minima of any sign by integer comparison
 __device__ __forceinline__ uint32_t float_key(float f) {
   const uint32_t b = __float_as_uint(f);
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
@@ -222,8 +221,12 @@ __global__ __launch_bounds__(256) void k_leaves(const uint4* __restrict__ rec, i
       const int x = lx * 8 + (v & 7), y = ly * 8 + ((v >> 3) & 7), z = lz * 8 + (v >> 6);
       // the record's density is in the first word, which the pair's even lane holds
       const float d = __uint_as_float((uint32_t)__shfl((int)w[k].x, (int)(threadIdx.x & 62u)));
-      // by masks: hipcc compiled the choice between two uint4 under this condition wrongly
-      // (three of the four words of a corner voxel of density 0 became background)
+      // by masks: a choice between two uint4 under a condition with || leaves a block of
+      // nothing but extracts of the loaded words, entered from both sides of the ||.  The
+      // backend's structurizer (structurizecfg of ROCm 7.2.0) hoists the extracts and loses
+      // the values on the second edge: its input was right, and in its output three of
+      // the four words of a corner voxel of density 0 were background.  The structurizer's
+      // input has no other such block in this library's kernels.
       const bool act = (x < nx) & (y < ny) & (z < nz) & ((d > 0.f) | is_corner(x, y, z, nx, ny, nz));
       const uint32_t m = act ? 0xFFFFFFFFu : 0u, ior = h ? 0x3C00u : 0u;
       dst[2 * v + h] = make_uint4(w[k].x & m, w[k].y & m, w[k].z & m, (w[k].w & m) | (ior & ~m));

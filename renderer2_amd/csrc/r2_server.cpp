@@ -434,7 +434,7 @@ extern "C" int64_t r2_server_submit(r2_server* s, const r2_request* req) {
   }
   r2host::render_chunking(r->scene, &r->chunk, &r->nchunks);
   r->fp64 = (r->params.flags & R2_FLAG_FP64_ACCUM) != 0;
-  // scenes with surfaces run the general-instance form of the batched kernel
+  // surfaces and the scene's instances choose the batched kernel's form (kernel_form)
   r->surf = r->scene.n_surf > 0;
   r->form = r2host::inst_form(r->scene);
   if (r->hs.precision < 0) return R2_ERR_UNSUPPORTED;  // instances mix FP32 and packed grids
