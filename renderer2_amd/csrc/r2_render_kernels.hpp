@@ -285,7 +285,7 @@ __device__ __forceinline__ bool sched_step(const DScene& s, PathLane& p, Cnt& cn
   } else {
     // traversal steps run in a loop of their own while the rule above keeps choosing
     // them: around the outer loop the compiler moves the lane's state between the
-    // registers of the three blocks, some 80 moves a step
+    // registers of the three blocks (without: 256^3 frame 3.2 % slower)
     __builtin_amdgcn_s_setprio(kPrioTrav);
     int mh, ms, mt;
     do {
